@@ -426,7 +426,8 @@ int care_get_tuning(care_context* ctx, care_tuning* out) {
     if (ctx->blocksPerCU == 0 && ctx->rs.maxLen) {
         try {
             HIP_TRY(hipSetDevice(ctx->device));
-            const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk);
+            const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk,
+                                                 o.correct_candidates, o.new_columns_to_correct);
             out->correct_blocks_per_cu = correct_resident_blocks(T, lds, gatedK);
         } catch (const HipError& e) {
             return fail(CARE_ERR_DEVICE, "%s: %s", e.what, hipGetErrorString(e.err));
@@ -1160,10 +1161,12 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         ensure_batch(ctx, B);
         const int T = ctx->blockThreads;
         const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
-        const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk);
-        if (lds > size_t(kMaxLdsBytes))
+        const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk);
+        if (need > size_t(kMaxLdsBytes))
             return fail(CARE_ERR_CAPACITY, "reads of length %d need %zu bytes of LDS per correction workgroup (limit %d)",
-                        ctx->rs.maxLen, lds, kMaxLdsBytes);
+                        ctx->rs.maxLen, need, kMaxLdsBytes);
+        const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk,
+                                             o.correct_candidates, o.new_columns_to_correct);
         const int blocksPerCU = ctx->blocksPerCU > 0 ? ctx->blocksPerCU
                                                      : correct_resident_blocks(T, lds, gatedK | (P.gatedRefine ? 4 : 0));
         hipStream_t s = ctx->stream;
@@ -1894,8 +1897,11 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
             const int autoChunk = correct_msa_chunk(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, 0);
             for (int chunk : {0, autoChunk / 2}) {
                 if (chunk != 0 && (chunk < 16 || chunk == autoChunk)) continue;
-                const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, chunk);
-                if (lds > size_t(kMaxLdsBytes)) continue;
+                if (correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, chunk) >
+                    size_t(kMaxLdsBytes))
+                    continue;
+                const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, chunk,
+                                                     o.correct_candidates, o.new_columns_to_correct);
                 const int bpc = ctx->blocksPerCU > 0 ? ctx->blocksPerCU : correct_resident_blocks(T, lds, gatedK);
                 const int blocks = std::max(1, std::min(n, ctx->numCUs * bpc));
                 const float ms = timed([&] {
@@ -2008,10 +2014,12 @@ extern "C" int care_correct_batch_noalloc(care_context* ctx, uint64_t first, int
         HIP_TRY(hipSetDevice(ctx->device));
         const int T = ctx->blockThreads;
         const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
-        const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk);
-        if (lds > size_t(kMaxLdsBytes))
+        const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk);
+        if (need > size_t(kMaxLdsBytes))
             return fail(CARE_ERR_CAPACITY, "reads of length %d need %zu bytes of LDS per correction workgroup (limit %d)",
-                        ctx->rs.maxLen, lds, kMaxLdsBytes);
+                        ctx->rs.maxLen, need, kMaxLdsBytes);
+        const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk,
+                                             o.correct_candidates, o.new_columns_to_correct);
         const int blocksPerCU = ctx->blocksPerCU > 0 ? ctx->blocksPerCU : correct_resident_blocks(T, lds, gatedK);
         // carve the scratch for batches of B anchors
         const size_t mc = size_t(ctx->maxCand);

@@ -12,6 +12,7 @@
 // order: per column, anchor first, then candidates in ascending index.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "device_common.h"
 #include "mlp_device.h"
@@ -43,14 +44,24 @@ __device__ __forceinline__ void store_meta(CandMeta* p, const CandMeta& m) {
     *reinterpret_cast<uint4*>(p) = b.v;
 }
 
-// pack the even bits (0,2,..,30) of x into the low 16 bits
-__device__ __forceinline__ u32 even_bits(u32 x) {
-    x &= 0x55555555u;
-    x = (x | (x >> 1)) & 0x33333333u;
-    x = (x | (x >> 2)) & 0x0F0F0F0Fu;
-    x = (x | (x >> 4)) & 0x00FF00FFu;
-    x = (x | (x >> 8)) & 0x0000FFFFu;
-    return x;
+// 16 bases of a 2-bit word as bit planes: the bases' high bits in the high
+// half, their low bits in the low half, order kept
+__device__ __forceinline__ u32 split_planes(u32 x) {
+    u32 t = (x ^ (x >> 1)) & 0x22222222u;
+    x ^= t ^ (t << 1);
+    t = (x ^ (x >> 2)) & 0x0C0C0C0Cu;
+    x ^= t ^ (t << 2);
+    t = (x ^ (x >> 4)) & 0x00F000F0u;
+    x ^= t ^ (t << 4);
+    t = (x ^ (x >> 8)) & 0x0000FF00u;
+    return x ^ t ^ (t << 8);
+}
+
+// plane word of the 32 bases in x0, x1 of which the first `valid` exist
+__device__ __forceinline__ uint2 plane_word(u32 x0, u32 x1, int valid) {
+    const u32 a = split_planes(x0), b = split_planes(x1);
+    const u32 mask = valid >= 32 ? ~0u : valid > 0 ? ~0u << (32 - valid) : 0u;
+    return make_uint2(((a & 0xFFFF0000u) | (b >> 16)) & mask, ((a << 16) | (b & 0xFFFFu)) & mask);
 }
 
 // Shifts still under their mismatch limit after the first 64 bases, queued
@@ -70,6 +81,7 @@ struct Lds {
     float* qw;      // [256] quality weight per quality character
     u32* aw;        // anchor 2-bit words [pitch]
     uint2* ap;      // anchor planes [hw + 3]
+    uint2* arp;     // planes of the anchor's reverse complement [hw + 3]
     char* anchorQ;  // [maxLen]
     u32* keys;      // [chunk][2] alignment keys (forward, reverse complement) of the staged candidates,
                     // followed by the survivor slices of the waves [waves][2][kSurvivors]
@@ -81,25 +93,41 @@ struct Lds {
     u16* cnt;       // [4][cols]
     float* wgt;     // [4][cols]
     int* scratch;   // [32]
+    u32* differ;    // [pitch] anchor bases some candidate disagrees with (build_msa)
+    float* qbin;    // [4] weights of the quality bins
+    u16* clist;     // [cols] columns whose weights are summed (build_msa)
     u16* dec;       // gated mode: decision columns (anchor positions) [maxLen]
     u8* gacc;       // gated mode: accepted flag per anchor position [maxLen]
     char* gscr;     // gated mode: feature tile and MLP scratch, overlays mst/rows/qrows
-};
+};  // MSA columns (cons .. wgt) are those within reach of the anchor, from the first of them
+
+// MSA columns read beyond the anchor's: candidate correction reaches
+// new_columns past it, gate features two columns past a corrected read, the
+// plain and forest decisions none
+__host__ __device__ inline int msa_margin(bool gated, int correctCandidates, int newColumns) {
+    return correctCandidates ? max(0, newColumns) + 2 : gated ? 2 : 0;
+}
 
 struct LdsDims {
     int pitch, qpitch, hw, maxLen, cols, waves, chunk, gated;
+    // threads as (row, word) pairs of rows of pitch, qpitch and pw words:
+    // rows the workgroup covers at once, and 65536 / words rounded up (the
+    // quotient t / words is t * inverse >> 16 for t < 1024, words <= 64)
+    int stepS, stepQ, stepP, invS, invQ, invP;
     __host__ __device__ int pw() const { return hw + 3; }
     __host__ __device__ size_t bytes() const {
         size_t b = 0;
         b += size_t(chunk) * (sizeof(CandMeta) + sizeof(u32) * (pitch + qpitch));
         b += sizeof(float) * 256;
-        b += sizeof(u32) * pitch;
-        b += sizeof(uint2) * pw();
+        b += sizeof(u32) * 2 * pitch;  // aw, differ
+        b += sizeof(float) * 4;
+        b += 2 * sizeof(uint2) * pw();
         b += (size_t(maxLen) + 3) / 4 * 4;
         b += size_t(chunk) * 2 * sizeof(uint2) * pw();
         b += (size_t(cols) + 3) / 4 * 4;
-        b += sizeof(float) * cols + 2 * sizeof(int) * cols;
+        b += sizeof(float) * cols + sizeof(int) * (2 * cols + 1);
         b += 4 * sizeof(u16) * cols + 4 * sizeof(float) * cols;
+        b += (sizeof(u16) * size_t(cols) + 3) / 4 * 4;
         b += 32 * sizeof(int);
         b += 2 * sizeof(u32) * size_t(chunk);
         b += 2 * sizeof(u32) * size_t(kSurvivors) * size_t(waves);  // survivor slices after the keys
@@ -114,17 +142,21 @@ __device__ Lds carve(char* base, const LdsDims& d) {
     // 16-byte aligned base: 16- and 8-byte records first
     l.mst = reinterpret_cast<CandMeta*>(p); p += sizeof(CandMeta) * d.chunk;
     l.ap = reinterpret_cast<uint2*>(p); p += sizeof(uint2) * d.pw();
+    l.arp = reinterpret_cast<uint2*>(p); p += sizeof(uint2) * d.pw();
     l.cpl = reinterpret_cast<uint2*>(p); p += size_t(d.chunk) * 2 * sizeof(uint2) * d.pw();
     l.rows = reinterpret_cast<u32*>(p); p += sizeof(u32) * size_t(d.chunk) * d.pitch;
     l.qrows = reinterpret_cast<u32*>(p); p += sizeof(u32) * size_t(d.chunk) * d.qpitch;
     l.qw = reinterpret_cast<float*>(p); p += sizeof(float) * 256;
     l.aw = reinterpret_cast<u32*>(p); p += sizeof(u32) * d.pitch;
+    l.differ = reinterpret_cast<u32*>(p); p += sizeof(u32) * d.pitch;
+    l.qbin = reinterpret_cast<float*>(p); p += sizeof(float) * 4;
     l.support = reinterpret_cast<float*>(p); p += sizeof(float) * d.cols;
-    l.coverage = reinterpret_cast<int*>(p); p += sizeof(int) * d.cols;
+    l.coverage = reinterpret_cast<int*>(p); p += sizeof(int) * (d.cols + 1);
     l.origCov = reinterpret_cast<int*>(p); p += sizeof(int) * d.cols;
     l.wgt = reinterpret_cast<float*>(p); p += 4 * sizeof(float) * d.cols;
     l.scratch = reinterpret_cast<int*>(p); p += 32 * sizeof(int);
     l.cnt = reinterpret_cast<u16*>(p); p += 4 * sizeof(u16) * d.cols;
+    l.clist = reinterpret_cast<u16*>(p); p += (sizeof(u16) * size_t(d.cols) + 3) / 4 * 4;
     l.cons = reinterpret_cast<u8*>(p); p += (size_t(d.cols) + 3) / 4 * 4;
     l.anchorQ = reinterpret_cast<char*>(p); p += (size_t(d.maxLen) + 3) / 4 * 4;
     l.keys = reinterpret_cast<u32*>(p); p += 2 * sizeof(u32) * size_t(d.chunk);
@@ -145,21 +177,12 @@ __device__ Lds carve(char* base, const LdsDims& d) {
     return l;
 }
 
+// MSA columns held in LDS: those within `margin` of the anchor
 struct Msa {
     int cols;
     int ab;  // first anchor column
 };
 
-// Builds the MSA of the anchor and candidates meta[0..m) into LDS
-// (src/msa.cpp:9-173).  One thread per column; per column the weights are
-// summed anchor first, then candidates in index order, as on the CPU.
-// Candidate records, 2-bit rows and quality rows are staged through LDS in
-// chunks of dims.chunk candidates.  Only the columns within `margin` of the
-// anchor are computed: every reader of the MSA (refinement, properties,
-// anchor correction and its features, candidate correction within
-// new_columns of the anchor and the gate features two columns around a
-// corrected read) stays inside them, and columns are independent of each
-// other.  All threads must call.
 // per-column sums of the MSA: base counts and weight sums, the weights
 // added in candidate order as the CPU adds them
 struct MsaSums {
@@ -182,57 +205,108 @@ __device__ __forceinline__ void msa_add(MsaSums& s, u32 b, float w) {
 
 // adds the staged candidates 0..nc-1 to the sums of MSA column colRel
 // (relative to the anchor's first base).  kQ is the quality width (0: no
-// qualities, else 1, 2 or 8 bits per base); q4 holds the weights of the
-// 1- and 2-bit bins.  The body has no branch: the orientation selects
-// indices, not code paths.  kSkipMiss: a wavefront skips the candidates
-// that miss all of its columns (measured faster in the plain kernel and
-// slower in the gated one).  Left rolled: unrolled copies hold more loads in
-// flight and raise the registers of the calling kernels.
-template <int kQ, bool kSkipMiss>
-__device__ __forceinline__ void msa_add_staged(const Lds& L, int nc, int colRel, int pitch, int qpitch, int maxLen,
-                                               const float (&q4)[4], MsaSums& s) {
+// qualities, else 1, 2 or 8 bits per base).  The staged rows are oriented, so
+// the body has no branch and 2-bit qualities share the bases' word index and
+// bit offset; the bins' weights are read from LDS (selects cost more).  A
+// candidate that does not cover the column reads words of other rows, which
+// are dropped.  Left rolled (unrolled copies hold more loads in flight and
+// raise the registers of the calling kernels); the next candidate's record is
+// read one iteration ahead.
+template <int kQ>
+__device__ __forceinline__ void msa_add_staged(const Lds& L, int nc, int colRel, int pitch, int qpitch, MsaSums& s) {
+    CandMeta next = L.mst[0];
+    const u32* row = L.rows;
+    const u32* qrow = L.qrows;
 #pragma unroll 1
-    for (int c = 0; c < nc; c++) {
-        const CandMeta cm = L.mst[c];
-        const int len = cm.len;
-        const int p0 = colRel - int(cm.shift);
-        const bool in = u32(p0) < u32(len);
-        if (kSkipMiss && !__any(in)) continue;  // the candidate misses every column of this wavefront
-        const int pos = in ? p0 : 0;
-        const bool rc = cm.flag == 2;
-        // reverse complement: base len-1-pos of the stored read, complemented
-        const int i = rc ? len - 1 - pos : pos;
-        const u32 word = L.rows[c * pitch + (i >> 4)];
-        const u32 b = ((word >> (30 - 2 * (i & 15))) & 3u) ^ (rc ? 3u : 0u);
+    for (int c = 0; c < nc; c++, row += pitch, qrow += qpitch) {
+        const CandMeta cm = next;
+        next = L.mst[c + 1 < nc ? c + 1 : c];
+        const int p = colRel - int(cm.shift);
+        const bool in = u32(p) < u32(cm.len);
+        const u32 at = u32(30 - 2 * p) & 31u;
+        const u32 b = (row[p >> 4] >> at) & 3u;
         float w = cm.u.weight;
-        if (kQ != 0) {
-            const int qi = rc ? maxLen - 1 - pos : pos;
-            const u32* qr = L.qrows + c * qpitch;
-            float qw;
-            if (kQ == 8) {
-                qw = L.qw[(qr[qi >> 2] >> (8 * (qi & 3))) & 0xFFu];
-            } else if (kQ == 2) {
-                const u32 v = (qr[qi >> 4] >> (30 - 2 * (qi & 15))) & 3u;
-                qw = v == 0u ? q4[0] : v == 1u ? q4[1] : v == 2u ? q4[2] : q4[3];
-            } else {
-                qw = ((qr[qi >> 5] >> (31 - (qi & 31))) & 1u) ? q4[1] : q4[0];
-            }
-            w = cm.u.weight * qw;
-        }
+        if (kQ == 8) w = cm.u.weight * L.qw[(qrow[p >> 2] >> (8 * (p & 3))) & 0xFFu];
+        if (kQ == 2) w = cm.u.weight * L.qbin[(qrow[p >> 4] >> at) & 3u];
+        if (kQ == 1) w = cm.u.weight * L.qbin[(qrow[p >> 5] >> (31 - (p & 31))) & 1u];
         msa_add(s, in ? b : 4u, w);
     }
 }
 
-template <bool kSkipMiss>
+// The 16 bases from base b0 on (which may be negative) of a 2-bit row of n
+// words; bases outside the row's words are arbitrary.
+__device__ __forceinline__ u32 bases16(const u32* row, int n, int b0) {
+    const int e = ((b0 + 15) >> 4) - 1;
+    const u32 hi = row[min(max(e, 0), n - 1)], lo = row[min(max(e + 1, 0), n - 1)];
+    return __builtin_amdgcn_alignbit(hi, lo, u32(-2 * b0) & 31u);
+}
+
+// word w of the reverse complement of a 2-bit row of n words and len bases
+__device__ __forceinline__ u32 complement16(const u32* row, int n, int len, int w) {
+    const u32 r = __brev(bases16(row, n, len - 16 - 16 * w));
+    return ~(((r & 0x55555555u) << 1) | ((r >> 1) & 0x55555555u));
+}
+
+// word w of a binned quality row of n words in the order of the reverse
+// complement, position i taking the quality at maxLen - 1 - i
+__device__ __forceinline__ u32 reversed_quality(const u32* row, int n, int maxLen, int w, int bits) {
+    if (bits == 2) {
+        const u32 r = __brev(bases16(row, n, maxLen - 16 - 16 * w));
+        return ((r & 0x55555555u) << 1) | ((r >> 1) & 0x55555555u);
+    }
+    // the word of 32 / bits values that ends at value maxLen - 1 - w * 32 / bits
+    const int per = 32 / bits, b0 = maxLen - per - per * w;
+    const int e = b0 >= 0 ? b0 / per : -1;
+    const u32 r = u32(b0 - e * per);  // values to skip in word e
+    const u32 a = row[min(max(e, 0), n - 1)], b = row[min(max(e + 1, 0), n - 1)];
+    if (bits == 1) return __brev(r ? (a << r) | (b >> (32 - r)) : a);
+    const u32 x = r ? (a >> (8 * r)) | (b << (32 - 8 * r)) : a;  // little-endian bytes
+    return (x << 24) | ((x & 0xFF00u) << 8) | ((x >> 8) & 0xFF00u) | (x >> 24);
+}
+
+// Builds the MSA of the anchor and candidates meta[0..m) into LDS
+// (src/msa.cpp:9-173).  Only the columns within `margin` of the anchor are
+// computed: every reader of the MSA (refinement, properties, anchor
+// correction and its features, candidate correction within new_columns of
+// the anchor and the gate features two columns around a corrected read)
+// stays inside them, and columns are independent of each other.
+//
+// A column of the anchor where every candidate has the anchor's base needs
+// no sums: its consensus is that base, its support (the base's weight sum
+// divided by itself; the anchor's weight is at least 0.001) is exactly 1,
+// its count the column's coverage, and no reader looks at its weights, which
+// are only read where a read differs from the consensus.  At 40 candidates
+// with 1 % substitutions that is about two columns in three, more with
+// fewer.  So the candidates are first compared with the anchor 16 bases a
+// thread, on the 2-bit words, which marks the columns that
+// differ; the coverages come from a prefix sum over candidate starts and
+// ends; and the weights (one thread per column, summed anchor first, then
+// candidates in index order, as on the CPU) are added for the marked columns
+// and those outside the anchor only, packed densely into wavefronts.
+// Candidate records, 2-bit rows and quality rows are staged through LDS in
+// chunks of dims.chunk candidates, the rows in the candidate's orientation
+// (turned a word at a time while staging: a word serves many columns).  All
+// threads must call.
 __device__ Msa build_msa(const CorrectParams& P, const Lds& L, const LdsDims& dims, const CandMeta* meta, int m,
                          int la, int margin, int* sMin, int* sMax) {
-    if (threadIdx.x == 0) {
+    const DevReadStore& rs = P.rs;
+    const bool useQ = P.useQuality != 0;
+    const int pitch = rs.pitch, qpitch = useQ ? rs.qpitch : 0;
+    CARE_CHECK(pitch == dims.pitch && qpitch == dims.qpitch);
+    // thread index opaque: the staging assignment is computed per build, not
+    // hoisted out of the anchor loop into registers held by every phase
+    int tx = int(threadIdx.x);
+    asm volatile("" : "+v"(tx));
+    if (tx == 0) {
         *sMin = 0;
         *sMax = la;
     }
+    const int most = min(dims.cols, la + 2 * margin);
+    for (int i = tx; i <= most; i += blockDim.x) L.coverage[i] = 0;
+    for (int i = tx; i < pitch; i += blockDim.x) L.differ[i] = 0;
     __syncthreads();
     int lmin = 0, lmax = la;
-    for (int c = threadIdx.x; c < m; c += blockDim.x) {
+    for (int c = tx; c < m; c += blockDim.x) {
         const int s = meta[c].shift;
         lmin = min(lmin, s);
         lmax = max(lmax, s + int(meta[c].len));
@@ -245,75 +319,140 @@ __device__ Msa build_msa(const CorrectParams& P, const Lds& L, const LdsDims& di
         atomicMax(sMax, lmax);
     }
     __syncthreads();
+    // columns [first, last) of the MSA, relative to the anchor's first base
+    const int first = max(*sMin, -margin), last = min(*sMax, la + margin);
     Msa msa;
-    msa.cols = *sMax - *sMin;
-    msa.ab = -*sMin;
-    CARE_CHECK(msa.cols <= dims.cols && msa.ab >= 0);
-    const int ae = msa.ab + la;
-    const DevReadStore& rs = P.rs;
-    const bool useQ = P.useQuality != 0;
-    const int cols = msa.cols;
-    const int pitch = rs.pitch, qpitch = useQ ? rs.qpitch : 0;
-    CARE_CHECK(pitch == dims.pitch && qpitch == dims.qpitch);
+    msa.cols = last - first;
+    msa.ab = -first;
+    const int cols = msa.cols, ab = msa.ab;
+    CARE_CHECK(cols <= dims.cols && cols <= most && ab >= 0);
     // staging assignment: thread -> (row r0 + k * rowsPerStep, word w)
-    // thread index opaque: the staging assignment is computed per build, not
-    // hoisted out of the anchor loop into registers held by every phase
-    int tx = int(threadIdx.x);
-    asm volatile("" : "+v"(tx));
-    const int rowsS = int(blockDim.x) / pitch;
-    const int r0S = tx / pitch, wS = tx - r0S * pitch;
-    const int rowsQ = qpitch ? int(blockDim.x) / qpitch : 0;
-    const int r0Q = qpitch ? tx / qpitch : 0, wQ = tx - r0Q * qpitch;
-    const int wb = max(0, msa.ab - margin), we = min(cols, ae + margin);
-    // quality width of the candidate rows, and the weights of the bin
-    // characters of 2-bit ('$', '(', '1', '9') and 1-bit ('(', '5') rows
-    const int qmode = useQ ? rs.qbits : 0;
-    float q4[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-    if (qmode == 2) {
-        q4[0] = L.qw['$'];
-        q4[1] = L.qw['('];
-        q4[2] = L.qw['1'];
-        q4[3] = L.qw['9'];
-    } else if (qmode == 1) {
-        q4[0] = L.qw['('];
-        q4[1] = L.qw['5'];
+    const int rowsS = dims.stepS, rowsQ = dims.stepQ;
+    const int r0S = (tx * dims.invS) >> 16, wS = tx - r0S * pitch;
+    auto stage = [&](int c0, int nc, bool quals) {
+        for (int i = tx; i < nc; i += blockDim.x) {
+            CARE_CHECK(c0 + i < P.maxCand && meta[c0 + i].id < rs.n);
+            store_meta(L.mst + i, load_meta(meta + c0 + i));
+        }
+        if (r0S < rowsS)
+            for (int c = r0S; c < nc; c += rowsS) {
+                const CandMeta cm = load_meta(meta + c0 + c);
+                const u32* row = rs.seqs + u64(cm.id) * pitch;
+                L.rows[c * pitch + wS] = cm.flag == 2 ? complement16(row, pitch, cm.len, wS) : row[wS];
+            }
+        if (!quals || !qpitch) return;
+        const int r0Q = (tx * dims.invQ) >> 16, wQ = tx - r0Q * qpitch;
+        if (r0Q < rowsQ)
+            for (int c = r0Q; c < nc; c += rowsQ) {
+                const CandMeta cm = load_meta(meta + c0 + c);
+                const u32* row = rs.quals + u64(cm.id) * qpitch;
+                L.qrows[c * qpitch + wQ] =
+                    cm.flag == 2 ? reversed_quality(row, qpitch, rs.maxLen, wQ, rs.qbits) : row[wQ];
+            }
+    };
+    const bool oneChunk = m <= dims.chunk;
+    for (int c0 = 0; c0 < m; c0 += dims.chunk) {
+        const int nc = min(dims.chunk, m - c0);
+        if (c0) __syncthreads();  // the previous chunk's rows are no longer read
+        stage(c0, nc, oneChunk);
+        __syncthreads();
+        if (r0S >= rowsS) continue;
+        const int b0 = 16 * wS;  // this thread's anchor bases b0 .. b0 + 15
+        const u32 aw = L.aw[wS];
+        for (int c = r0S; c < nc; c += rowsS) {
+            const int s = L.mst[c].shift, lc = L.mst[c].len;
+            const int lo = min(max(s - b0, 0), 16), hi = min(max(min(la, s + lc) - b0, 0), 16);
+            if (lo < hi) {
+                u32 x = bases16(L.rows + c * pitch, pitch, b0 - s) ^ aw;
+                x = (x | (x >> 1)) & 0x55555555u & (~0u >> (2 * lo)) & (~0u << (32 - 2 * hi));
+                if (x) atomicOr(&L.differ[wS], x);
+            }
+            if (wS == 0) {
+                // covered columns, as +1 at the first and -1 behind the last
+                const int from = min(max(s + ab, 0), cols), to = min(s + lc + ab, cols);
+                if (from < to) {
+                    atomicAdd(&L.coverage[from], 1);
+                    atomicAdd(&L.coverage[to], -1);
+                }
+            }
+        }
     }
-    for (int cb = wb; cb < we; cb += blockDim.x) {
-        const int col = cb + int(threadIdx.x);
-        const bool active = col < we;
+    __syncthreads();
+    // coverage of every column; the columns to sum, listed in order; results
+    // of the others
+    int listed = 0;
+    {
+        const int lane = tx % kWave, wave = tx / kWave, nwaves = int(blockDim.x) / kWave;
+        const u64 below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+        int carry = 0;
+        for (int base = 0; base < cols; base += blockDim.x) {
+            const int col = base + tx;
+            const int i = col - ab;
+            const bool inAnchor = u32(i) < u32(la) && col < cols;
+            bool sum = col < cols;
+            if (inAnchor) sum = ((L.differ[i >> 4] >> (30 - 2 * (i & 15))) & 1u) != 0u;
+            int incl = col < cols ? L.coverage[col] : 0;
+            for (int o = 1; o < kWave; o <<= 1) {
+                const int v = __shfl_up(incl, o, kWave);
+                if (lane >= o) incl += v;
+            }
+            const u64 bal = __ballot(sum);
+            if (lane == kWave - 1) L.scratch[16 + wave] = incl;
+            if (lane == 0) L.scratch[8 + wave] = __popcll(bal);
+            __syncthreads();
+            int at = listed + __popcll(bal & below), cov = carry + incl;
+            for (int w = 0; w < nwaves; w++) {
+                const int k = L.scratch[8 + w], t = L.scratch[16 + w];
+                if (w < wave) {
+                    at += k;
+                    cov += t;
+                }
+                listed += k;
+                carry += t;
+            }
+            if (sum) {
+                CARE_CHECK(at < dims.cols);
+                L.clist[at] = u16(col);
+            } else if (col < cols) {
+                const u32 b = base_at(L.aw, i);
+                L.cons[col] = u8(b);
+                L.support[col] = 1.0f;
+                L.coverage[col] = cov + 1;
+                L.origCov[col] = cov + 1;
+                for (u32 k = 0; k < 4; k++) L.cnt[k * cols + col] = k == b ? u16(cov + 1) : u16(0);
+            }
+            __syncthreads();
+        }
+    }
+    const int qmode = useQ ? rs.qbits : 0;  // quality width of the candidate rows
+    for (int j0 = 0; j0 < listed; j0 += blockDim.x) {
+        const bool active = j0 + tx < listed;
+        const int col = active ? int(L.clist[j0 + tx]) : 0;
         MsaSums sums = {0, 0, 0, 0, 0.f, 0.f, 0.f, 0.f};
         u32 anchorBase = 0;
-        const bool inAnchor = active && col >= msa.ab && col < ae;
+        const int colRel = col - ab;
+        const bool inAnchor = active && u32(colRel) < u32(la);
         if (inAnchor) {
-            const int i = col - msa.ab;
-            anchorBase = base_at(L.aw, i);
-            const float w = useQ ? L.qw[(unsigned char)L.anchorQ[i]] : 1.0f;
+            anchorBase = base_at(L.aw, colRel);
+            const float w = useQ ? L.qw[(unsigned char)L.anchorQ[colRel]] : 1.0f;
             msa_add(sums, anchorBase, 1.0f * w);
         }
         for (int c0 = 0; c0 < m; c0 += dims.chunk) {
             const int nc = min(dims.chunk, m - c0);
-            __syncthreads();
-            for (int i = threadIdx.x; i < nc; i += blockDim.x) {
-                CARE_CHECK(c0 + i < P.maxCand && meta[c0 + i].id < rs.n);
-                store_meta(L.mst + i, load_meta(meta + c0 + i));
+            if (!oneChunk) {
+                __syncthreads();
+                stage(c0, nc, true);
+                __syncthreads();
             }
-            if (r0S < rowsS)
-                for (int c = r0S; c < nc; c += rowsS)
-                    L.rows[c * pitch + wS] = rs.seqs[u64(meta[c0 + c].id) * pitch + wS];
-            if (r0Q < rowsQ)
-                for (int c = r0Q; c < nc; c += rowsQ)
-                    L.qrows[c * qpitch + wQ] = rs.quals[u64(meta[c0 + c].id) * qpitch + wQ];
-            __syncthreads();
-            // a wave-uniform test: lanes past the window run the loop with
+            // a wave-uniform test: lanes past the list run the loop with
             // the others (harmlessly, their sums are dropped), which keeps
             // its counter scalar
             if (!__any(active)) continue;
-            const int colRel = col - msa.ab;
             const int ncU = __builtin_amdgcn_readfirstlane(nc);  // uniform: a scalar loop counter
-            if (qmode == 0) msa_add_staged<0, kSkipMiss>(L, ncU, colRel, pitch, qpitch, rs.maxLen, q4, sums);
-            else if (qmode == 2) msa_add_staged<2, kSkipMiss>(L, ncU, colRel, pitch, qpitch, rs.maxLen, q4, sums);
-            else if (qmode == 1) msa_add_staged<1, kSkipMiss>(L, ncU, colRel, pitch, qpitch, rs.maxLen, q4, sums);
-            else msa_add_staged<8, kSkipMiss>(L, ncU, colRel, pitch, qpitch, rs.maxLen, q4, sums);
+            if (qmode == 0) msa_add_staged<0>(L, ncU, colRel, pitch, qpitch, sums);
+            else if (qmode == 2) msa_add_staged<2>(L, ncU, colRel, pitch, qpitch, sums);
+            else if (qmode == 1) msa_add_staged<1>(L, ncU, colRel, pitch, qpitch, sums);
+            else msa_add_staged<8>(L, ncU, colRel, pitch, qpitch, sums);
         }
         if (!active) continue;
         const int cA = sums.cA, cC = sums.cC, cG = sums.cG, cT = sums.cT;
@@ -342,28 +481,21 @@ __device__ Msa build_msa(const CorrectParams& P, const Lds& L, const LdsDims& di
     return msa;
 }
 
-// masks of the two words j, j + 1 of a lane with nw words whose last word
-// keeps the bits of lastMask
-__device__ __forceinline__ void word_masks(int j, int nw, u32 lastMask, u32* m1, u32* m2) {
-    const u32 a = j + 1 < nw ? ~0u : lastMask;
-    const u32 b = j + 2 < nw ? ~0u : lastMask;
-    *m1 = j < nw ? a : 0u;
-    *m2 = j + 1 < nw ? b : 0u;
-}
-
 struct AlignCtx {
     const uint2* ap;   // anchor planes
+    const uint2* arp;  // planes of the anchor's reverse complement
     const uint2* cpl;  // candidate planes of the chunk, 2 x pw per candidate
     const CandMeta* mst;
     u32* keys;         // [chunk][2] keys, combined by atomic minimum
     u32* survA;        // this wave's survivor slice
     u32* survB;
     int la, pw, minov;
+    bool same;  // every staged candidate is as long as the anchor
     float maxErrorRate;
 };
 
-// Finishes the queued survivors of a wavefront (one per lane): the words
-// from 64 on, then the keys into the candidates' minima.  All lanes call.
+// Finishes the queued survivors of a wavefront (one per lane): the words not
+// compared yet, then the keys into the candidates' minima.  All lanes call.
 __device__ __forceinline__ void finish_survivors(const AlignCtx& A, int count) {
     const int lane = lane_id();
     const bool valid = lane < count;
@@ -372,7 +504,7 @@ __device__ __forceinline__ void finish_survivors(const AlignCtx& A, int count) {
         ea = A.survA[lane];
         eb = A.survB[lane];
     }
-    const int c = int(ea >> 11), u = int(ea & 2047u);
+    const int c = int(ea >> 11) & 511, u = int(ea & 2047u), done = int(ea >> 20);
     int mf = int(eb & 0xFFFFu), mr = int(eb >> 16);
     const int lc = valid ? int(A.mst[c].len) : 0;
     const int la = A.la;
@@ -382,22 +514,26 @@ __device__ __forceinline__ void finish_survivors(const AlignCtx& A, int count) {
     const int ov = valid ? (pos ? min(la - s, lc) : min(la, lc + s)) : 0;
     const int lim = int(float(ov) * A.maxErrorRate);
     const int nw = valid ? (ov + 31) >> 5 : 0;
-    const int d = pos ? s : -s;
+    // the words counted so far are those of the same strand: see align_window
+    const int t = la - lc - s;
+    const bool inside = !pos && t < 0;
+    const int d = pos ? s : inside ? -s : t;
     const u32 sh = u32(32 - (d & 31)) & 31u;
     const int off = (d >> 5) + ((d & 31) != 0);
     const uint2* fp = A.cpl + size_t(2 * c) * A.pw;
     const uint2* rp = fp + A.pw;
-    const uint2* p0 = (pos ? A.ap : fp) + off;  // shifted side, forward candidate
-    const uint2* p1 = (pos ? A.ap : rp) + off;  // shifted side, reverse-complement candidate
-    const uint2* q0 = (pos ? fp : A.ap) + 1;    // word-aligned side
-    const uint2* q1 = (pos ? rp : A.ap) + 1;
+    const uint2* ap = pos || inside ? A.ap : A.arp;
+    const uint2* p0 = (inside ? fp : ap) + off;  // shifted side, forward candidate
+    const uint2* p1 = (inside ? rp : ap) + off;  // shifted side, reverse-complement candidate
+    const uint2* q0 = (inside ? ap : pos ? fp : rp) + 1;  // word-aligned side
+    const uint2* q1 = (inside ? ap : pos ? rp : fp) + 1;
     const u32 lastMask = (ov & 31) ? ~(~0u >> (ov & 31)) : ~0u;
     // one word per iteration: the lanes are mostly full here, and fewer
     // words in flight keep the registers of the calling kernels
     for (int j = 2; __any(j < nw && (mf < lim || mr < lim)); j++) {
         const uint2 a0 = p0[j], a1 = p0[j + 1], b0 = p1[j], b1 = p1[j + 1];
         const uint2 va = q0[j], vb = q1[j];
-        const u32 msk = j + 1 < nw ? ~0u : (j < nw ? lastMask : 0u);
+        const u32 msk = j < done ? 0u : j + 1 < nw ? ~0u : (j < nw ? lastMask : 0u);
         const u32 xf = (__builtin_amdgcn_alignbit(a0.x, a1.x, sh) ^ va.x) |
                        (__builtin_amdgcn_alignbit(a0.y, a1.y, sh) ^ va.y);
         const u32 xr = (__builtin_amdgcn_alignbit(b0.x, b1.x, sh) ^ vb.x) |
@@ -413,11 +549,11 @@ __device__ __forceinline__ void finish_survivors(const AlignCtx& A, int count) {
     wave_sync();
 }
 
-// appends the lanes in `survive` (their order index u and mismatch counts)
-// to the wave's survivor slice, finishing the queued ones first when the
-// slice would overflow; `count` is wave-uniform
+// appends the lanes in `survive` (their order index u and mismatch counts
+// over the first `words` words) to the wave's survivor slice, finishing the
+// queued ones first when the slice would overflow; `count` is wave-uniform
 __device__ __forceinline__ void queue_survivors(const AlignCtx& A, int c, bool survive, int u, int mf, int mr,
-                                                int& count) {
+                                                int words, int& count) {
     const u64 bal = __ballot(survive);
     if (!bal) return;
     const int k = __popcll(bal);
@@ -428,108 +564,165 @@ __device__ __forceinline__ void queue_survivors(const AlignCtx& A, int c, bool s
     const int lane = lane_id();
     if (survive) {
         const int slot = count + __popcll(bal & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
-        A.survA[slot] = (u32(c) << 11) | u32(u);
+        A.survA[slot] = (u32(words) << 20) | (u32(c) << 11) | u32(u);
         A.survB[slot] = u32(mf) | (u32(mr) << 16);
     }
     count += k;
     wave_sync();
 }
 
-// Alignment of the anchor against the candidate planes of one wave, all
-// shifts in parallel, both orientations of a shift in the same lane; key =
-// score << 11 | order index u (u = s for the shifts s >= 0, then
-// u = nPos - 1 - s for s < 0), combined into keys[2c], keys[2c + 1] by
-// atomic minimum (both set to ~0u by the caller first).  The shifts s >= 0
-// and s < 0 run in separate wave-uniform loops.  For s >= 0 the anchor is
-// read from base s against the candidate from base 0, so the shifted anchor
-// words serve both orientations; for s < 0 the candidate is read from base
-// -s against the anchor from base 0, whose words are the same in every
-// lane.  Every shift compares its first 64 bases here; the few shifts still
-// under their mismatch limit (in either orientation) with more bases to go
-// are queued and finished later a wavefront at a time (finish_survivors),
-// instead of holding a wavefront of mostly finished lanes.  Mismatch counts
-// only grow, so counting past the limit changes no result; reads past a
-// lane's last word stay inside the workgroup's LDS and are masked.
-__device__ __forceinline__ void align_wave(const AlignCtx& A, int c, int lc, int& count) {
-    const int lane = lane_id();
+// Alignment of the anchor against the staged candidates, both orientations.
+// The key of a shift is score << 11 | order index u (u = s for the shifts
+// s >= 0, then u = nPos - 1 + d for s = -d < 0), combined into keys[2c]
+// (forward), keys[2c + 1] (reverse complement) by atomic minimum.
+//
+// Every shift is compared over the first W words (32 W bases) of its overlap
+// here; the few still under their mismatch limit in either orientation are
+// queued and finished a wavefront at a time (finish_survivors).  A lane holds
+// one shift's window of the anchor in registers and is compared with the
+// first W words of every candidate, which are the same for all lanes: a
+// candidate costs a wavefront two broadcast reads and four instructions per
+// word and orientation.  That serves both signs of the shift: for s >= 0 the
+// window starts at base s of the anchor and meets the candidate from its
+// first base on; s = -d < 0 is, seen from the other strand, the reverse
+// complement of the anchor from its base t = la - lc + d on against the
+// candidate's reverse complement (for the forward candidate) or the candidate
+// itself (for its reverse complement).  Its overlap la - t does not depend on
+// the candidate's length either.  Shifts with t < 0, which place the whole
+// anchor inside a longer candidate, are compared by align_inside.
+// (Reading the shifted words of every candidate and shift from LDS instead
+// issued about three times the vector instructions.)  Mismatch counts only
+// grow, so counting past the limit changes no result.
+template <int W>
+__device__ __forceinline__ void align_window(const AlignCtx& A, bool neg, int t0, int c0, int c1, int& count) {
+    const int la = A.la;
+    const int nPos = la - A.minov + 1;  // at least 1 here
+    const int t = t0 + lane_id();       // s, or its counterpart on the other strand
+    const bool live = t < nPos;
+    const int ov = live ? la - t : 0;   // bounded by the candidate's length below
+    const int lim = int(float(ov) * A.maxErrorRate);
+    u32 h[W], l[W], msk[W];
+    {
+        const int ts = live ? t : 0;
+        const u32 sh = u32(32 - (ts & 31)) & 31u;
+        const uint2* p = (neg ? A.arp : A.ap) + (ts >> 5) + ((ts & 31) != 0);
+        uint2 a = p[0];
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            // words past the anchor's planes are other data, masked below
+            const uint2 b = p[j + 1];
+            h[j] = __builtin_amdgcn_alignbit(a.x, b.x, sh);
+            l[j] = __builtin_amdgcn_alignbit(a.y, b.y, sh);
+            a = b;
+            const int bits = ov - 32 * j;
+            msk[j] = bits >= 32 ? ~0u : bits > 0 ? ~0u << (32 - bits) : 0u;
+        }
+    }
+    // compares the candidates; kWhole: every overlap spans the W words, kSame:
+    // every candidate is as long as the anchor
+    auto compare = [&](auto kWhole, auto kSame) {
+        const int lim0 = neg && t == 0 ? 0 : lim;  // kSame: t = 0 is no negative shift
+        const uint2* fp = A.cpl + size_t(2 * c0) * A.pw + 1 + (neg ? A.pw : 0);
+        const uint2* rp = A.cpl + size_t(2 * c0) * A.pw + 1 + (neg ? 0 : A.pw);
+#pragma unroll 2
+        for (int c = c0; c < c1; c++, fp += 2 * A.pw, rp += 2 * A.pw) {
+            int mf = 0, mr = 0, limit = lim0;
+#pragma unroll
+            for (int j = 0; j < W; j++) {
+                const uint2 f = fp[j], r = rp[j];
+                u32 x = (h[j] ^ f.x) | (l[j] ^ f.y), y = (h[j] ^ r.x) | (l[j] ^ r.y);
+                if (!kWhole.value) {
+                    u32 k = msk[j];
+                    if (!kSame.value) {
+                        const int bits = int(A.mst[c].len) - 32 * j;
+                        k &= bits >= 32 ? ~0u : bits > 0 ? ~0u << (32 - bits) : 0u;
+                    }
+                    x &= k;
+                    y &= k;
+                }
+                mf += __popc(x);
+                mr += __popc(y);
+            }
+            if (!kSame.value) {
+                // the limit of min(ov, lc) is the smaller of the two limits;
+                // on the other strand the shifts with t <= la - lc are not
+                // negative
+                limit = min(lim, int(A.mst[c].shift));
+                if (neg) limit = t > la - int(A.mst[c].len) ? limit : 0;
+            }
+            const bool survive = min(mf, mr) < limit;
+            if (__any(survive)) {
+                const int u = neg ? nPos - 1 + t + int(A.mst[c].len) - la : t;
+                queue_survivors(A, c, survive, u, mf, mr, W, count);
+            }
+        }
+    };
+    using True = std::integral_constant<bool, true>;
+    using False = std::integral_constant<bool, false>;
+    if (A.same) {
+        if (__all(!live || ov >= 32 * W)) compare(True(), True());
+        else compare(False(), True());
+    } else {
+        compare(False(), False());
+    }
+}
+
+// shifts -d, d = 1 .. dMax, of a candidate that is longer than the anchor and
+// contains it: the candidate is read from base d on
+__device__ __forceinline__ void align_inside(const AlignCtx& A, int c, int dMax, int& count) {
     const int la = A.la;
     const int nPos = max(0, la - A.minov + 1);
-    const int nNeg = max(0, lc - A.minov);
-    const int total = la + lc;
-    const uint2* ap = A.ap;
-    const uint2* fp = A.cpl + size_t(2 * c) * A.pw;
-    const uint2* rp = fp + A.pw;
-    u32 kf = ~0u, kr = ~0u;
-    for (int u0 = 0; u0 < nPos; u0 += kWave) {
-        const int s = u0 + lane;  // order index u = s
-        const int ov = min(la - s, lc);
-        const int lim = int(float(ov) * A.maxErrorRate);
-        const int nw = (s < nPos && lim > 0) ? (ov + 31) >> 5 : 0;
-        const u32 sh = u32(32 - (s & 31)) & 31u;
-        const uint2* p = ap + (s >> 5) + ((s & 31) != 0);
-        const u32 lastMask = (ov & 31) ? ~(~0u >> (ov & 31)) : ~0u;
-        int mf = 0, mr = 0;
-        // the first two words: one LDS round trip covers 64 bases
-        if (__any(nw > 0)) {
-            const uint2 a0 = p[0], a1 = p[1], a2 = p[2];
-            const uint2 f1 = fp[1], f2 = fp[2], r1 = rp[1], r2 = rp[2];
-            u32 msk, msk2;
-            word_masks(0, nw, lastMask, &msk, &msk2);
-            const u32 h1 = __builtin_amdgcn_alignbit(a0.x, a1.x, sh), l1 = __builtin_amdgcn_alignbit(a0.y, a1.y, sh);
-            const u32 h2 = __builtin_amdgcn_alignbit(a1.x, a2.x, sh), l2 = __builtin_amdgcn_alignbit(a1.y, a2.y, sh);
-            mf += __popc(((h1 ^ f1.x) | (l1 ^ f1.y)) & msk) + __popc(((h2 ^ f2.x) | (l2 ^ f2.y)) & msk2);
-            mr += __popc(((h1 ^ r1.x) | (l1 ^ r1.y)) & msk) + __popc(((h2 ^ r2.x) | (l2 ^ r2.y)) & msk2);
-        }
-        const bool survive = nw > 2 && (mf < lim || mr < lim);
-        // finished under the limit (rare: most shifts end over it)
-        if (nw > 0 && !survive && (mf < lim || mr < lim)) {
-            const u32 base = u32(total - 2 * ov);
-            if (mf < lim) kf = min(kf, ((u32(mf) + base) << 11) | u32(s));
-            if (mr < lim) kr = min(kr, ((u32(mr) + base) << 11) | u32(s));
-        }
-        queue_survivors(A, c, survive, s, mf, mr, count);
+    const int lim = int(float(la) * A.maxErrorRate);
+    const u32 m1 = la >= 32 ? ~0u : ~(~0u >> la);
+    const u32 m2 = la >= 64 ? ~0u : la > 32 ? ~(~0u >> (la - 32)) : 0u;
+    const uint2 a1 = A.ap[1], a2 = A.ap[2];
+    for (int d0 = 1; d0 <= dMax; d0 += kWave) {
+        const int d = d0 + lane_id();
+        const int dd = min(d, dMax);
+        const u32 sh = u32(32 - (dd & 31)) & 31u;
+        const uint2* pf = A.cpl + size_t(2 * c) * A.pw + (dd >> 5) + ((dd & 31) != 0);
+        const uint2* pr = pf + A.pw;
+        const uint2 f0 = pf[0], f1 = pf[1], f2 = pf[2], r0 = pr[0], r1 = pr[1], r2 = pr[2];
+        const u32 xf = (__builtin_amdgcn_alignbit(f0.x, f1.x, sh) ^ a1.x) | (__builtin_amdgcn_alignbit(f0.y, f1.y, sh) ^ a1.y);
+        const u32 xr = (__builtin_amdgcn_alignbit(r0.x, r1.x, sh) ^ a1.x) | (__builtin_amdgcn_alignbit(r0.y, r1.y, sh) ^ a1.y);
+        const u32 yf = (__builtin_amdgcn_alignbit(f1.x, f2.x, sh) ^ a2.x) | (__builtin_amdgcn_alignbit(f1.y, f2.y, sh) ^ a2.y);
+        const u32 yr = (__builtin_amdgcn_alignbit(r1.x, r2.x, sh) ^ a2.x) | (__builtin_amdgcn_alignbit(r1.y, r2.y, sh) ^ a2.y);
+        const int mf = __popc(xf & m1) + __popc(yf & m2), mr = __popc(xr & m1) + __popc(yr & m2);
+        queue_survivors(A, c, d <= dMax && min(mf, mr) < lim, nPos - 1 + d, mf, mr, 2, count);
     }
-    for (int v0 = 0; v0 < nNeg; v0 += kWave) {
-        const int d = v0 + lane + 1;  // shift s = -d, order index u = nPos - 1 + d
-        const int ov = min(la, lc - d);
-        const int lim = int(float(ov) * A.maxErrorRate);
-        const int nw = (d <= nNeg && lim > 0) ? (ov + 31) >> 5 : 0;
-        const u32 sh = u32(32 - (d & 31)) & 31u;
-        const int off = (d >> 5) + ((d & 31) != 0);
-        const uint2* pf = fp + off;
-        const uint2* pr = rp + off;
-        const u32 lastMask = (ov & 31) ? ~(~0u >> (ov & 31)) : ~0u;
-        int mf = 0, mr = 0;
-        if (__any(nw > 0)) {
-            const uint2 f0 = pf[0], f1 = pf[1], f2 = pf[2], r0 = pr[0], r1 = pr[1], r2 = pr[2];
-            const uint2 a1 = ap[1], a2 = ap[2];
-            u32 msk, msk2;
-            word_masks(0, nw, lastMask, &msk, &msk2);
-            const u32 xf = (__builtin_amdgcn_alignbit(f0.x, f1.x, sh) ^ a1.x) |
-                           (__builtin_amdgcn_alignbit(f0.y, f1.y, sh) ^ a1.y);
-            const u32 xr = (__builtin_amdgcn_alignbit(r0.x, r1.x, sh) ^ a1.x) |
-                           (__builtin_amdgcn_alignbit(r0.y, r1.y, sh) ^ a1.y);
-            const u32 xf2 = (__builtin_amdgcn_alignbit(f1.x, f2.x, sh) ^ a2.x) |
-                            (__builtin_amdgcn_alignbit(f1.y, f2.y, sh) ^ a2.y);
-            const u32 xr2 = (__builtin_amdgcn_alignbit(r1.x, r2.x, sh) ^ a2.x) |
-                            (__builtin_amdgcn_alignbit(r1.y, r2.y, sh) ^ a2.y);
-            mf += __popc(xf & msk) + __popc(xf2 & msk2);
-            mr += __popc(xr & msk) + __popc(xr2 & msk2);
-        }
-        const int u = nPos - 1 + d;
-        const bool survive = nw > 2 && (mf < lim || mr < lim);
-        if (nw > 0 && !survive && (mf < lim || mr < lim)) {
-            const u32 base = u32(total - 2 * ov);
-            if (mf < lim) kf = min(kf, ((u32(mf) + base) << 11) | u32(u));
-            if (mr < lim) kr = min(kr, ((u32(mr) + base) << 11) | u32(u));
-        }
-        queue_survivors(A, c, survive, u, mf, mr, count);
+}
+
+// One wavefront's share of the alignment of the nc staged candidates: the
+// pairs (window of 64 shifts, candidate), window by window, are cut into
+// equal parts, so that a wavefront sets up one or two windows.
+__device__ __forceinline__ void align_chunk(const AlignCtx& A, int nc, int wave, int nwaves) {
+    int count = 0;  // queued survivors of this wave (wave-uniform)
+    const int la = A.la;
+    const int nPos = max(0, la - A.minov + 1);
+    const int nWin = (nPos + kWave - 1) / kWave;  // of either sign
+    const int total = 2 * nWin * nc;
+    const int end = total * (wave + 1) / nwaves;
+    for (int it = total * wave / nwaves; it < end;) {
+        const int win = it / nc, c0 = it - win * nc;
+        const int c1 = min(nc, c0 + end - it);
+        const bool neg = win >= nWin;
+        const int t0 = kWave * (neg ? win - nWin : win);
+        // words that end most random shifts over the window's largest limit:
+        // three in four random bases differ, so 64 bases reach a limit of 30
+        // (150 bases at the default ratio of 0.2) and 96 bases one of 50 by
+        // five standard deviations
+        const int most = int(float(la - t0) * A.maxErrorRate);
+        if (most <= 30) align_window<2>(A, neg, t0, c0, c1, count);
+        else if (most <= 50) align_window<3>(A, neg, t0, c0, c1, count);
+        else align_window<4>(A, neg, t0, c0, c1, count);
+        it += c1 - c0;
     }
-    // few lanes hold a key here, so each adds its own instead of a
-    // wavefront reduction per candidate
-    if (kf != ~0u) atomicMin(&A.keys[2 * c], kf);
-    if (kr != ~0u) atomicMin(&A.keys[2 * c + 1], kr);
-    wave_sync();
+    for (int c = A.same ? nc : wave; c < nc; c += nwaves) {
+        const int lc = __builtin_amdgcn_readfirstlane(int(A.mst[c].len));
+        const int dMax = min(lc - A.minov, lc - la - 1);
+        if (dMax >= 1) align_inside(A, c, dMax, count);
+    }
+    if (count > 0) finish_survivors(A, count);
 }
 
 struct Aln {
@@ -657,7 +850,9 @@ __device__ ColumnStats column_stats_wave(const Lds& L, int first, int last) {
     cs.maxCov = wave_max_int(mxc);
     float sum = 0.0f;
     if (lane == 0) {
-#pragma unroll 8
+        // reads of 32 columns in flight: the additions wait for LDS five times
+        // in 150 columns instead of nineteen times
+#pragma unroll 32
         for (int c = first; c < last; c++) sum += L.support[c];
     }
     cs.avgSupport = sum / float(last - first);
@@ -849,16 +1044,25 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
     __shared__ int sAnchor, sMin, sMax, sCount[3], sFlag, sCol, sTotal;
     __shared__ float sThr;
     const DevReadStore& rs = P.rs;
-    const int tid = threadIdx.x;
-    const int lane = lane_id();
-    const int wave = tid / kWave;
     const int nwaves = blockDim.x / kWave;
     const int pw = dims.pw();
 
     if (P.useQuality) {
-        for (int i = tid; i < 256; i += blockDim.x) L.qw[i] = P.qweights[i];
+        for (int i = threadIdx.x; i < 256; i += blockDim.x) L.qw[i] = P.qweights[i];
+        // weights of the characters of 2-bit ('$', '(', '1', '9') and 1-bit
+        // ('(', '5') bins
+        if (threadIdx.x < 4)
+            L.qbin[threadIdx.x] = P.qweights[rs.qbits == 1 ? (threadIdx.x & 1 ? '5' : '(')
+                                                           : (unsigned char)(0x39312824u >> (8 * threadIdx.x))];
     }
     for (;;) {
+        // the thread index is opaque to the compiler in every iteration, so
+        // that nothing derived from it is computed once for all anchors and
+        // held in registers through every phase
+        int tid = int(threadIdx.x);
+        asm volatile("" : "+v"(tid));
+        const int lane = tid % kWave;
+        const int wave = tid / kWave;
         if (tid == 0) sAnchor = atomicAdd(P.queueHead, 1);
         __syncthreads();
         const int a = sAnchor;
@@ -887,24 +1091,23 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
             for (int i = tid; i < la; i += blockDim.x) L.anchorQ[i] = quality_char(q, i, rs.qbits);
         }
         __syncthreads();
-        for (int p = tid; p < pw; p += blockDim.x) {
-            const int w = p - 1;  // plane word (index 0 is padding)
-            u32 hi = 0, lo = 0;
-            if (w >= 0 && 2 * w < rs.pitch) {
-                const u32 x0 = L.aw[2 * w];
-                const u32 x1 = 2 * w + 1 < rs.pitch ? L.aw[2 * w + 1] : 0u;
-                hi = (even_bits(x0 >> 1) << 16) | even_bits(x1 >> 1);
-                lo = (even_bits(x0) << 16) | even_bits(x1);
-                // clear bits beyond the read
-                const int valid = la - 32 * w;
-                if (valid <= 0) { hi = 0; lo = 0; }
-                else if (valid < 32) {
-                    const u32 mask = ~0u << (32 - valid);
-                    hi &= mask;
-                    lo &= mask;
+        // planes of the anchor and its reverse complement (word 0 is padding)
+        for (int p = tid; p < 2 * pw; p += blockDim.x) {
+            const bool rc = p >= pw;
+            const int w = (rc ? p - pw : p) - 1;
+            uint2 v = make_uint2(0, 0);
+            if (w >= 0 && 32 * w < la) {
+                u32 x0, x1;
+                if (rc) {
+                    x0 = complement16(L.aw, rs.pitch, la, 2 * w);
+                    x1 = complement16(L.aw, rs.pitch, la, 2 * w + 1);
+                } else {
+                    x0 = L.aw[2 * w];
+                    x1 = 2 * w + 1 < rs.pitch ? L.aw[2 * w + 1] : 0u;
                 }
+                v = plane_word(x0, x1, la - 32 * w);
             }
-            L.ap[p] = make_uint2(hi, lo);
+            (rc ? L.arp : L.ap)[w + 1] = v;
         }
         __syncthreads();
 
@@ -932,18 +1135,22 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
         for (int c0 = 0; c0 < n; c0 += dims.chunk) {
             const int nc = min(dims.chunk, n - c0);
             __syncthreads();  // the previous chunk's rows and keys are no longer read
-            if (mateIds && mateN <= mateCap) {
+            if (tid == 0) sFlag = 0;  // some staged candidate differs in length from the anchor
+            if (mateIds && mateN <= mateCap)
                 for (int i = tid; i < mateN; i += blockDim.x) L.keys[i] = mateIds[i];
-                __syncthreads();
-            }
-            for (int i = tid; i < nc * rs.pitch; i += blockDim.x) {
-                const int c = i / rs.pitch, w = i - c * rs.pitch;
+            __syncthreads();
+            const int rS = (tid * dims.invS) >> 16, w = tid - rS * rs.pitch;
+            for (int c = rS < dims.stepS ? rS : nc; c < nc; c += dims.stepS) {
+                const int i = c * rs.pitch + w;
                 const u32 cid = ids[c0 + c];
                 CARE_CHECK(cid < rs.n && cid != u32(id) && c < dims.chunk);
                 L.rows[i] = rs.seqs[u64(cid) * rs.pitch + w];
                 if (w == 0) {
                     L.mst[c].id = cid;
-                    L.mst[c].len = u16(rs.lens[cid]);
+                    const int lc = rs.lens[cid];
+                    L.mst[c].len = u16(lc);
+                    if (lc != la) sFlag = 1;
+                    L.mst[c].shift = short(min(int(float(lc) * P.maxErrorRate), 32767));  // mismatch limit
                     // the candidate's mate is a candidate of the anchor's mate
                     // (include/corrector.hpp:763-807)
                     u8 paired = 0;
@@ -971,36 +1178,26 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
                 }
             }
             __syncthreads();
-            // bit planes of every staged candidate: forward ...
-            for (int it = tid; it < nc * pw; it += blockDim.x) {
-                const int c = it / pw, p = it - c * pw;
+            // bit planes of every staged candidate (word 0 is padding): forward ...
+            const int rP = (tid * dims.invP) >> 16, p = tid - rP * pw, wP = p - 1;
+            const int firstP = rP < dims.stepP ? rP : nc;
+            for (int c = firstP; c < nc; c += dims.stepP) {
                 const int lc = L.mst[c].len;
                 const u32* cenc = L.rows + c * rs.pitch;
-                const int w = p - 1;  // plane word (index 0 is padding)
-                u32 hi = 0, lo = 0;
-                if (w >= 0 && w < (lc + 31) / 32) {
-                    const u32 x0 = cenc[2 * w];
-                    const u32 x1 = 2 * w + 1 < rs.pitch ? cenc[2 * w + 1] : 0u;
-                    hi = (even_bits(x0 >> 1) << 16) | even_bits(x1 >> 1);
-                    lo = (even_bits(x0) << 16) | even_bits(x1);
-                    const int valid = lc - 32 * w;
-                    if (valid < 32) {
-                        const u32 mask = ~0u << (32 - valid);
-                        hi &= mask;
-                        lo &= mask;
-                    }
-                }
-                L.cpl[size_t(2 * c) * pw + p] = make_uint2(hi, lo);
+                uint2 v = make_uint2(0, 0);
+                if (wP >= 0 && 32 * wP < lc)
+                    v = plane_word(cenc[2 * wP], 2 * wP + 1 < rs.pitch ? cenc[2 * wP + 1] : 0u, lc - 32 * wP);
+                L.cpl[size_t(2 * c) * pw + p] = v;
             }
+            for (int i = tid; i < 2 * nc; i += blockDim.x) L.keys[i] = ~0u;
             __syncthreads();
             // ... and reverse complement: rc[q] = 1 - f[lc-1-q]
-            for (int it = tid; it < nc * pw; it += blockDim.x) {
-                const int c = it / pw, p = it - c * pw;
+            for (int c = firstP; c < nc; c += dims.stepP) {
                 const int lc = L.mst[c].len;
                 const uint2* fp = L.cpl + size_t(2 * c) * pw;
-                const int w = p - 1;
+                const int w = wP;
                 u32 hi = 0, lo = 0;
-                if (w >= 0 && w < (lc + 31) / 32) {
+                if (w >= 0 && 32 * w < lc) {
                     const int e = lc - 32 * (w + 1);  // first fwd bit of the window
                     u32 xh, xl;
                     if (e >= 0) {
@@ -1024,34 +1221,25 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
                 L.cpl[size_t(2 * c + 1) * pw + p] = make_uint2(hi, lo);
             }
             __syncthreads();
-            // each wave aligns a candidate at a time and leaves its two keys
-            // in LDS; the keys of the whole chunk are then decoded and the
-            // orientations chosen one thread per candidate (decoding in the
-            // aligning wave's lane 0 would issue every instruction for the
-            // whole wave)
+            // the waves leave every candidate's two keys in LDS; the keys of
+            // the whole chunk are then decoded and the orientations chosen
+            // one thread per candidate
             {
+                const int waveU = __builtin_amdgcn_readfirstlane(wave);
                 AlignCtx A;
                 A.ap = L.ap;
+                A.arp = L.arp;
                 A.cpl = L.cpl;
                 A.mst = L.mst;
                 A.keys = L.keys;
-                A.survA = L.keys + 2 * dims.chunk + 2 * kSurvivors * wave;
+                A.survA = L.keys + 2 * dims.chunk + 2 * kSurvivors * waveU;
                 A.survB = A.survA + kSurvivors;
                 A.la = la;
                 A.pw = pw;
                 A.minov = minovA;
+                A.same = sFlag == 0;
                 A.maxErrorRate = P.maxErrorRate;
-                int count = 0;  // queued survivors of this wave (wave-uniform)
-                for (int c = wave; c < nc; c += nwaves) {
-                    if (lane == 0) {
-                        CARE_CHECK(c0 + c < n);
-                        L.keys[2 * c] = ~0u;
-                        L.keys[2 * c + 1] = ~0u;
-                    }
-                    wave_sync();
-                    align_wave(A, c, L.mst[c].len, count);
-                }
-                if (count > 0) finish_survivors(A, count);
+                align_chunk(A, nc, waveU, nwaves);
             }
             __syncthreads();
             for (int c = tid; c < nc; c += blockDim.x)
@@ -1123,10 +1311,8 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
         // ---- phase C: MSA + refinement (include/corrector.hpp:1307-1421) ----
         CandMeta* cur = metaB;
         CandMeta* other = metaA;
-        // MSA columns read beyond the anchor: candidate correction reaches
-        // new_columns past it, gate features two columns past a corrected read
-        const int margin = P.correctCandidates ? P.newColumns + 2 : 2;
-        Msa msa = build_msa<!kGated>(P, L, dims, cur, m, la, margin, &sMin, &sMax);
+        const int margin = msa_margin(kGated, P.correctCandidates, P.newColumns);
+        Msa msa = build_msa(P, L, dims, cur, m, la, margin, &sMin, &sMax);
         const int maxIter = kRefine ? P.maxRefinements : 0;  // the gated mode skips refinement
         for (int iter = 0; iter < maxIter && m > 0; iter++) {
             // src/msa.cpp:532-734
@@ -1204,7 +1390,7 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
             cur = other;
             other = t;
             m = m2;
-            msa = build_msa<!kGated>(P, L, dims, cur, m, la, margin, &sMin, &sMax);
+            msa = build_msa(P, L, dims, cur, m, la, margin, &sMin, &sMax);
         }
 
         // ---- phase D: anchor correction (src/msa.cpp:304-453, include/corrector.hpp:1423-1472) ----
@@ -1409,20 +1595,28 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
 }
 
 // LDS shape of k_correct; MSA chunks hold up to 256 candidates and about
-// 16 KiB of staged rows
+// 16 KiB of staged rows; column arrays span the anchor and the margin
 // chunk: candidates staged per MSA pass (0 = about 16 KB of staged rows)
-static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk) {
+// margin: MSA columns held on either side of the anchor's
+static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk, int margin) {
     LdsDims d;
     d.pitch = (maxLen + 15) / 16;
     d.qpitch = useQuality ? qpitch : 0;
     d.hw = (maxLen + 31) / 32;
     d.maxLen = maxLen;
-    d.cols = 3 * maxLen + 2;
+    d.cols = int(std::min<long long>(3LL * maxLen + 2, maxLen + 2LL * margin));
     d.waves = threads / kWave;
     // LDS per staged candidate: record, 2-bit and quality rows, bit planes
     const int rowBytes = int(sizeof(CandMeta)) + 4 * (d.pitch + d.qpitch) + 2 * int(sizeof(uint2)) * d.pw();
     d.chunk = chunk > 0 ? chunk : std::max(16, std::min(256, 16384 / rowBytes));
     d.gated = gated;
+    auto inverse = [](int words) { return words ? (65536 + words - 1) / words : 0; };
+    d.stepS = threads / d.pitch;
+    d.stepQ = d.qpitch ? threads / d.qpitch : 0;
+    d.stepP = threads / d.pw();
+    d.invS = inverse(d.pitch);
+    d.invQ = inverse(d.qpitch);
+    d.invP = inverse(d.pw());
     if (gated) {
         // the staging area doubles as the gates' feature tiles and MLP scratch
         // (bit 0: anchor gate, two waves; bit 1: candidate gate, every wave)
@@ -1434,12 +1628,28 @@ static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, in
     return d;
 }
 
-size_t correct_lds_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk) {
-    return make_dims(maxLen, useQuality, qpitch, threads, gated, chunk).bytes();
+size_t correct_lds_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk,
+                         int correctCandidates, int newColumns) {
+    return make_dims(maxLen, useQuality, qpitch, threads, gated, chunk,
+                     msa_margin((gated & 1) != 0, correctCandidates, newColumns)).bytes();
+}
+
+// A launch shape is accepted for a read length if its staging area and 37
+// bytes for each of 3 maxLen + 2 columns (an MSA of candidates that reach a
+// whole read past both ends of the anchor) stay within kMaxLdsBytes.  The
+// kernel itself needs less, see make_dims.
+size_t correct_capacity_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk) {
+    const LdsDims d = make_dims(maxLen, useQuality, qpitch, threads, gated, chunk, 0);
+    const size_t cols = 3 * size_t(maxLen) + 2, c = size_t(d.chunk);
+    size_t b = c * (sizeof(CandMeta) + sizeof(u32) * (d.pitch + d.qpitch) + 2 * sizeof(uint2) * d.pw() + 8);
+    b += 1024 + sizeof(u32) * d.pitch + sizeof(uint2) * d.pw() + (size_t(maxLen) + 3) / 4 * 4;
+    b += (cols + 3) / 4 * 4 + 36 * cols + 128 + 8 * size_t(kSurvivors) * size_t(d.waves);
+    if (gated & 1) b += 3 * ((size_t(maxLen) + 15) / 16 * 16);
+    return b;
 }
 
 int correct_msa_chunk(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk) {
-    return make_dims(maxLen, useQuality, qpitch, threads, gated, chunk).chunk;
+    return make_dims(maxLen, useQuality, qpitch, threads, gated, chunk, 0).chunk;
 }
 
 int correct_resident_blocks(int threads, size_t ldsBytes, int gated) {
@@ -1459,7 +1669,8 @@ int correct_gate_mode(int correctionType, int correctCandidates, int correctionT
 
 void launch_correct(const CorrectParams& p, int blocks, int threads, int chunk, hipStream_t stream) {
     const int gm = correct_gate_mode(p.correctionType, p.correctCandidates, p.correctionTypeCands);
-    const LdsDims d = make_dims(p.rs.maxLen, p.useQuality, p.rs.qpitch, threads, gm, chunk);
+    const LdsDims d = make_dims(p.rs.maxLen, p.useQuality, p.rs.qpitch, threads, gm, chunk,
+                                msa_margin((gm & 1) != 0, p.correctCandidates, p.newColumns));
     // the candidate gate has its own instantiation: its registers would lower
     // the occupancy of the anchor-only gated mode
     if (gm & 2)

@@ -196,7 +196,9 @@ void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigne
 // anchor gate (correction type 3), bit 1 the candidate gate
 int correct_gate_mode(int correctionType, int correctCandidates, int correctionTypeCands);
 void launch_correct(const CorrectParams& p, int blocks, int threads, int chunk, hipStream_t stream);
-size_t correct_lds_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk);
+size_t correct_lds_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk,
+                         int correctCandidates, int newColumns);
+size_t correct_capacity_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk);
 int correct_msa_chunk(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk);
 // correction workgroups resident per compute unit at once (occupancy)
 int correct_resident_blocks(int threads, size_t ldsBytes, int gated);
