@@ -33,7 +33,7 @@ void launch_scatter_values(const u64* sigs, u64 n, int h, int map, const u64* tk
 void launch_sort_buckets(const u32* toff, const u32* tcount, u64 tsize, u32* values, hipStream_t s);
 void launch_insert_triples(const u64* keys, const u32* offs, const u32* counts, u64 numKeys, u64* fkeys,
                            uint2* foffcnt, u64 fmask, int* overflow, hipStream_t s);
-void launch_reset_counters(int* queue, int* candOut, hipStream_t s);
+void launch_reset_counters(int* queue, int* candOut, int* heavy, hipStream_t s);
 }  // namespace care_engine
 
 using namespace care_engine;
@@ -150,7 +150,7 @@ struct care_context {
     int maxCand = 0;
     int queryCap = 0;  // hit lists sorted in LDS up to this length, longer ones in global scratch
     int queryRegMax = 0;  // hit lists sorted in registers up to this length (0 = kernel maximum)
-    int blockThreads = 256;  // correction workgroup
+    int blockThreads = 0;    // correction workgroup (0 = automatic, see correct_threads)
     int blocksPerCU = 0;     // persistent correction workgroups per CU (0 = resident maximum)
     int msaChunk = 0;        // candidates per MSA staging pass (0 = automatic)
     int requestedBatch = 0;
@@ -166,7 +166,9 @@ struct care_context {
     DevBuf<u32> candOutIds;
     DevBuf<char> candOutSeq;
     int candOutCap = 0;
-    DevBuf<int> counters;  // [0] queue head, [1] candidate output count
+    DevBuf<int> counters;  // [0] queue head, [1] candidate output count, [2] recorded columns,
+                           // [32], [33] heavy anchors of even and odd device batches
+    DevBuf<u32> heavy;     // anchors with long candidate lists, of a batch
     DevBuf<unsigned long long> rawHits;
     DevBuf<float> qweights;
     PinnedBuf<int> hInts;
@@ -228,6 +230,7 @@ void ensure_batch(care_context* ctx, int batch) {
     ctx->rawCount.alloc(batch);
     ctx->metaA.alloc(size_t(batch) * mc);
     ctx->metaB.alloc(size_t(batch) * mc);
+    ctx->heavy.alloc(batch);
     ctx->outStatus.alloc(batch);
     ctx->outPitch = (ctx->rs.maxLen + 15) / 16 * 16;
     ctx->outSeq.alloc(size_t(batch) * ctx->outPitch);
@@ -256,17 +259,36 @@ int default_batch(care_context* ctx) {
     return int(b & ~size_t(1));
 }
 
+// Threads of a correction workgroup over n anchors, unless they were set.
+// Two wavefronts an anchor take the least time in all (fewer barriers and idle
+// wavefronts; 1M reads 2x150: plain 35.0 ms, 44.7 with four wavefronts, gated
+// 18.5 against 27.1), four the least time for one anchor.  The latter decides
+// where there are few anchors for the workgroups the device holds, and, when
+// candidate lists have no limit, while a long list of a repeat (thousands of
+// candidates) takes as long as all others together: 40,000 anchors of 300
+// bases 2.41 against 2.45 ms, 10,000 of 100-250 bases 1.27 against 1.77.
+int correct_threads(const care_context* ctx, int n) {
+    if (ctx->blockThreads) return ctx->blockThreads;
+    const int fill = 8 * ctx->numCUs;
+    return n > (ctx->opt.candidate_limit > 0 ? fill : 32 * fill) ? 128 : 256;
+}
+
+// Candidates from which an anchor is corrected before the others: about twice
+// what reads outside repeats have at this coverage.
+int heavy_min(const care_context* ctx) { return std::max(96, int(ctx->opt.coverage * 3.0f)); }
+
 }  // namespace
 
 namespace care_engine {
-__global__ void k_reset_counters(int* queue, int* candOut) {
+__global__ void k_reset_counters(int* queue, int* candOut, int* heavy) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         queue[0] = 0;
         if (candOut) candOut[0] = 0;
+        if (heavy) heavy[0] = heavy[1] = 0;
     }
 }
-void launch_reset_counters(int* queue, int* candOut, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, queue, candOut);
+void launch_reset_counters(int* queue, int* candOut, int* heavy, hipStream_t s) {
+    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, queue, candOut, heavy);
 }
 }  // namespace care_engine
 
@@ -342,7 +364,7 @@ int care_context_create(int device, const care_options* opt, care_context** out)
         }
         ctx->qweights.alloc(256);
         HIP_TRY(hipMemcpy(ctx->qweights.p, w, sizeof(w), hipMemcpyHostToDevice));
-        ctx->counters.alloc(4);
+        ctx->counters.alloc(40);
         ctx->rawHits.alloc(2);
         ctx->hInts.alloc(8);
         ctx->hU64.alloc(4);
@@ -401,7 +423,7 @@ int care_set_tuning(care_context* ctx, const care_tuning* t) {
     if (rm != 0 && (rm < 64 || rm > 2048 || (rm & (rm - 1))))
         return fail(CARE_ERR_ARGUMENT, "query_register_hits must be 0 or a power of two in 64..2048");
     ctx->requestedBatch = t->batch_anchors;
-    ctx->blockThreads = t->correct_threads ? t->correct_threads : 256;
+    ctx->blockThreads = t->correct_threads;
     ctx->blocksPerCU = t->correct_blocks_per_cu;
     ctx->msaChunk = t->msa_chunk;
     ctx->queryCap = q;
@@ -412,7 +434,7 @@ int care_set_tuning(care_context* ctx, const care_tuning* t) {
 int care_get_tuning(care_context* ctx, care_tuning* out) {
     if (!ctx || !out) return fail(CARE_ERR_ARGUMENT, "null argument");
     const auto& o = ctx->opt;
-    const int T = ctx->blockThreads;
+    const int T = correct_threads(ctx, 1 << 20);  // of a call that fills the device
     const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
     out->batch_anchors = ctx->rs.n ? default_batch(ctx) : ctx->requestedBatch;
     out->correct_threads = T;
@@ -1159,9 +1181,10 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         HIP_TRY(hipSetDevice(ctx->device));
         const int B = default_batch(ctx);
         ensure_batch(ctx, B);
-        const int T = ctx->blockThreads;
+        const int T = correct_threads(ctx, std::min(n, B));
         const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
-        const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk);
+        const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch,
+                                                   ctx->blockThreads ? T : 256, gatedK, ctx->msaChunk);
         if (need > size_t(kMaxLdsBytes))
             return fail(CARE_ERR_CAPACITY, "reads of length %d need %zu bytes of LDS per correction workgroup (limit %d)",
                         ctx->rs.maxLen, need, kMaxLdsBytes);
@@ -1182,6 +1205,8 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         P.candOutCount = ctx->counters.p + 1;
         P.candOutCap = ctx->candOutCap;
         P.queueHead = ctx->counters.p;
+        P.heavyList = ctx->heavy.p;
+        P.heavyMin = heavy_min(ctx);
         // Every device batch writes its slice of call-wide anchor outputs and
         // appends its candidate corrections to a call-wide candidate buffer
         // (one counter over the call), so the batches run back to back with
@@ -1241,17 +1266,22 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
             }
             try {
                 launch_fill_u64(reinterpret_cast<u64*>(ctx->rawHits.p), 2, 0, s);  // totals over the call
-                launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, s);  // candidate results over the call
+                // candidate results over the call, heavy anchors of the first batches
+                launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, ctx->counters.p + 32, s);
                 for (int done = 0, nb = 0; done < n; done += nb, bi++) {
                     nb = next_batch(B, n, n - done);
                     hipEvent_t* e = &ctx->batchEv[size_t(3 * bi)];
                     if (!graph) HIP_TRY(hipEventRecord(e[0], s));
+                    int* heavyCount = ctx->counters.p + 32 + (bi & 1);
                     launch_query(ctx->rs, ctx->tables, first + done, nb, ctx->maxCand, ctx->queryCap,
                                  ctx->queryRegMax, o.exclude_ambiguous, o.candidate_limit, ctx->candIds.p,
-                                 ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), ctx->rawCount.p, s);
-                    launch_sum_counts(ctx->rawCount.p, ctx->candCount.p, nb, ctx->rawHits.p, s);
+                                 ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), ctx->rawCount.p, s,
+                                 QueryAnchors(), QueryHeavy{ctx->heavy.p, heavyCount, P.heavyMin});
+                    launch_sum_counts(ctx->rawCount.p, ctx->candCount.p, nb, ctx->rawHits.p,
+                                      ctx->counters.p + 32 + ((bi + 1) & 1), s);
+                    P.heavyCount = heavyCount;
                     if (!graph) HIP_TRY(hipEventRecord(e[1], s));
-                    launch_reset_counters(ctx->counters.p, nullptr, s);  // work queue of this batch
+                    launch_reset_counters(ctx->counters.p, nullptr, nullptr, s);  // work queue of this batch
                     P.firstAnchor = first + done;
                     P.numAnchors = nb;
                     P.outStatus = ctx->outStatus.p + size_t(done);
@@ -1873,8 +1903,14 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         }
         ctx->queryCap = bestCap;
         ctx->queryRegMax = bestReg;
-        query(bestCap, bestReg);
+        launch_reset_counters(ctx->counters.p, nullptr, ctx->counters.p + 32, s);
+        launch_query(ctx->rs, ctx->tables, first, n, ctx->maxCand, bestCap, bestReg, o.exclude_ambiguous, candLimit,
+                     ctx->candIds.p, ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), nullptr, s,
+                     QueryAnchors(), QueryHeavy{ctx->heavy.p, ctx->counters.p + 32, heavy_min(ctx)});
         HIP_TRY(hipGetLastError());
+        P.heavyList = ctx->heavy.p;
+        P.heavyCount = ctx->counters.p + 32;
+        P.heavyMin = heavy_min(ctx);
         // correction: 2, 3 or 4 wavefronts per anchor, automatic and halved MSA chunks
         P.candIds = ctx->candIds.p;
         P.candCount = ctx->candCount.p;
@@ -1905,7 +1941,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
                 const int bpc = ctx->blocksPerCU > 0 ? ctx->blocksPerCU : correct_resident_blocks(T, lds, gatedK);
                 const int blocks = std::max(1, std::min(n, ctx->numCUs * bpc));
                 const float ms = timed([&] {
-                    launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, s);
+                    launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, nullptr, s);
                     launch_correct(P, blocks, T, chunk, s);
                 });
                 if (ms < bestC) {
@@ -2012,9 +2048,10 @@ extern "C" int care_correct_batch_noalloc(care_context* ctx, uint64_t first, int
     if (const int rc = scratch_address(ctx, &base)) return rc;
     try {
         HIP_TRY(hipSetDevice(ctx->device));
-        const int T = ctx->blockThreads;
+        const int T = correct_threads(ctx, std::min(n, B));
         const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
-        const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, ctx->msaChunk);
+        const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch,
+                                                   ctx->blockThreads ? T : 256, gatedK, ctx->msaChunk);
         if (need > size_t(kMaxLdsBytes))
             return fail(CARE_ERR_CAPACITY, "reads of length %d need %zu bytes of LDS per correction workgroup (limit %d)",
                         ctx->rs.maxLen, need, kMaxLdsBytes);
@@ -2058,7 +2095,7 @@ extern "C" int care_correct_batch_noalloc(care_context* ctx, uint64_t first, int
                          o.exclude_ambiguous, o.candidate_limit, candIds, candCount, reinterpret_cast<u32*>(metaA),
                          nullptr, s);
             // queue head and candidate result count start at zero in every batch
-            launch_reset_counters(counters, counters + 1, s);
+            launch_reset_counters(counters, counters + 1, nullptr, s);
             P.firstAnchor = first + done;
             P.numAnchors = nb;
             P.outStatus = outStatus;

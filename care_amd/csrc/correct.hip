@@ -209,15 +209,16 @@ __device__ __forceinline__ void msa_add(MsaSums& s, u32 b, float w) {
 // the body has no branch and 2-bit qualities share the bases' word index and
 // bit offset; the bins' weights are read from LDS (selects cost more).  A
 // candidate that does not cover the column reads words of other rows, which
-// are dropped.  Left rolled (unrolled copies hold more loads in flight and
-// raise the registers of the calling kernels); the next candidate's record is
-// read one iteration ahead.
+// are dropped.  Its chain of reads bounds it (one wavefront of a workgroup
+// has most of the listed columns), so four candidates' reads are in flight
+// and the next record is read ahead: 33.8 ms per 1M reads against 35.0 left
+// rolled, at the same four wavefronts per SIMD.
 template <int kQ>
 __device__ __forceinline__ void msa_add_staged(const Lds& L, int nc, int colRel, int pitch, int qpitch, MsaSums& s) {
     CandMeta next = L.mst[0];
     const u32* row = L.rows;
     const u32* qrow = L.qrows;
-#pragma unroll 1
+#pragma unroll 4
     for (int c = 0; c < nc; c++, row += pitch, qrow += qpitch) {
         const CandMeta cm = next;
         next = L.mst[c + 1 < nc ? c + 1 : c];
@@ -1047,6 +1048,8 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
     const int nwaves = blockDim.x / kWave;
     const int pw = dims.pw();
 
+    // read once: the queue's atomics keep this line busy
+    const int nHeavy = P.heavyCount ? __builtin_amdgcn_readfirstlane(*P.heavyCount) : 0;
     if (P.useQuality) {
         for (int i = threadIdx.x; i < 256; i += blockDim.x) L.qw[i] = P.qweights[i];
         // weights of the characters of 2-bit ('$', '(', '1', '9') and 1-bit
@@ -1065,9 +1068,15 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
         const int wave = tid / kWave;
         if (tid == 0) sAnchor = atomicAdd(P.queueHead, 1);
         __syncthreads();
-        const int a = sAnchor;
+        const int q = sAnchor;
         __syncthreads();
-        if (a >= P.numAnchors) break;
+        // first the anchors with long candidate lists, then all others in
+        // order: taken in read order, one near the end of the batch kept a
+        // workgroup busy for up to 50 average anchors' time after the rest of
+        // the device had drained
+        if (q >= P.numAnchors + nHeavy) break;
+        const int a = q < nHeavy ? int(P.heavyList[q]) : q - nHeavy;
+        if (q >= nHeavy && nHeavy > 0 && P.candCount[a] > P.heavyMin) continue;
 
         const u64 id = P.firstAnchor + u64(a);
         CARE_CHECK(id < rs.n);
@@ -1447,21 +1456,21 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
                     nd += cnt;
                 }
                 __syncthreads();
-                bf16raw* xt = reinterpret_cast<bf16raw*>(L.gscr);                  // [32][32]
-                float* zt = reinterpret_cast<float*>(L.gscr + 32 * kMlpIn * 2);   // [32]
-                char* tileScr = L.gscr + 32 * kMlpIn * 2 + 32 * 4;                // 2 x kMlpTileScratch
-                float* ft = reinterpret_cast<float*>(tileScr + 2 * kMlpTileScratch);  // [32][33] features
-                // the tiles overlay the candidate staging area, which ends at qw
-                CARE_CHECK(reinterpret_cast<char*>(ft + 32 * (kMlpIn + 1)) <= reinterpret_cast<char*>(L.qw));
-                for (int g0 = 0; g0 < nd; g0 += 32) {
-                    const int ng = min(32, nd - g0);
-                    // thread and wave indices made opaque: the feature-tile
-                    // and MLP addresses are computed here rather than hoisted
-                    // out of the anchor loop (which would keep them in
-                    // registers through every phase and cost a wave per SIMD)
-                    int gt = tid, gw = wave;
-                    asm volatile("" : "+v"(gt), "+v"(gw));
-                    if (gt < 32) {
+                bf16raw* xt = reinterpret_cast<bf16raw*>(L.gscr);              // [16][32]
+                float* zt = reinterpret_cast<float*>(L.gscr + 16 * kMlpIn * 2);  // [16]
+                char* tileScr = L.gscr + 16 * kMlpIn * 2 + 16 * 4;             // kMlpTileScratch
+                float* ft = reinterpret_cast<float*>(tileScr + kMlpTileScratch);  // [16][33] features
+                // the tile overlays the candidate staging area, which ends at qw
+                CARE_CHECK(reinterpret_cast<char*>(ft + 16 * (kMlpIn + 1)) <= reinterpret_cast<char*>(L.qw));
+                for (int g0 = 0; g0 < nd; g0 += 16) {
+                    const int ng = min(16, nd - g0);
+                    // thread index made opaque: the feature-tile and MLP
+                    // addresses are computed here rather than hoisted out of
+                    // the anchor loop (which would keep them in registers
+                    // through every phase and cost a wave per SIMD)
+                    int gt = tid;
+                    asm volatile("" : "+v"(gt));
+                    if (gt < 16) {
                         float* f = ft + gt * (kMlpIn + 1);
                         if (gt < ng) {
                             const int i = int(L.dec[g0 + gt]);
@@ -1485,7 +1494,7 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
                         }
                     }
                     __syncthreads();
-                    if (P.gateParams && wave < 2 && 16 * wave < ng) {
+                    if (P.gateParams && wave == 0) {
                         MlpWeights W;
                         W.w1 = P.gateW1;
                         W.w2 = P.gateW2;
@@ -1495,7 +1504,7 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
                         W.b3 = P.gateParams + kMlpB3;
                         W.w4 = P.gateParams + kMlpW4;
                         W.b4 = P.gateParams[kMlpB4];
-                        mlp_tile_forward(W, xt + 16 * gw * kMlpIn, tileScr + gw * kMlpTileScratch, zt + 16 * gw);
+                        mlp_tile_forward(W, xt, tileScr, zt);
                     }
                     __syncthreads();
                     if (tid < ng) L.gacc[L.dec[g0 + tid]] = (P.gateParams && zt[tid] >= P.gateLogit) ? 1 : 0;
@@ -1608,8 +1617,19 @@ static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, in
     d.waves = threads / kWave;
     // LDS per staged candidate: record, 2-bit and quality rows, bit planes
     const int rowBytes = int(sizeof(CandMeta)) + 4 * (d.pitch + d.qpitch) + 2 * int(sizeof(uint2)) * d.pw();
-    d.chunk = chunk > 0 ? chunk : std::max(16, std::min(256, 16384 / rowBytes));
     d.gated = gated;
+    d.chunk = 0;
+    if (chunk > 0) {
+        d.chunk = chunk;
+    } else {
+        // the kernel's registers allow 16 wavefronts per compute unit: the
+        // chunk is what leaves LDS for as many workgroups (2 x 150 reads, 128
+        // threads, 1M reads: 36.5 ms with 48 candidates and 8 workgroups,
+        // 39.7 with 32 and 8, 44.6 with 73 and 6)
+        const long long share = 160 * 1024 / (16 * kWave / threads) - 512;  // 512: static LDS
+        const long long left = share - (long long)d.bytes();
+        d.chunk = int(std::max(16LL, std::min({256LL, 16384LL / rowBytes, left / (rowBytes + 8)})));
+    }
     auto inverse = [](int words) { return words ? (65536 + words - 1) / words : 0; };
     d.stepS = threads / d.pitch;
     d.stepQ = d.qpitch ? threads / d.qpitch : 0;
@@ -1619,9 +1639,9 @@ static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, in
     d.invP = inverse(d.pw());
     if (gated) {
         // the staging area doubles as the gates' feature tiles and MLP scratch
-        // (bit 0: anchor gate, two waves; bit 1: candidate gate, every wave)
+        // (bit 0: anchor gate, one wave; bit 1: candidate gate, every wave)
         int need = 0;
-        if (gated & 1) need = 32 * kMlpIn * 2 + 32 * 4 + 2 * kMlpTileScratch + 32 * (kMlpIn + 1) * 4;
+        if (gated & 1) need = kCandGateTile;
         if (gated & 2) need = std::max(need, d.waves * cand_gate_scratch(maxLen));
         while (d.chunk * rowBytes < need) d.chunk++;
     }
@@ -1639,9 +1659,14 @@ size_t correct_lds_bytes(int maxLen, int useQuality, int qpitch, int threads, in
 // whole read past both ends of the anchor) stay within kMaxLdsBytes.  The
 // kernel itself needs less, see make_dims.
 size_t correct_capacity_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk) {
-    const LdsDims d = make_dims(maxLen, useQuality, qpitch, threads, gated, chunk, 0);
-    const size_t cols = 3 * size_t(maxLen) + 2, c = size_t(d.chunk);
-    size_t b = c * (sizeof(CandMeta) + sizeof(u32) * (d.pitch + d.qpitch) + 2 * sizeof(uint2) * d.pw() + 8);
+    const LdsDims d = make_dims(maxLen, useQuality, qpitch, threads, 0, 16, 0);
+    const size_t cols = 3 * size_t(maxLen) + 2;
+    const size_t row = sizeof(CandMeta) + sizeof(u32) * (d.pitch + d.qpitch) + 2 * sizeof(uint2) * d.pw();
+    size_t c = chunk > 0 ? size_t(chunk) : std::max<size_t>(16, std::min<size_t>(256, 16384 / row));
+    size_t need = gated & 1 ? 14592 : 0;
+    if (gated & 2) need = std::max<size_t>(need, size_t(d.waves) * cand_gate_scratch(maxLen));
+    while (c * row < need) c++;
+    size_t b = c * (row + 8);
     b += 1024 + sizeof(u32) * d.pitch + sizeof(uint2) * d.pw() + (size_t(maxLen) + 3) / 4 * 4;
     b += (cols + 3) / 4 * 4 + 36 * cols + 128 + 8 * size_t(kSurvivors) * size_t(d.waves);
     if (gated & 1) b += 3 * ((size_t(maxLen) + 15) / 16 * 16);

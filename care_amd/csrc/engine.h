@@ -108,6 +108,10 @@ struct CorrectParams {
     int* candOutCount;
     int candOutCap;
     int* queueHead;
+    // anchors with more than heavyMin candidates, taken first (null: none)
+    const u32* heavyList;
+    const int* heavyCount;
+    int heavyMin;
     const float* qweights;  // 256 entries
     // options
     int pairedEnd;
@@ -178,20 +182,30 @@ struct QueryAnchors {
     const u32* ids = nullptr;
     const int* lens = nullptr;
 };
+// Where a query lists the anchors that keep more than `min` candidates
+// (list null: nowhere); count starts at 0.
+struct QueryHeavy {
+    u32* list = nullptr;
+    int* count = nullptr;
+    int min = 0;
+};
 // spill: 4 * maxCand words per anchor of the batch (sort/merge buffers of
 // anchors with more than capL hits); regMax: longest hit list sorted in
 // registers (0 = the kernel's maximum, 1024), longer lists are merged;
 // rawCount (may be null): table hits per anchor before de-duplication
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
                   int excludeAmbiguous, int candLimit, u32* candIds, int* candCount, u32* spill, int* rawCount,
-                  hipStream_t stream, const QueryAnchors& anchors = QueryAnchors());
+                  hipStream_t stream, const QueryAnchors& anchors = QueryAnchors(),
+                  const QueryHeavy& heavy = QueryHeavy());
 // read-store gathers by read id into device buffers (store.hip)
 void launch_gather_sequences(const DevReadStore& rs, const u32* ids, int n, u32* out, int outPitch, hipStream_t s);
 void launch_gather_lengths(const DevReadStore& rs, const u32* ids, int n, int* out, hipStream_t s);
 void launch_gather_qualities(const DevReadStore& rs, const u32* ids, int n, char* out, int outPitch, hipStream_t s);
 void launch_gather_ambiguous(const DevReadStore& rs, const u32* ids, int n, u8* out, hipStream_t s);
 // totals[0] += sum(rawCount[0..n)), totals[1] += sum(candCount[0..n))
-void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, hipStream_t s);
+// nextHeavy[0] = 0: the heavy-anchor count of the batch after
+void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, int* nextHeavy,
+                       hipStream_t s);
 // chunk: candidates staged per MSA pass (0 = automatic); gated: bit 0 the
 // anchor gate (correction type 3), bit 1 the candidate gate
 int correct_gate_mode(int correctionType, int correctCandidates, int correctionTypeCands);

@@ -656,7 +656,8 @@ __device__ __forceinline__ int keep_top(u32* out, HitBuf hits, int written, int 
 template <int kMaxK>
 __global__ void __launch_bounds__(256) k_query(DevReadStore rs, DevTables t, u64 first, int n, int maxCand, int capL,
                                                int regMax, int excludeAmbiguous, int candLimit, u32* candIds,
-                                               int* candCount, u32* spill, int* rawCount, QueryAnchors qa) {
+                                               int* candCount, u32* spill, int* rawCount, QueryAnchors qa,
+                                               QueryHeavy heavy) {
     HIP_DYNAMIC_SHARED(uint4, ldsRaw)
     const int wave = threadIdx.x / kWave;
     const int wpb = blockDim.x / kWave;
@@ -741,6 +742,7 @@ __global__ void __launch_bounds__(256) k_query(DevReadStore rs, DevTables t, u64
         if (lane == 0) {
             candCount[a] = written;
             if (rawCount) rawCount[a] = total;
+            if (heavy.list && written > heavy.min) heavy.list[atomicAdd(heavy.count, 1)] = u32(a);
         }
         wave_sync_mem();  // counts and buffers are rewritten by the next anchor
     }
@@ -749,7 +751,7 @@ __global__ void __launch_bounds__(256) k_query(DevReadStore rs, DevTables t, u64
 // totals[0] += sum of raw hit counts, totals[1] += sum of candidate counts
 // (one workgroup, so no atomics)
 __global__ void __launch_bounds__(1024) k_sum_counts(const int* rawCount, const int* candCount, int n,
-                                                     unsigned long long* totals) {
+                                                     unsigned long long* totals, int* nextHeavy) {
     __shared__ unsigned long long part[2][16];
     unsigned long long r = 0, c = 0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -773,6 +775,7 @@ __global__ void __launch_bounds__(1024) k_sum_counts(const int* rawCount, const 
         }
         totals[0] += r;
         totals[1] += c;
+        nextHeavy[0] = 0;
     }
 }
 
@@ -785,7 +788,7 @@ int query_lds_bytes(int h, int cap, int maxLen, int threads, int candLimit, int 
 
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
                   int excludeAmbiguous, int candLimit, u32* candIds, int* candCount, u32* spill, int* rawCount,
-                  hipStream_t stream, const QueryAnchors& qa) {
+                  hipStream_t stream, const QueryAnchors& qa, const QueryHeavy& heavy) {
     if (n <= 0) return;
     const int threads = 256;
     const int wpb = threads / kWave;
@@ -799,15 +802,16 @@ void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, 
     // used only when asked for lists of more than 1024 hits
     if (regMax > 16 * kWave)
         hipLaunchKernelGGL(k_query<32>, dim3(blocks), dim3(threads), lds, stream, rs, t, first, n, maxCand, capL, regMax,
-                           excludeAmbiguous, candLimit, candIds, candCount, spill, rawCount, qa);
+                           excludeAmbiguous, candLimit, candIds, candCount, spill, rawCount, qa, heavy);
     else
         hipLaunchKernelGGL(k_query<16>, dim3(blocks), dim3(threads), lds, stream, rs, t, first, n, maxCand, capL, regMax,
-                           excludeAmbiguous, candLimit, candIds, candCount, spill, rawCount, qa);
+                           excludeAmbiguous, candLimit, candIds, candCount, spill, rawCount, qa, heavy);
 }
 
-void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, hipStream_t s) {
+void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, int* nextHeavy,
+                       hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_sum_counts, dim3(1), dim3(1024), 0, s, rawCount, candCount, n, totals);
+    hipLaunchKernelGGL(k_sum_counts, dim3(1), dim3(1024), 0, s, rawCount, candCount, n, totals, nextHeavy);
 }
 
 }  // namespace care_engine
