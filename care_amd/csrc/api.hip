@@ -157,7 +157,7 @@ struct care_context {
     DevBuf<u32> candIds;
     DevBuf<int> candCount;
     DevBuf<int> rawCount;  // table hits per anchor of a batch (statistics)
-    DevBuf<CandMeta> metaA, metaB;
+    DevBuf<CandMeta> metaA, metaB;  // a row of maxCand records per correction workgroup
     DevBuf<u8> outStatus;
     DevBuf<char> outSeq;
     int outPitch = 0;
@@ -221,15 +221,28 @@ struct care_context {
 
 namespace {
 
-// Batch buffers sized for `batch` anchors.
-void ensure_batch(care_context* ctx, int batch) {
+// Record rows of the correction workgroups, and spill rows of the query's
+// wavefronts, which are as long as a row of records.
+void ensure_rows(care_context* ctx, int spillRows, int blocks) {
+    const size_t mc = size_t(ctx->maxCand);
+    const size_t a = size_t(std::max(spillRows, blocks)) * mc, b = size_t(blocks) * mc;
+    if (ctx->metaA.n < a) ctx->metaA.alloc(a);
+    if (ctx->metaB.n < b) ctx->metaB.alloc(b);
+}
+
+// Batch buffers of a call over n anchors in device batches of up to B: small
+// calls take what they need, rounded up to a power of two, so a program of a
+// few thousand reads does not allocate for 262,144 anchors.
+void ensure_batch(care_context* ctx, int B, int n) {
+    int batch = 1024;
+    while (batch < n && batch < B) batch *= 2;
+    batch = std::min(batch, B);
+    ensure_rows(ctx, query_spill_rows(batch), 0);
     if (batch <= ctx->batchCap) return;
     const size_t mc = size_t(ctx->maxCand);
     ctx->candIds.alloc(size_t(batch) * mc);
     ctx->candCount.alloc(batch);
     ctx->rawCount.alloc(batch);
-    ctx->metaA.alloc(size_t(batch) * mc);
-    ctx->metaB.alloc(size_t(batch) * mc);
     ctx->heavy.alloc(batch);
     ctx->outStatus.alloc(batch);
     ctx->outPitch = (ctx->rs.maxLen + 15) / 16 * 16;
@@ -245,15 +258,15 @@ void ensure_batch(care_context* ctx, int batch) {
     ctx->batchCap = batch;
 }
 
-// Anchors per device batch: the batch scratch (candidate ids and two
-// records per candidate slot, h x cap slots per anchor) gets a quarter of the
-// device memory free when the context was created, between 2 and 24 GiB, and
-// a batch holds at most 2^18 anchors.  Fewer, larger batches mean fewer
-// launches and fewer drains of the persistent correction kernel.
+// Anchors per device batch: the candidate lists (h x cap slots per anchor)
+// get a quarter of the device memory free when the context was created,
+// between 2 and 4 GiB, and a batch holds at most 2^18 anchors.  Fewer, larger
+// batches mean fewer launches and fewer drains of the persistent correction
+// kernel.
 int default_batch(care_context* ctx) {
     if (ctx->requestedBatch > 0) return ctx->requestedBatch;
-    const size_t perAnchor = size_t(ctx->maxCand) * (sizeof(u32) + 2 * sizeof(CandMeta)) + ctx->rs.maxLen + 64;
-    const size_t budget = std::min(std::max(ctx->freeAtCreate / 4, size_t(2) << 30), size_t(24) << 30);
+    const size_t perAnchor = size_t(ctx->maxCand) * sizeof(u32) + ctx->rs.maxLen + 64;
+    const size_t budget = std::min(std::max(ctx->freeAtCreate / 4, size_t(2) << 30), size_t(4) << 30);
     size_t b = budget / perAnchor;
     b = std::max<size_t>(256, std::min<size_t>(b, size_t(1) << 18));
     return int(b & ~size_t(1));
@@ -906,6 +919,7 @@ int care_minhash_import(care_context* ctx, const care_map_view* maps, int num_ma
         ctx->opt.num_hash_maps = num_maps;
         ctx->cap = results_per_map;
         ctx->maxCand = num_maps * results_per_map;
+        ctx->batchCap = 0;  // rows of candIds hold maxCand ids
         ctx->queryCap = std::min((ctx->maxCand + 15) / 16 * 16, kDefaultQueryCap);
         ctx->queryRegMax = 0;
         ctx->sigs.alloc(n * num_maps);
@@ -993,7 +1007,7 @@ int care_minhash_query(care_context* ctx, uint64_t first, int n, uint32_t* ids, 
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         const int B = default_batch(ctx);
-        ensure_batch(ctx, B);
+        ensure_batch(ctx, B, n);
         std::vector<int> counts;
         std::vector<u32> buf;
         uint64_t written = 0;
@@ -1180,7 +1194,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         const int B = default_batch(ctx);
-        ensure_batch(ctx, B);
+        ensure_batch(ctx, B, n);
         const int T = correct_threads(ctx, std::min(n, B));
         const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
         const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch,
@@ -1193,6 +1207,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         const int blocksPerCU = ctx->blocksPerCU > 0 ? ctx->blocksPerCU
                                                      : correct_resident_blocks(T, lds, gatedK | (P.gatedRefine ? 4 : 0));
         hipStream_t s = ctx->stream;
+        ensure_rows(ctx, 0, std::min(std::min(n, B), ctx->numCUs * blocksPerCU));
         P.candIds = ctx->candIds.p;
         P.candCount = ctx->candCount.p;
         P.metaA = ctx->metaA.p;
@@ -1860,7 +1875,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         const int B = default_batch(ctx);
         n = std::min(n, std::min(B, 65536)) & ~1;
         if (n == 0) n = 2 > int(ctx->rs.n - first) ? 1 : 2;
-        ensure_batch(ctx, B);
+        ensure_batch(ctx, B, n);
         hipStream_t s = ctx->stream;
         const int candLimit = o.candidate_limit;
         auto timed = [&](auto&& launch) {
@@ -1940,6 +1955,9 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
                                                      o.correct_candidates, o.new_columns_to_correct);
                 const int bpc = ctx->blocksPerCU > 0 ? ctx->blocksPerCU : correct_resident_blocks(T, lds, gatedK);
                 const int blocks = std::max(1, std::min(n, ctx->numCUs * bpc));
+                ensure_rows(ctx, 0, blocks);
+                P.metaA = ctx->metaA.p;
+                P.metaB = ctx->metaB.p;
                 const float ms = timed([&] {
                     launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, nullptr, s);
                     launch_correct(P, blocks, T, chunk, s);

@@ -1131,8 +1131,12 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
                 mateN = P.candCount[mate];
             }
         }
-        CandMeta* metaA = P.metaA + u64(a) * P.maxCand;
-        CandMeta* metaB = P.metaB + u64(a) * P.maxCand;
+        // one anchor at a time: its records live in the workgroup's own rows
+        // and stay in the caches (rows for every anchor of a batch came to
+        // 20 GB at 262,144 anchors of 2,400 candidate slots, whose allocation
+        // alone took 0.1 s)
+        CandMeta* metaA = P.metaA + u64(blockIdx.x) * P.maxCand;
+        CandMeta* metaB = P.metaB + u64(blockIdx.x) * P.maxCand;
         // candidate ids, lengths, 2-bit rows and pair flags of a chunk are
         // gathered into LDS by the whole block, so their global loads (and
         // the binary searches in the mate's candidate list) run in parallel

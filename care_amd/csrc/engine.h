@@ -98,7 +98,7 @@ struct CorrectParams {
     const u32* candIds;     // [numAnchors][maxCand]
     const int* candCount;   // [numAnchors]
     int maxCand;
-    CandMeta* metaA;        // [numAnchors][maxCand]
+    CandMeta* metaA;        // [workgroups][maxCand]
     CandMeta* metaB;
     u8* outStatus;
     char* outSeq;
@@ -182,6 +182,7 @@ struct QueryAnchors {
     const u32* ids = nullptr;
     const int* lens = nullptr;
 };
+int query_spill_rows(int n);
 // Where a query lists the anchors that keep more than `min` candidates
 // (list null: nowhere); count starts at 0.
 struct QueryHeavy {
@@ -189,8 +190,8 @@ struct QueryHeavy {
     int* count = nullptr;
     int min = 0;
 };
-// spill: 4 * maxCand words per anchor of the batch (sort/merge buffers of
-// anchors with more than capL hits); regMax: longest hit list sorted in
+// spill: 4 * maxCand words for each of query_spill_rows(n) wavefronts
+// (sort/merge buffers of anchors with more than capL hits); regMax: longest hit list sorted in
 // registers (0 = the kernel's maximum, 1024), longer lists are merged;
 // rawCount (may be null): table hits per anchor before de-duplication
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,

@@ -349,8 +349,8 @@ void launch_insert_triples(const u64* keys, const u32* offs, const u32* counts, 
 // stored signature value j, the h hit lists (each sorted ascending) are
 // gathered and merged pairwise, then unique, self and ambiguous reads are
 // removed in order.  Hit lists of up to `capL` entries are merged in the
-// wave's LDS slice; longer ones (heavy repeats) in the anchor's rows of the
-// global scratch `spill` (4 * maxCand words per anchor).
+// wave's LDS slice; longer ones (heavy repeats) in the wavefront's row of
+// the global scratch `spill` (4 * maxCand words).
 // ---------------------------------------------------------------------------
 // With candLimit > 0 only the candLimit candidates hit by the most maps are
 // kept (ties broken by smaller read id), still in ascending id order.
@@ -720,7 +720,8 @@ __global__ void __launch_bounds__(256) k_query(DevReadStore rs, DevTables t, u64
         wave_sync_mem();
 
         u32* out = candIds + u64(a) * maxCand;
-        u32* gs = spill + u64(a) * 4 * maxCand;  // [maxCand] + [maxCand] + hit bytes
+        // this wavefront's row: [maxCand] + [maxCand] + hit bytes
+        u32* gs = spill + (u64(blockIdx.x) * wpb + wave) * 4 * maxCand;
         u8* gh = reinterpret_cast<u8*>(gs + 2 * maxCand);
         int written;
         if (total <= capL) {
@@ -786,6 +787,11 @@ int query_lds_bytes(int h, int cap, int maxLen, int threads, int candLimit, int 
     return int(size_t(threads / kWave) * query_wave_lds_bytes(capL, candLimit));
 }
 
+// Wavefronts of a query over n anchors: at most 16,384, two to four times what
+// the 256 compute units hold at once, each taking every so manieth anchor; a
+// spill row per wavefront instead of per anchor bounds the scratch.
+int query_spill_rows(int n) { return std::min(n, 1 << 14); }
+
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
                   int excludeAmbiguous, int candLimit, u32* candIds, int* candCount, u32* spill, int* rawCount,
                   hipStream_t stream, const QueryAnchors& qa, const QueryHeavy& heavy) {
@@ -793,7 +799,7 @@ void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, 
     const int threads = 256;
     const int wpb = threads / kWave;
     const int lds = query_lds_bytes(t.h, maxCand / t.h, rs.maxLen, threads, candLimit, capL);
-    const int blocks = std::min((n + wpb - 1) / wpb, 1 << 16);
+    const int blocks = (query_spill_rows(n) + wpb - 1) / wpb;
     const bool wide = maxCand > 16 * kWave;  // lists may exceed the 16-per-lane network
     const int kernelMax = wide ? 32 * kWave : 16 * kWave;
     regMax = regMax > 0 ? std::min(regMax, kernelMax) : kernelMax;
