@@ -33,7 +33,7 @@ void launch_scatter_values(const u64* sigs, u64 n, int h, int map, const u64* tk
 void launch_sort_buckets(const u32* toff, const u32* tcount, u64 tsize, u32* values, hipStream_t s);
 void launch_insert_triples(const u64* keys, const u32* offs, const u32* counts, u64 numKeys, u64* fkeys,
                            uint2* foffcnt, u64 fmask, int* overflow, hipStream_t s);
-void launch_reset_counters(int* queue, int* candOut, int* heavy, hipStream_t s);
+void launch_reset_counters(int* queue, int* candOut, int* heavy, unsigned long long* totals, hipStream_t s);
 }  // namespace care_engine
 
 using namespace care_engine;
@@ -157,6 +157,10 @@ struct care_context {
     DevBuf<u32> candIds;
     DevBuf<int> candCount;
     DevBuf<int> rawCount;  // table hits per anchor of a batch (statistics)
+    // packed candidate lists of a query (care_minhash_query)
+    DevBuf<u64> packStarts;
+    DevBuf<int> packOffsets;
+    DevBuf<u32> packed;
     DevBuf<CandMeta> metaA, metaB;  // a row of maxCand records per correction workgroup
     DevBuf<u8> outStatus;
     DevBuf<char> outSeq;
@@ -293,15 +297,16 @@ int heavy_min(const care_context* ctx) { return std::max(96, int(ctx->opt.covera
 }  // namespace
 
 namespace care_engine {
-__global__ void k_reset_counters(int* queue, int* candOut, int* heavy) {
+__global__ void k_reset_counters(int* queue, int* candOut, int* heavy, unsigned long long* totals) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         queue[0] = 0;
         if (candOut) candOut[0] = 0;
         if (heavy) heavy[0] = heavy[1] = 0;
+        if (totals) totals[0] = totals[1] = 0;
     }
 }
-void launch_reset_counters(int* queue, int* candOut, int* heavy, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, queue, candOut, heavy);
+void launch_reset_counters(int* queue, int* candOut, int* heavy, unsigned long long* totals, hipStream_t s) {
+    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, queue, candOut, heavy, totals);
 }
 }  // namespace care_engine
 
@@ -1008,8 +1013,6 @@ int care_minhash_query(care_context* ctx, uint64_t first, int n, uint32_t* ids, 
         HIP_TRY(hipSetDevice(ctx->device));
         const int B = default_batch(ctx);
         ensure_batch(ctx, B, n);
-        std::vector<int> counts;
-        std::vector<u32> buf;
         uint64_t written = 0;
         for (int done = 0; done < n; done += B) {
             const int nb = std::min(B, n - done);
@@ -1018,19 +1021,28 @@ int care_minhash_query(care_context* ctx, uint64_t first, int n, uint32_t* ids, 
                          ctx->candIds.p, ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), nullptr,
                          ctx->stream);
             HIP_TRY(hipGetLastError());
-            counts.resize(nb);
-            buf.resize(size_t(nb) * ctx->maxCand);
-            HIP_TRY(hipMemcpyAsync(counts.data(), ctx->candCount.p, sizeof(int) * nb, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(hipMemcpyAsync(buf.data(), ctx->candIds.p, sizeof(u32) * size_t(nb) * ctx->maxCand,
-                                   hipMemcpyDeviceToHost, ctx->stream));
+            // the lists are packed on the device, so that only their entries
+            // are copied, straight into the caller's arrays (the rows of
+            // candIds hold h x cap slots, of which 2 % are used at 30x)
+            if (ctx->packStarts.n < size_t(pack_scratch(nb))) ctx->packStarts.alloc(size_t(pack_scratch(nb)));
+            if (ctx->packOffsets.n < size_t(nb)) ctx->packOffsets.alloc(size_t(nb));
+            launch_pack_offsets(ctx->candCount.p, nb, written, ctx->packOffsets.p, ctx->packStarts.p, ctx->stream);
+            HIP_TRY(hipGetLastError());
+            HIP_TRY(hipMemcpyAsync(ctx->hU64.p, ctx->packStarts.p + nb, sizeof(u64), hipMemcpyDeviceToHost, ctx->stream));
             HIP_TRY(hipStreamSynchronize(ctx->stream));
-            for (int i = 0; i < nb; i++) {
-                const int c = counts[i];
-                if (written + c > ids_capacity) return fail(CARE_ERR_CAPACITY, "ids_capacity exceeded");
-                std::memcpy(ids + written, buf.data() + size_t(i) * ctx->maxCand, sizeof(u32) * c);
-                written += c;
-                offsets[done + i + 1] = int32_t(written);
-            }
+            const u64 total = ctx->hU64.p[0];
+            if (written + total > ids_capacity) return fail(CARE_ERR_CAPACITY, "ids_capacity exceeded");
+            if (ctx->packed.n < total) ctx->packed.alloc(total + total / 4);
+            launch_pack_candidates(ctx->candIds.p, ctx->candCount.p, nb, ctx->maxCand, ctx->packStarts.p, ctx->packed.p,
+                                   ctx->stream);
+            HIP_TRY(hipGetLastError());
+            HIP_TRY(hipMemcpyAsync(offsets + done + 1, ctx->packOffsets.p, sizeof(int) * nb, hipMemcpyDeviceToHost,
+                                   ctx->stream));
+            if (total)
+                HIP_TRY(hipMemcpyAsync(ids + written, ctx->packed.p, sizeof(u32) * total, hipMemcpyDeviceToHost,
+                                       ctx->stream));
+            HIP_TRY(hipStreamSynchronize(ctx->stream));
+            written += total;
         }
     } catch (const HipError& e) {
         return fail(CARE_ERR_DEVICE, "%s: %s", e.what, hipGetErrorString(e.err));
@@ -1280,9 +1292,8 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
                 HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             }
             try {
-                launch_fill_u64(reinterpret_cast<u64*>(ctx->rawHits.p), 2, 0, s);  // totals over the call
-                // candidate results over the call, heavy anchors of the first batches
-                launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, ctx->counters.p + 32, s);
+                // totals and candidate results over the call, heavy anchors of the first batches
+                launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, ctx->counters.p + 32, ctx->rawHits.p, s);
                 for (int done = 0, nb = 0; done < n; done += nb, bi++) {
                     nb = next_batch(B, n, n - done);
                     hipEvent_t* e = &ctx->batchEv[size_t(3 * bi)];
@@ -1292,11 +1303,10 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
                                  ctx->queryRegMax, o.exclude_ambiguous, o.candidate_limit, ctx->candIds.p,
                                  ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), ctx->rawCount.p, s,
                                  QueryAnchors(), QueryHeavy{ctx->heavy.p, heavyCount, P.heavyMin});
-                    launch_sum_counts(ctx->rawCount.p, ctx->candCount.p, nb, ctx->rawHits.p,
+                    launch_sum_counts(ctx->rawCount.p, ctx->candCount.p, nb, ctx->rawHits.p, ctx->counters.p,
                                       ctx->counters.p + 32 + ((bi + 1) & 1), s);
                     P.heavyCount = heavyCount;
                     if (!graph) HIP_TRY(hipEventRecord(e[1], s));
-                    launch_reset_counters(ctx->counters.p, nullptr, nullptr, s);  // work queue of this batch
                     P.firstAnchor = first + done;
                     P.numAnchors = nb;
                     P.outStatus = ctx->outStatus.p + size_t(done);
@@ -1918,7 +1928,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         }
         ctx->queryCap = bestCap;
         ctx->queryRegMax = bestReg;
-        launch_reset_counters(ctx->counters.p, nullptr, ctx->counters.p + 32, s);
+        launch_reset_counters(ctx->counters.p, nullptr, ctx->counters.p + 32, nullptr, s);
         launch_query(ctx->rs, ctx->tables, first, n, ctx->maxCand, bestCap, bestReg, o.exclude_ambiguous, candLimit,
                      ctx->candIds.p, ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), nullptr, s,
                      QueryAnchors(), QueryHeavy{ctx->heavy.p, ctx->counters.p + 32, heavy_min(ctx)});
@@ -1959,7 +1969,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
                 P.metaA = ctx->metaA.p;
                 P.metaB = ctx->metaB.p;
                 const float ms = timed([&] {
-                    launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, nullptr, s);
+                    launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, nullptr, nullptr, s);
                     launch_correct(P, blocks, T, chunk, s);
                 });
                 if (ms < bestC) {
@@ -2113,7 +2123,7 @@ extern "C" int care_correct_batch_noalloc(care_context* ctx, uint64_t first, int
                          o.exclude_ambiguous, o.candidate_limit, candIds, candCount, reinterpret_cast<u32*>(metaA),
                          nullptr, s);
             // queue head and candidate result count start at zero in every batch
-            launch_reset_counters(counters, counters + 1, nullptr, s);
+            launch_reset_counters(counters, counters + 1, nullptr, nullptr, s);
             P.firstAnchor = first + done;
             P.numAnchors = nb;
             P.outStatus = outStatus;

@@ -204,9 +204,17 @@ void launch_gather_lengths(const DevReadStore& rs, const u32* ids, int n, int* o
 void launch_gather_qualities(const DevReadStore& rs, const u32* ids, int n, char* out, int outPitch, hipStream_t s);
 void launch_gather_ambiguous(const DevReadStore& rs, const u32* ids, int n, u8* out, hipStream_t s);
 // totals[0] += sum(rawCount[0..n)), totals[1] += sum(candCount[0..n))
-// nextHeavy[0] = 0: the heavy-anchor count of the batch after
-void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, int* nextHeavy,
-                       hipStream_t s);
+// queue[0] = 0: the work queue of the correction that follows; nextHeavy[0] =
+// 0: the heavy-anchor count of the batch after
+void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, int* queue,
+                       int* nextHeavy, hipStream_t s);
+// candidate rows [n][maxCand] packed one behind the other into `packed`:
+// offsets[a] = base + candidates of anchors 0 .. a, truncated to 32 bits;
+// starts holds pack_scratch(n) words, starts[n] the number of candidates
+int pack_scratch(int n);
+void launch_pack_offsets(const int* candCount, int n, u64 base, int* offsets, u64* starts, hipStream_t s);
+void launch_pack_candidates(const u32* candIds, const int* candCount, int n, int maxCand, const u64* starts,
+                            u32* packed, hipStream_t s);
 // chunk: candidates staged per MSA pass (0 = automatic); gated: bit 0 the
 // anchor gate (correction type 3), bit 1 the candidate gate
 int correct_gate_mode(int correctionType, int correctCandidates, int correctionTypeCands);

@@ -749,13 +749,18 @@ __global__ void __launch_bounds__(256) k_query(DevReadStore rs, DevTables t, u64
     }
 }
 
-// totals[0] += sum of raw hit counts, totals[1] += sum of candidate counts
-// (one workgroup, so no atomics)
-__global__ void __launch_bounds__(1024) k_sum_counts(const int* rawCount, const int* candCount, int n,
-                                                     unsigned long long* totals, int* nextHeavy) {
-    __shared__ unsigned long long part[2][16];
+// totals[0] += sum of raw hit counts, totals[1] += sum of candidate counts;
+// the correction's work queue and the next batch's heavy-anchor count start
+// at 0.  One workgroup took 61 us for 200,000 anchors; several, with two
+// atomics a wavefront, take 5.
+__global__ void __launch_bounds__(256) k_sum_counts(const int* rawCount, const int* candCount, int n,
+                                                    unsigned long long* totals, int* queue, int* nextHeavy) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        queue[0] = 0;
+        nextHeavy[0] = 0;
+    }
     unsigned long long r = 0, c = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         r += u64(rawCount[i]);
         c += u64(candCount[i]);
     }
@@ -763,21 +768,72 @@ __global__ void __launch_bounds__(1024) k_sum_counts(const int* rawCount, const 
         r += __shfl_xor(r, o, kWave);
         c += __shfl_xor(c, o, kWave);
     }
-    const int w = threadIdx.x / kWave;
-    if (lane_id() == 0) {
-        part[0][w] = r;
-        part[1][w] = c;
+    if (lane_id() == 0 && r) {
+        atomicAdd(&totals[0], r);
+        atomicAdd(&totals[1], c);
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 1; k < int(blockDim.x / kWave); k++) {
-            r += part[0][k];
-            c += part[1][k];
+}
+
+// Packed candidate lists.  A tile of kPackTile anchors a block: the first
+// kernel sums the tiles; the second adds the tiles before its own (few: one
+// for every 1,024 anchors) and scans its counts into the caller's offsets
+// and, for the copy, 64-bit starts; the third copies a row a wavefront.
+constexpr int kPackTile = 1024;
+
+__global__ void __launch_bounds__(256) k_pack_sums(const int* candCount, int n, u64* tileSums) {
+    __shared__ u64 scr[8];
+    u64 v = 0, total;
+    for (int i = threadIdx.x; i < kPackTile; i += blockDim.x) {
+        const int a = blockIdx.x * kPackTile + i;
+        v += a < n ? u64(candCount[a]) : 0;
+    }
+    block_exclusive_sum(v, scr, &total);
+    if (threadIdx.x == 0) tileSums[blockIdx.x] = total;
+}
+
+__global__ void __launch_bounds__(256) k_pack_offsets(const int* candCount, int n, u64 base, const u64* tileSums,
+                                                      u64* starts, int* offsets) {
+    __shared__ u64 scr[8];
+    u64 before = 0, run;
+    for (int t = threadIdx.x; t < int(blockIdx.x); t += blockDim.x) before += tileSums[t];
+    block_exclusive_sum(before, scr, &run);
+    for (int i = 0; i < kPackTile; i += blockDim.x) {
+        const int a = blockIdx.x * kPackTile + i + threadIdx.x;
+        const u64 c = a < n ? u64(candCount[a]) : 0;
+        u64 sum;
+        const u64 ex = block_exclusive_sum(c, scr, &sum);
+        if (a < n) {
+            starts[a] = run + ex;
+            offsets[a] = int(base + run + ex + c);
+            if (a == n - 1) starts[n] = run + ex + c;
         }
-        totals[0] += r;
-        totals[1] += c;
-        nextHeavy[0] = 0;
+        run += sum;
     }
+}
+
+__global__ void __launch_bounds__(256) k_pack_candidates(const u32* candIds, const int* candCount, int n, int maxCand,
+                                                         const u64* starts, u32* packed) {
+    const int wpb = blockDim.x / kWave;
+    for (int a = blockIdx.x * wpb + threadIdx.x / kWave; a < n; a += gridDim.x * wpb) {
+        const u64 at = starts[a];
+        const int c = candCount[a];
+        for (int i = lane_id(); i < c; i += kWave) packed[at + i] = candIds[u64(a) * maxCand + i];
+    }
+}
+
+int pack_scratch(int n) { return n + 1 + (n + kPackTile - 1) / kPackTile; }
+
+void launch_pack_offsets(const int* candCount, int n, u64 base, int* offsets, u64* scratch, hipStream_t s) {
+    const int tiles = (n + kPackTile - 1) / kPackTile;
+    u64* tileSums = scratch + n + 1;
+    hipLaunchKernelGGL(k_pack_sums, dim3(tiles), dim3(256), 0, s, candCount, n, tileSums);
+    hipLaunchKernelGGL(k_pack_offsets, dim3(tiles), dim3(256), 0, s, candCount, n, base, tileSums, scratch, offsets);
+}
+
+void launch_pack_candidates(const u32* candIds, const int* candCount, int n, int maxCand, const u64* scratch,
+                            u32* packed, hipStream_t s) {
+    hipLaunchKernelGGL(k_pack_candidates, dim3(grid_for(u64(n) * kWave, 256)), dim3(256), 0, s, candIds, candCount, n,
+                       maxCand, scratch, packed);
 }
 
 int query_lds_bytes(int h, int cap, int maxLen, int threads, int candLimit, int capL) {
@@ -814,10 +870,11 @@ void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, 
                            excludeAmbiguous, candLimit, candIds, candCount, spill, rawCount, qa, heavy);
 }
 
-void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, int* nextHeavy,
-                       hipStream_t s) {
+void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, int* queue,
+                       int* nextHeavy, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_sum_counts, dim3(1), dim3(1024), 0, s, rawCount, candCount, n, totals, nextHeavy);
+    hipLaunchKernelGGL(k_sum_counts, dim3(std::min(64, (n + 255) / 256)), dim3(256), 0, s, rawCount, candCount, n,
+                       totals, queue, nextHeavy);
 }
 
 }  // namespace care_engine
