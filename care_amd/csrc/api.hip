@@ -19,17 +19,9 @@ namespace care_engine {
 // launchers of minhash.hip
 void launch_fill_u64(u64* p, u64 n, u64 v, hipStream_t s);
 void launch_fill_u32(u32* p, u64 n, u32 v, hipStream_t s);
-void launch_count_keys(const u64* sigs, u64 n, int h, int map, u64* tkeys, u32* tcount, u64 tmask, int* overflow,
-                       hipStream_t s);
-// value offsets of the keys with 2..cap values in slot order; tileSums holds
-// assign_offsets_scratch(tsize) words
-u64 assign_offsets_scratch(u64 tsize);
-void launch_assign_offsets(const u64* tkeys, const u32* tcount, u64 tsize, int cap, u32* toff, u64* tileSums,
-                           unsigned long long* counters, hipStream_t s);
-void launch_insert_final(const u64* tkeys, const u32* tcount, const u32* toff, u64 tsize, u64* fkeys, uint2* foffcnt,
-                         u64 fmask, int* overflow, hipStream_t s);
-void launch_scatter_values(const u64* sigs, u64 n, int h, int map, const u64* tkeys, const u32* toff, u64 tmask,
-                           u32* tfill, u32* values, hipStream_t s);
+u64 group_tiles(u64 tsize);
+void launch_group_count(const MapGroup& g, hipStream_t s);
+void launch_group_fill(const MapGroup& g, hipStream_t s);
 void launch_sort_buckets(const u32* toff, const u32* tcount, u64 tsize, u32* values, hipStream_t s);
 void launch_insert_triples(const u64* keys, const u32* offs, const u32* counts, u64 numKeys, u64* fkeys,
                            uint2* foffcnt, u64 fmask, int* overflow, hipStream_t s);
@@ -100,9 +92,12 @@ struct PinnedBuf {
 };
 
 struct MapStore {
-    DevBuf<u64> keys;
-    DevBuf<uint2> offcnt;
-    DevBuf<u32> values;
+    // keys, offcnt and values lie in `mem`, their own or that of the first
+    // map of the group they were built in
+    std::shared_ptr<DevBuf<unsigned char>> mem;
+    u64* keys = nullptr;
+    uint2* offcnt = nullptr;
+    u32* values = nullptr;
     u64 mask = 0;
     u64 numKeys = 0;
     u64 numValues = 0;
@@ -765,7 +760,6 @@ int care_minhash_build(care_context* ctx) {
     if (!ctx->hasReads) return fail(CARE_ERR_STATE, "no read store uploaded");
     const int h = ctx->opt.num_hash_maps;
     const u64 n = ctx->rs.n;
-    // one query workgroup holds up to h * cap hits twice in LDS
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
@@ -773,55 +767,81 @@ int care_minhash_build(care_context* ctx) {
         sigs.alloc(n * h);
         launch_signatures(ctx->rs, 0, int(n), ctx->opt.kmer_length, h, sigs.p, s);
         HIP_TRY(hipGetLastError());
-        // scratch table at load <= 0.5
-        u64 tsize = 1;
-        while (tsize < 2 * n) tsize <<= 1;
-        DevBuf<u64> tkeys;
-        DevBuf<u32> tcount, tfill, toff;
-        tkeys.alloc(tsize);
-        tcount.alloc(tsize);
-        tfill.alloc(tsize);
-        toff.alloc(tsize);
-        DevBuf<unsigned long long> counters;
-        counters.alloc(2);
-        DevBuf<u64> tileSums;
-        tileSums.alloc(assign_offsets_scratch(tsize));
-        DevBuf<int> overflow;
-        overflow.alloc(1);
+        MapGroup g{};
+        g.sigs = sigs.p;
+        g.n = n;
+        g.h = h;
+        g.cap = ctx->cap;
+        // scratch tables at load <= 0.5
+        g.tsize = 1;
+        while (g.tsize < 2 * n) g.tsize <<= 1;
+        // maps built together: as many as fit 256 MiB of scratch (its
+        // allocation takes about 5 ms a GiB), at least one
+        const u64 perMap = g.tsize * 16 + n * 12 + group_tiles(g.tsize) * 16;
+        const int G = int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), (u64(256) << 20) / perMap})));
+        DevBuf<u64> keys64;  // tkeys, tile sums, counters
+        DevBuf<u32> words;   // tcount, toff, slot, arrival, packed, overflow
+        keys64.alloc(size_t(G) * (g.tsize + 2 * group_tiles(g.tsize) + 2));
+        words.alloc(size_t(G) * (2 * g.tsize + 3 * n) + 1);
+        PinnedBuf<unsigned long long> totals;
+        totals.alloc(size_t(2) * G + 1);
+        g.tkeys = keys64.p;
+        g.tileSums = g.tkeys + size_t(G) * g.tsize;
+        g.counters = reinterpret_cast<unsigned long long*>(g.tileSums + size_t(G) * 2 * group_tiles(g.tsize));
+        g.tcount = words.p;
+        g.toff = g.tcount + size_t(G) * g.tsize;
+        g.slot = g.toff + size_t(G) * g.tsize;
+        g.arrival = g.slot + size_t(G) * n;
+        g.packed = g.arrival + size_t(G) * n;
+        g.overflow = reinterpret_cast<int*>(g.packed + size_t(G) * n);
+        ctx->hasTables = false;
         ctx->maps.clear();
         std::vector<DevMap> hostMaps(h);
-        for (int m = 0; m < h; m++) {
-            launch_fill_u64(tkeys.p, tsize, kEmptyKey, s);
-            launch_fill_u32(tcount.p, tsize, 0, s);
-            launch_fill_u32(tfill.p, tsize, 0, s);
-            launch_fill_u64(reinterpret_cast<u64*>(counters.p), 2, 0, s);
-            launch_fill_u32(reinterpret_cast<u32*>(overflow.p), 1, 0, s);
-            launch_count_keys(sigs.p, n, h, m, tkeys.p, tcount.p, tsize - 1, overflow.p, s);
-            launch_assign_offsets(tkeys.p, tcount.p, tsize, ctx->cap, toff.p, tileSums.p, counters.p, s);
+        for (int m0 = 0; m0 < h; m0 += G) {
+            g.first = m0;
+            g.count = std::min(G, h - m0);
+            launch_group_count(g, s);
             HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(ctx->hU64.p, counters.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+            HIP_TRY(hipMemcpyAsync(totals.p, g.counters, size_t(2 * g.count) * sizeof(unsigned long long),
+                                   hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
-            const u64 numValues = ctx->hU64.p[0];
-            const u64 numKeys = ctx->hU64.p[1];
-            auto ms = std::make_unique<MapStore>();
-            u64 fsize = 1;
-            while (fsize < 2 * numKeys + 2) fsize <<= 1;
-            ms->keys.alloc(fsize);
-            ms->offcnt.alloc(fsize);
-            ms->values.alloc(numValues);
-            ms->mask = fsize - 1;
-            ms->numKeys = numKeys;
-            ms->numValues = numValues;
-            launch_fill_u64(ms->keys.p, fsize, kEmptyKey, s);
-            launch_insert_final(tkeys.p, tcount.p, toff.p, tsize, ms->keys.p, ms->offcnt.p, ms->mask, overflow.p, s);
-            launch_scatter_values(sigs.p, n, h, m, tkeys.p, toff.p, tsize - 1, tfill.p, ms->values.p, s);
-            launch_sort_buckets(toff.p, tcount.p, tsize, ms->values.p, s);
+            // one allocation for the group's tables: all keys, all ranges,
+            // all values
+            u64 slots = 0, values = 0;
+            for (int i = 0; i < g.count; i++) {
+                auto ms = std::make_unique<MapStore>();
+                ms->numValues = totals.p[2 * i];
+                ms->numKeys = totals.p[2 * i + 1];
+                u64 fsize = 1;
+                while (fsize < 2 * ms->numKeys + 2) fsize <<= 1;
+                ms->mask = fsize - 1;
+                slots += fsize;
+                values += ms->numValues;
+                ctx->maps.push_back(std::move(ms));
+            }
+            auto mem = std::make_shared<DevBuf<unsigned char>>();
+            mem->alloc(size_t(slots) * (sizeof(u64) + sizeof(uint2)) + size_t(values) * sizeof(u32));
+            u64* keys = reinterpret_cast<u64*>(mem->p);
+            uint2* offcnt = reinterpret_cast<uint2*>(keys + slots);
+            u32* vals = reinterpret_cast<u32*>(offcnt + slots);
+            launch_fill_u64(keys, slots, kEmptyKey, s);
+            for (int i = 0; i < g.count; i++) {
+                MapStore& ms = *ctx->maps[size_t(m0 + i)];
+                ms.mem = mem;
+                ms.keys = keys;
+                ms.offcnt = offcnt;
+                ms.values = vals;
+                keys += ms.mask + 1;
+                offcnt += ms.mask + 1;
+                vals += ms.numValues;
+                hostMaps[size_t(m0 + i)] = g.fin[i] = DevMap{ms.keys, ms.offcnt, ms.values, ms.mask};
+            }
+            launch_group_fill(g, s);
             HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(ctx->hInts.p, overflow.p, sizeof(int), hipMemcpyDeviceToHost, s));
+            HIP_TRY(hipMemcpyAsync(totals.p + 2 * G, g.overflow, sizeof(int), hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
-            if (ctx->hInts.p[0]) return fail(CARE_ERR_DEVICE, "hash table overflow while building map %d", m);
-            hostMaps[m] = DevMap{ms->keys.p, ms->offcnt.p, ms->values.p, ms->mask};
-            ctx->maps.push_back(std::move(ms));
+            if (*reinterpret_cast<const int*>(totals.p + 2 * G))
+                return fail(CARE_ERR_DEVICE, "hash table overflow while building maps %d to %d", m0, m0 + g.count - 1);
         }
         ctx->devMaps.alloc(h);
         HIP_TRY(hipMemcpy(ctx->devMaps.p, hostMaps.data(), sizeof(DevMap) * h, hipMemcpyHostToDevice));
@@ -885,9 +905,11 @@ int care_minhash_import(care_context* ctx, const care_map_view* maps, int num_ma
             auto ms = std::make_unique<MapStore>();
             u64 fsize = 1;
             while (fsize < 2 * v.num_keys + 2) fsize <<= 1;
-            ms->keys.alloc(fsize);
-            ms->offcnt.alloc(fsize);
-            ms->values.alloc(v.num_values);
+            ms->mem = std::make_shared<DevBuf<unsigned char>>();
+            ms->mem->alloc(size_t(fsize) * (sizeof(u64) + sizeof(uint2)) + size_t(v.num_values) * sizeof(u32));
+            ms->keys = reinterpret_cast<u64*>(ms->mem->p);
+            ms->offcnt = reinterpret_cast<uint2*>(ms->keys + fsize);
+            ms->values = reinterpret_cast<u32*>(ms->offcnt + fsize);
             ms->mask = fsize - 1;
             ms->numKeys = v.num_keys;
             ms->numValues = v.num_values;
@@ -902,20 +924,20 @@ int care_minhash_import(care_context* ctx, const care_map_view* maps, int num_ma
                 HIP_TRY(hipMemcpy(dcounts.p, v.counts, sizeof(u32) * v.num_keys, hipMemcpyHostToDevice));
             }
             if (v.num_values)
-                HIP_TRY(hipMemcpy(ms->values.p, v.values, sizeof(u32) * v.num_values, hipMemcpyHostToDevice));
-            launch_fill_u64(ms->keys.p, fsize, kEmptyKey, s);
+                HIP_TRY(hipMemcpy(ms->values, v.values, sizeof(u32) * v.num_values, hipMemcpyHostToDevice));
+            launch_fill_u64(ms->keys, fsize, kEmptyKey, s);
             launch_fill_u32(reinterpret_cast<u32*>(overflow.p), 1, 0, s);
             if (v.num_keys) {
-                launch_insert_triples(dkeys.p, doffs.p, dcounts.p, v.num_keys, ms->keys.p, ms->offcnt.p, ms->mask,
+                launch_insert_triples(dkeys.p, doffs.p, dcounts.p, v.num_keys, ms->keys, ms->offcnt, ms->mask,
                                       overflow.p, s);
                 // the query merges each key's values as ascending lists
-                launch_sort_buckets(doffs.p, dcounts.p, v.num_keys, ms->values.p, s);
+                launch_sort_buckets(doffs.p, dcounts.p, v.num_keys, ms->values, s);
             }
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipMemcpyAsync(ctx->hInts.p, overflow.p, sizeof(int), hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
             if (ctx->hInts.p[0]) return fail(CARE_ERR_DEVICE, "hash table overflow while importing map %d", m);
-            hostMaps[m] = DevMap{ms->keys.p, ms->offcnt.p, ms->values.p, ms->mask};
+            hostMaps[m] = DevMap{ms->keys, ms->offcnt, ms->values, ms->mask};
             ctx->maps.push_back(std::move(ms));
         }
         ctx->devMaps.alloc(num_maps);
@@ -975,9 +997,9 @@ int care_minhash_export_map(care_context* ctx, int map, uint64_t* keys, uint32_t
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
-        HIP_TRY(hipMemcpy(slotKeys.data(), ms.keys.p, sizeof(u64) * fsize, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(slotOffcnt.data(), ms.offcnt.p, sizeof(uint2) * fsize, hipMemcpyDeviceToHost));
-        if (nv) HIP_TRY(hipMemcpy(slotValues.data(), ms.values.p, sizeof(u32) * nv, hipMemcpyDeviceToHost));
+        HIP_TRY(hipMemcpy(slotKeys.data(), ms.keys, sizeof(u64) * fsize, hipMemcpyDeviceToHost));
+        HIP_TRY(hipMemcpy(slotOffcnt.data(), ms.offcnt, sizeof(uint2) * fsize, hipMemcpyDeviceToHost));
+        if (nv) HIP_TRY(hipMemcpy(slotValues.data(), ms.values, sizeof(u32) * nv, hipMemcpyDeviceToHost));
     } catch (const HipError& e) {
         return fail(CARE_ERR_DEVICE, "%s: %s", e.what, hipGetErrorString(e.err));
     }

@@ -42,6 +42,27 @@ struct DevMap {
     u64 mask;
 };
 
+// A group of maps while they are built (minhash.hip): scratch arrays indexed
+// [map][slot] or, per read, [read][map]; `fin` holds the finished tables.
+constexpr int kMaxBuildMaps = 64;
+struct MapGroup {
+    const u64* sigs;  // [n][h]
+    u64 n;
+    int h, first, count;  // maps first .. first + count - 1
+    int cap;
+    u64 tsize;    // slots of a scratch table, a power of two
+    u64* tkeys;   // [count][tsize]
+    u32* tcount;  // [count][tsize]
+    u32* toff;    // [count][tsize]
+    u32* slot;    // [n][count] scratch slot of the read's key, ~0 if the table overflowed
+    u32* arrival; // [n][count] how many reads of the key came before
+    u32* packed;  // [n * count] value ranges, unsorted
+    u64* tileSums;
+    unsigned long long* counters;  // [count][2] values, keys
+    int* overflow;
+    DevMap fin[kMaxBuildMaps];
+};
+
 struct DevTables {
     const DevMap* maps = nullptr;
     int h = 0;

@@ -11,10 +11,13 @@
 //              ambiguous candidates under --excludeAmbiguous).
 //
 // The reference GPU path stores warpcore multi-value tables and compacts
-// them (include/gpu/gpuhashtable.cuh:314-760).  Here every map is built with
-// one counting pass into a scratch open-addressing table, an offset pass, a
-// scatter pass and a per-bucket sort, then re-inserted into a compact table
-// that only holds keys with 2..cap values.
+// them (include/gpu/gpuhashtable.cuh:314-760).  Here the maps are built a
+// group at a time, every kernel covering the group: a counting pass into
+// scratch open-addressing tables, an offset pass, an unordered scatter and a
+// pass that ranks every value within its key's range, and the keys with
+// 2..cap values re-inserted into compact tables.
+
+#include <algorithm>
 
 #include "device_common.h"
 
@@ -134,24 +137,41 @@ __device__ __forceinline__ u64 find_slot(const u64* keys, u64 mask, u64 key) {
     return ~u64(0);
 }
 
-// count occurrences of every key of map `map`
-__global__ void k_count_keys(const u64* sigs, u64 n, int h, int map, u64* tkeys, u32* tcount, u64 tmask,
-                             int* overflow) {
-    for (u64 r = blockIdx.x * u64(blockDim.x) + threadIdx.x; r < n; r += u64(gridDim.x) * blockDim.x) {
-        const u64 key = sigs[r * h + map];
-        const u64 slot = find_or_insert(tkeys, tmask, key);
+__global__ void k_group_clear(u64* tkeys, u32* tcount, u64 slots, unsigned long long* counters, int count,
+                              int* overflow) {
+    const u64 i0 = blockIdx.x * u64(blockDim.x) + threadIdx.x;
+    if (i0 < u64(2 * count)) counters[i0] = 0;
+    if (i0 == 0) overflow[0] = 0;
+    for (u64 i = i0; i < slots; i += u64(gridDim.x) * blockDim.x) {
+        tkeys[i] = kEmptyKey;
+        tcount[i] = 0;
+    }
+}
+
+// Counts the reads of every key, and keeps each read's slot and how many came
+// before it, so that the later passes neither probe nor count again.  A
+// thread is a (read, map) pair, maps of a read adjacent: signature rows are
+// read whole (a pass per map used 8 of every 64 bytes).
+__global__ void k_count_keys(MapGroup g) {
+    const u64 items = g.n * u64(g.count);
+    for (u64 i = blockIdx.x * u64(blockDim.x) + threadIdx.x; i < items; i += u64(gridDim.x) * blockDim.x) {
+        const u64 r = i / u32(g.count);
+        const int m = int(i - r * u32(g.count));
+        const u64 slot = find_or_insert(g.tkeys + u64(m) * g.tsize, g.tsize - 1, g.sigs[r * g.h + g.first + m]);
         if (slot == ~u64(0)) {
-            atomicExch(overflow, 1);
+            atomicExch(g.overflow, 1);
+            g.slot[i] = ~0u;
             continue;
         }
-        atomicAdd(&tcount[slot], 1u);
+        g.slot[i] = u32(slot);
+        g.arrival[i] = atomicAdd(&g.tcount[u64(m) * g.tsize + slot], 1u);
     }
 }
 
 // Value offsets of the keys with 2..cap values, in slot order: every block
-// sums a tile of kTile slots (values, keys), one block scans the tile sums,
-// then every block assigns the offsets of its tile.  Deterministic, and no
-// same-address atomics.  counters[0] = values, counters[1] = valid keys.
+// sums a tile of kTile slots (values, keys), one block a map scans the tile
+// sums, then every block assigns the offsets of its tile.  Deterministic, and
+// no same-address atomics.  counters[0] = values, counters[1] = valid keys.
 constexpr int kTile = 4096;
 
 __device__ __forceinline__ u32 slot_values(const u64* tkeys, const u32* tcount, u64 s, u64 tsize, int cap) {
@@ -184,9 +204,13 @@ __device__ __forceinline__ u64 block_exclusive_sum(u64 v, u64* scratch, u64* tot
     return before + incl - v;
 }
 
-__global__ void __launch_bounds__(256) k_tile_sums(const u64* tkeys, const u32* tcount, u64 tsize, int cap,
-                                                   u64* tileSums) {
+__global__ void __launch_bounds__(256) k_tile_sums(MapGroup g) {
     __shared__ u64 scr[8];
+    const u64* tkeys = g.tkeys + u64(blockIdx.y) * g.tsize;
+    const u32* tcount = g.tcount + u64(blockIdx.y) * g.tsize;
+    u64* tileSums = g.tileSums + 2 * u64(blockIdx.y) * gridDim.x;
+    const u64 tsize = g.tsize;
+    const int cap = g.cap;
     const u64 t0 = u64(blockIdx.x) * kTile;
     u64 vals = 0, keys = 0;
     for (int i = threadIdx.x; i < kTile; i += blockDim.x) {
@@ -203,9 +227,11 @@ __global__ void __launch_bounds__(256) k_tile_sums(const u64* tkeys, const u32* 
     }
 }
 
-// one block: tileSums[2t] becomes the first value offset of tile t
-__global__ void __launch_bounds__(1024) k_scan_tiles(u64* tileSums, u64 nt, unsigned long long* counters) {
+// one block a map: tileSums[2t] becomes the first value offset of tile t
+__global__ void __launch_bounds__(1024) k_scan_tiles(MapGroup g, u64 nt) {
     __shared__ u64 scr[17];
+    u64* tileSums = g.tileSums + 2 * u64(blockIdx.x) * nt;
+    unsigned long long* counters = g.counters + 2 * blockIdx.x;
     u64 carryV = 0, carryK = 0;
     for (u64 b = 0; b < nt; b += blockDim.x) {
         const u64 t = b + threadIdx.x;
@@ -224,9 +250,14 @@ __global__ void __launch_bounds__(1024) k_scan_tiles(u64* tileSums, u64 nt, unsi
     }
 }
 
-__global__ void __launch_bounds__(256) k_tile_offsets(const u64* tkeys, const u32* tcount, u64 tsize, int cap,
-                                                      const u64* tileSums, u32* toff) {
+__global__ void __launch_bounds__(256) k_tile_offsets(MapGroup g) {
     __shared__ u64 scr[8];
+    const u64* tkeys = g.tkeys + u64(blockIdx.y) * g.tsize;
+    const u32* tcount = g.tcount + u64(blockIdx.y) * g.tsize;
+    u32* toff = g.toff + u64(blockIdx.y) * g.tsize;
+    const u64* tileSums = g.tileSums + 2 * u64(blockIdx.y) * gridDim.x;
+    const u64 tsize = g.tsize;
+    const int cap = g.cap;
     const u64 t0 = u64(blockIdx.x) * kTile;
     u64 run = tileSums[2 * u64(blockIdx.x)];
     for (int r = 0; r < kTile; r += blockDim.x) {
@@ -239,32 +270,58 @@ __global__ void __launch_bounds__(256) k_tile_offsets(const u64* tkeys, const u3
     }
 }
 
-// insert valid keys into the compact table
-__global__ void k_insert_final(const u64* tkeys, const u32* tcount, const u32* toff, u64 tsize, u64* fkeys,
-                               uint2* foffcnt, u64 fmask, int* overflow) {
-    for (u64 s = blockIdx.x * u64(blockDim.x) + threadIdx.x; s < tsize; s += u64(gridDim.x) * blockDim.x) {
+// insert valid keys into the compact tables
+__global__ void k_insert_final(MapGroup g) {
+    const int m = blockIdx.y;
+    const u64* tkeys = g.tkeys + u64(m) * g.tsize;
+    const u32* tcount = g.tcount + u64(m) * g.tsize;
+    const u32* toff = g.toff + u64(m) * g.tsize;
+    u64* fkeys = const_cast<u64*>(g.fin[m].keys);
+    uint2* foffcnt = const_cast<uint2*>(g.fin[m].offcnt);
+    for (u64 s = blockIdx.x * u64(blockDim.x) + threadIdx.x; s < g.tsize; s += u64(gridDim.x) * blockDim.x) {
         if (toff[s] == 0xFFFFFFFFu) continue;
-        const u64 key = tkeys[s];
-        const u64 slot = find_or_insert(fkeys, fmask, key);
+        const u64 slot = find_or_insert(fkeys, g.fin[m].mask, tkeys[s]);
         if (slot == ~u64(0)) {
-            atomicExch(overflow, 1);
+            atomicExch(g.overflow, 1);
             continue;
         }
         foffcnt[slot] = make_uint2(toff[s], tcount[s]);
     }
 }
 
-// scatter read ids into their key's value range
-__global__ void k_scatter_values(const u64* sigs, u64 n, int h, int map, const u64* tkeys, const u32* toff, u64 tmask,
-                                 u32* tfill, u32* values) {
-    for (u64 r = blockIdx.x * u64(blockDim.x) + threadIdx.x; r < n; r += u64(gridDim.x) * blockDim.x) {
-        const u64 key = sigs[r * h + map];
-        const u64 slot = find_slot(tkeys, tmask, key);
-        if (slot == ~u64(0)) continue;
-        const u32 off = toff[slot];
+// read ids into their key's value range of the scratch array, in the order in
+// which the counting pass met them
+__global__ void k_scatter_values(MapGroup g) {
+    const u64 items = g.n * u64(g.count);
+    for (u64 i = blockIdx.x * u64(blockDim.x) + threadIdx.x; i < items; i += u64(gridDim.x) * blockDim.x) {
+        const u64 r = i / u32(g.count);
+        const int m = int(i - r * u32(g.count));
+        const u32 slot = g.slot[i];
+        if (slot == ~0u) continue;
+        const u32 off = g.toff[u64(m) * g.tsize + slot];
         if (off == 0xFFFFFFFFu) continue;
-        const u32 pos = atomicAdd(&tfill[slot], 1u);
-        values[u64(off) + pos] = u32(r);
+        g.packed[u64(m) * g.n + off + g.arrival[i]] = u32(r);
+    }
+}
+
+// Ascending read ids within every range: a thread per value counts the smaller
+// ones of its range (at most cap values, a few cache lines shared by its
+// neighbours).  A thread per range sorting it by insertion in memory took
+// 200 us a map at 300,000 reads, two thirds of the build.
+__global__ void k_rank_values(MapGroup g) {
+    const u64 items = g.n * u64(g.count);
+    for (u64 i = blockIdx.x * u64(blockDim.x) + threadIdx.x; i < items; i += u64(gridDim.x) * blockDim.x) {
+        const u64 r = i / u32(g.count);
+        const int m = int(i - r * u32(g.count));
+        const u32 slot = g.slot[i];
+        if (slot == ~0u) continue;
+        const u32 off = g.toff[u64(m) * g.tsize + slot];
+        if (off == 0xFFFFFFFFu) continue;
+        const int c = int(g.tcount[u64(m) * g.tsize + slot]);
+        const u32* v = g.packed + u64(m) * g.n + off;
+        int rank = 0;
+        for (int k = 0; k < c; k++) rank += v[k] < u32(r);
+        const_cast<u32*>(g.fin[m].values)[u64(off) + rank] = u32(r);
     }
 }
 
@@ -311,30 +368,28 @@ void launch_fill_u64(u64* p, u64 n, u64 v, hipStream_t s) {
 void launch_fill_u32(u32* p, u64 n, u32 v, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, 256)), dim3(256), 0, s, p, n, v);
 }
-void launch_count_keys(const u64* sigs, u64 n, int h, int map, u64* tkeys, u32* tcount, u64 tmask, int* overflow,
-                       hipStream_t s) {
-    hipLaunchKernelGGL(k_count_keys, dim3(grid_for(n, 256)), dim3(256), 0, s, sigs, n, h, map, tkeys, tcount, tmask,
-                       overflow);
-}
-u64 assign_offsets_scratch(u64 tsize) { return 2 * ((tsize + kTile - 1) / kTile); }
+u64 group_tiles(u64 tsize) { return (tsize + kTile - 1) / kTile; }
 
-void launch_assign_offsets(const u64* tkeys, const u32* tcount, u64 tsize, int cap, u32* toff, u64* tileSums,
-                           unsigned long long* counters, hipStream_t s) {
-    const u64 nt = (tsize + kTile - 1) / kTile;
-    hipLaunchKernelGGL(k_tile_sums, dim3(unsigned(nt)), dim3(256), 0, s, tkeys, tcount, tsize, cap, tileSums);
-    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, tileSums, nt, counters);
-    hipLaunchKernelGGL(k_tile_offsets, dim3(unsigned(nt)), dim3(256), 0, s, tkeys, tcount, tsize, cap, tileSums, toff);
+// keys counted and value ranges assigned: counters hold every map's values
+// and keys once the stream is done
+void launch_group_count(const MapGroup& g, hipStream_t s) {
+    const u64 slots = u64(g.count) * g.tsize;
+    const unsigned nt = unsigned(group_tiles(g.tsize));
+    hipLaunchKernelGGL(k_group_clear, dim3(grid_for(slots, 256)), dim3(256), 0, s, g.tkeys, g.tcount, slots,
+                       g.counters, g.count, g.overflow);
+    hipLaunchKernelGGL(k_count_keys, dim3(grid_for(g.n * u64(g.count), 256)), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_tile_sums, dim3(nt, g.count), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_scan_tiles, dim3(g.count), dim3(1024), 0, s, g, u64(nt));
+    hipLaunchKernelGGL(k_tile_offsets, dim3(nt, g.count), dim3(256), 0, s, g);
 }
-void launch_insert_final(const u64* tkeys, const u32* tcount, const u32* toff, u64 tsize, u64* fkeys, uint2* foffcnt,
-                         u64 fmask, int* overflow, hipStream_t s) {
-    hipLaunchKernelGGL(k_insert_final, dim3(grid_for(tsize, 256)), dim3(256), 0, s, tkeys, tcount, toff, tsize, fkeys,
-                       foffcnt, fmask, overflow);
+
+// the tables of g.fin (keys cleared before)
+void launch_group_fill(const MapGroup& g, hipStream_t s) {
+    hipLaunchKernelGGL(k_insert_final, dim3(std::min(grid_for(g.tsize, 256), 4096), g.count), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_scatter_values, dim3(grid_for(g.n * u64(g.count), 256)), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_rank_values, dim3(grid_for(g.n * u64(g.count), 256)), dim3(256), 0, s, g);
 }
-void launch_scatter_values(const u64* sigs, u64 n, int h, int map, const u64* tkeys, const u32* toff, u64 tmask,
-                           u32* tfill, u32* values, hipStream_t s) {
-    hipLaunchKernelGGL(k_scatter_values, dim3(grid_for(n, 256)), dim3(256), 0, s, sigs, n, h, map, tkeys, toff, tmask,
-                       tfill, values);
-}
+
 void launch_sort_buckets(const u32* toff, const u32* tcount, u64 tsize, u32* values, hipStream_t s) {
     hipLaunchKernelGGL(k_sort_buckets, dim3(grid_for(tsize, 256)), dim3(256), 0, s, toff, tcount, tsize, values);
 }

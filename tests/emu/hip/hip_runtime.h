@@ -365,7 +365,7 @@ void launch_run(const char* name, K kernel, dim3 grid, dim3 block, size_t ldsByt
     s.arg = &call;
     sched() = &s;
     s.fibers.resize(nthreads);
-    for (unsigned b = 0; b < grid.x; b++) {
+    for (unsigned b = 0; b < grid.x * grid.y; b++) {
         if (poison_byte() >= 0) std::memset(lds().data(), poison_byte(), lds().size());
         for (auto& f : s.fibers) {
             f.done = false;
@@ -379,7 +379,7 @@ void launch_run(const char* name, K kernel, dim3 grid, dim3 block, size_t ldsByt
         s.blockArrived = 0;
         for (unsigned t = 0; t < nthreads; t++) {
             s.fibers[t].c.tid = dim3(t);
-            s.fibers[t].c.bid = dim3(b);
+            s.fibers[t].c.bid = dim3(b % grid.x, b / grid.x);
             s.fibers[t].c.bdim = block;
             s.fibers[t].c.gdim = grid;
         }
