@@ -156,7 +156,8 @@ struct care_context {
     DevBuf<u64> packStarts;
     DevBuf<int> packOffsets;
     DevBuf<u32> packed;
-    DevBuf<CandMeta> metaA, metaB;  // a row of maxCand records per correction workgroup
+    DevBuf<u32> spill;  // query_spill_words(maxCand) words per query wavefront
+    DevBuf<CandMeta> metaA, metaB;  // a row of records per correction workgroup
     DevBuf<u8> outStatus;
     DevBuf<char> outSeq;
     int outPitch = 0;
@@ -220,26 +221,34 @@ struct care_context {
 
 namespace {
 
-// Record rows of the correction workgroups, and spill rows of the query's
-// wavefronts, which are as long as a row of records.
-void ensure_rows(care_context* ctx, int spillRows, int blocks) {
-    const size_t mc = size_t(ctx->maxCand);
-    const size_t a = size_t(std::max(spillRows, blocks)) * mc, b = size_t(blocks) * mc;
-    if (ctx->metaA.n < a) ctx->metaA.alloc(a);
-    if (ctx->metaB.n < b) ctx->metaB.alloc(b);
+template <class T>
+void at_least(DevBuf<T>& buf, size_t n) {
+    if (buf.n < n) buf.alloc(n);
+}
+
+// Candidate ids of an anchor that reach the correction: h x cap at most, or
+// the limit.
+int row_candidates(const care_context* ctx) {
+    const int limit = ctx->opt.candidate_limit;
+    return limit > 0 ? std::min(limit, ctx->maxCand) : ctx->maxCand;
+}
+
+// Record rows of the correction workgroups.
+void ensure_rows(care_context* ctx, int blocks) {
+    at_least(ctx->metaA, size_t(blocks) * size_t(row_candidates(ctx)));
+    at_least(ctx->metaB, size_t(blocks) * size_t(row_candidates(ctx)));
 }
 
 // Batch buffers of a call over n anchors in device batches of up to B: small
-// calls take what they need, rounded up to a power of two, so a program of a
-// few thousand reads does not allocate for 262,144 anchors.
+// calls take what they need, rounded up to a power of two.  Memory costs a
+// program about 25 ms a GiB (allocated, freed and cleared by the driver).
 void ensure_batch(care_context* ctx, int B, int n) {
     int batch = 1024;
     while (batch < n && batch < B) batch *= 2;
     batch = std::min(batch, B);
-    ensure_rows(ctx, query_spill_rows(batch), 0);
+    at_least(ctx->spill, size_t(query_spill_rows(batch)) * query_spill_words(ctx->maxCand));
+    at_least(ctx->candIds, size_t(batch) * size_t(row_candidates(ctx)));
     if (batch <= ctx->batchCap) return;
-    const size_t mc = size_t(ctx->maxCand);
-    ctx->candIds.alloc(size_t(batch) * mc);
     ctx->candCount.alloc(batch);
     ctx->rawCount.alloc(batch);
     ctx->heavy.alloc(batch);
@@ -257,17 +266,19 @@ void ensure_batch(care_context* ctx, int B, int n) {
     ctx->batchCap = batch;
 }
 
-// Anchors per device batch: the candidate lists (h x cap slots per anchor)
-// get a quarter of the device memory free when the context was created,
-// between 2 and 4 GiB, and a batch holds at most 2^18 anchors.  Fewer, larger
-// batches mean fewer launches and fewer drains of the persistent correction
-// kernel.
-int default_batch(care_context* ctx) {
+// Anchors per device batch of a call over n (0: any): the candidate lists get
+// a quarter of the device memory free when the context was created, between 2
+// and 4 GiB, and a batch holds at most 2^18 anchors.  Fewer, larger batches
+// mean fewer launches and fewer drains of the persistent correction kernel,
+// so a call is cut into eight at the least; beyond that larger batches only
+// take memory.
+int default_batch(care_context* ctx, int n) {
     if (ctx->requestedBatch > 0) return ctx->requestedBatch;
-    const size_t perAnchor = size_t(ctx->maxCand) * sizeof(u32) + ctx->rs.maxLen + 64;
+    const size_t perAnchor = size_t(row_candidates(ctx)) * sizeof(u32) + ctx->rs.maxLen + 64;
     const size_t budget = std::min(std::max(ctx->freeAtCreate / 4, size_t(2) << 30), size_t(4) << 30);
     size_t b = budget / perAnchor;
     b = std::max<size_t>(256, std::min<size_t>(b, size_t(1) << 18));
+    if (n > 0) b = std::min<size_t>(b, std::max(32768, n / 8));
     return int(b & ~size_t(1));
 }
 
@@ -449,7 +460,7 @@ int care_get_tuning(care_context* ctx, care_tuning* out) {
     const auto& o = ctx->opt;
     const int T = correct_threads(ctx, 1 << 20);  // of a call that fills the device
     const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
-    out->batch_anchors = ctx->rs.n ? default_batch(ctx) : ctx->requestedBatch;
+    out->batch_anchors = ctx->rs.n ? default_batch(ctx, 0) : ctx->requestedBatch;
     out->correct_threads = T;
     out->msa_chunk = correct_msa_chunk(ctx->rs.maxLen ? ctx->rs.maxLen : 1, o.use_quality, ctx->rs.qpitch, T, gatedK,
                                        ctx->msaChunk);
@@ -727,7 +738,7 @@ int care_minhash_query_async(care_context* ctx, const uint32_t* d_seqs, int seq_
         qa.ids = d_read_ids;
         qa.lens = d_lengths;
         launch_query(ctx->rs, ctx->tables, 0, n, ctx->maxCand, ctx->queryCap, ctx->queryRegMax, o.exclude_ambiguous,
-                     o.candidate_limit, d_candidates, d_counts, spill, nullptr, stream, qa);
+                     o.candidate_limit, d_candidates, ctx->maxCand, d_counts, spill, nullptr, stream, qa);
         HIP_TRY(hipGetLastError());
     } catch (const HipError& e) {
         return fail(CARE_ERR_DEVICE, "%s: %s", e.what, hipGetErrorString(e.err));
@@ -775,10 +786,10 @@ int care_minhash_build(care_context* ctx) {
         // scratch tables at load <= 0.5
         g.tsize = 1;
         while (g.tsize < 2 * n) g.tsize <<= 1;
-        // maps built together: as many as fit 256 MiB of scratch (its
-        // allocation takes about 5 ms a GiB), at least one
+        // maps built together: as many as fit 128 MiB of scratch (memory
+        // costs about 25 ms a GiB, a group two waits for the device)
         const u64 perMap = g.tsize * 16 + n * 12 + group_tiles(g.tsize) * 16;
-        const int G = int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), (u64(256) << 20) / perMap})));
+        const int G = int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), (u64(128) << 20) / perMap})));
         DevBuf<u64> keys64;  // tkeys, tile sums, counters
         DevBuf<u32> words;   // tcount, toff, slot, arrival, packed, overflow
         keys64.alloc(size_t(G) * (g.tsize + 2 * group_tiles(g.tsize) + 2));
@@ -1033,15 +1044,15 @@ int care_minhash_query(care_context* ctx, uint64_t first, int n, uint32_t* ids, 
     offsets[0] = 0;
     try {
         HIP_TRY(hipSetDevice(ctx->device));
-        const int B = default_batch(ctx);
+        const int B = default_batch(ctx, n);
         ensure_batch(ctx, B, n);
+        const int pitch = row_candidates(ctx);
         uint64_t written = 0;
         for (int done = 0; done < n; done += B) {
             const int nb = std::min(B, n - done);
             launch_query(ctx->rs, ctx->tables, first + done, nb, ctx->maxCand, ctx->queryCap, ctx->queryRegMax,
                          ctx->opt.exclude_ambiguous, ctx->opt.candidate_limit,
-                         ctx->candIds.p, ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), nullptr,
-                         ctx->stream);
+                         ctx->candIds.p, pitch, ctx->candCount.p, ctx->spill.p, nullptr, ctx->stream);
             HIP_TRY(hipGetLastError());
             // the lists are packed on the device, so that only their entries
             // are copied, straight into the caller's arrays (the rows of
@@ -1055,7 +1066,7 @@ int care_minhash_query(care_context* ctx, uint64_t first, int n, uint32_t* ids, 
             const u64 total = ctx->hU64.p[0];
             if (written + total > ids_capacity) return fail(CARE_ERR_CAPACITY, "ids_capacity exceeded");
             if (ctx->packed.n < total) ctx->packed.alloc(total + total / 4);
-            launch_pack_candidates(ctx->candIds.p, ctx->candCount.p, nb, ctx->maxCand, ctx->packStarts.p, ctx->packed.p,
+            launch_pack_candidates(ctx->candIds.p, ctx->candCount.p, nb, pitch, ctx->packStarts.p, ctx->packed.p,
                                    ctx->stream);
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipMemcpyAsync(offsets + done + 1, ctx->packOffsets.p, sizeof(int) * nb, hipMemcpyDeviceToHost,
@@ -1227,7 +1238,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
     if (const int rc = prepare_params(ctx, P)) return rc;
     try {
         HIP_TRY(hipSetDevice(ctx->device));
-        const int B = default_batch(ctx);
+        const int B = default_batch(ctx, n);
         ensure_batch(ctx, B, n);
         const int T = correct_threads(ctx, std::min(n, B));
         const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
@@ -1241,7 +1252,8 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         const int blocksPerCU = ctx->blocksPerCU > 0 ? ctx->blocksPerCU
                                                      : correct_resident_blocks(T, lds, gatedK | (P.gatedRefine ? 4 : 0));
         hipStream_t s = ctx->stream;
-        ensure_rows(ctx, 0, std::min(std::min(n, B), ctx->numCUs * blocksPerCU));
+        ensure_rows(ctx, std::min(std::min(n, B), ctx->numCUs * blocksPerCU));
+        P.maxCand = row_candidates(ctx);
         P.candIds = ctx->candIds.p;
         P.candCount = ctx->candCount.p;
         P.metaA = ctx->metaA.p;
@@ -1299,7 +1311,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
                                                "anchor_sequences (care_host_buffer_alloc)");
             key_append(key, first, n, r->anchor_status, r->anchor_sequences, r->sequence_pitch, candCap, B, T,
                        blocksPerCU, ctx->msaChunk, ctx->queryCap, ctx->queryRegMax, ctx->numCUs, ctx->outPitch, o,
-                       P, ctx->tables, ctx->rs, ctx->candIds.p, ctx->candCount.p, ctx->metaA.p, ctx->rawCount.p,
+                       P, ctx->tables, ctx->rs, ctx->candIds.p, ctx->candCount.p, ctx->metaA.p, ctx->spill.p, ctx->rawCount.p,
                        ctx->rawHits.p, ctx->counters.p, ctx->outStatus.p, ctx->outSeq.p);
         }
         const bool replay = graph && gc.exec && gc.key == key;
@@ -1323,7 +1335,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
                     int* heavyCount = ctx->counters.p + 32 + (bi & 1);
                     launch_query(ctx->rs, ctx->tables, first + done, nb, ctx->maxCand, ctx->queryCap,
                                  ctx->queryRegMax, o.exclude_ambiguous, o.candidate_limit, ctx->candIds.p,
-                                 ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), ctx->rawCount.p, s,
+                                 P.maxCand, ctx->candCount.p, ctx->spill.p, ctx->rawCount.p, s,
                                  QueryAnchors(), QueryHeavy{ctx->heavy.p, heavyCount, P.heavyMin});
                     launch_sum_counts(ctx->rawCount.p, ctx->candCount.p, nb, ctx->rawHits.p, ctx->counters.p,
                                       ctx->counters.p + 32 + ((bi + 1) & 1), s);
@@ -1904,7 +1916,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
     P.gateCap = 0;
     try {
         HIP_TRY(hipSetDevice(ctx->device));
-        const int B = default_batch(ctx);
+        const int B = default_batch(ctx, n);
         n = std::min(n, std::min(B, 65536)) & ~1;
         if (n == 0) n = 2 > int(ctx->rs.n - first) ? 1 : 2;
         ensure_batch(ctx, B, n);
@@ -1926,7 +1938,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         };
         auto query = [&](int capL, int regMax) {
             launch_query(ctx->rs, ctx->tables, first, n, ctx->maxCand, capL, regMax, o.exclude_ambiguous, candLimit,
-                         ctx->candIds.p, ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), nullptr, s);
+                         ctx->candIds.p, row_candidates(ctx), ctx->candCount.p, ctx->spill.p, nullptr, s);
         };
         // query: LDS hit capacities up to the longest possible list and, for
         // tables whose lists can exceed 1024 hits (unless pinned by
@@ -1952,12 +1964,13 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         ctx->queryRegMax = bestReg;
         launch_reset_counters(ctx->counters.p, nullptr, ctx->counters.p + 32, nullptr, s);
         launch_query(ctx->rs, ctx->tables, first, n, ctx->maxCand, bestCap, bestReg, o.exclude_ambiguous, candLimit,
-                     ctx->candIds.p, ctx->candCount.p, reinterpret_cast<u32*>(ctx->metaA.p), nullptr, s,
+                     ctx->candIds.p, row_candidates(ctx), ctx->candCount.p, ctx->spill.p, nullptr, s,
                      QueryAnchors(), QueryHeavy{ctx->heavy.p, ctx->counters.p + 32, heavy_min(ctx)});
         HIP_TRY(hipGetLastError());
         P.heavyList = ctx->heavy.p;
         P.heavyCount = ctx->counters.p + 32;
         P.heavyMin = heavy_min(ctx);
+        P.maxCand = row_candidates(ctx);
         // correction: 2, 3 or 4 wavefronts per anchor, automatic and halved MSA chunks
         P.candIds = ctx->candIds.p;
         P.candCount = ctx->candCount.p;
@@ -1987,7 +2000,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
                                                      o.correct_candidates, o.new_columns_to_correct);
                 const int bpc = ctx->blocksPerCU > 0 ? ctx->blocksPerCU : correct_resident_blocks(T, lds, gatedK);
                 const int blocks = std::max(1, std::min(n, ctx->numCUs * bpc));
-                ensure_rows(ctx, 0, blocks);
+                ensure_rows(ctx, blocks);
                 P.metaA = ctx->metaA.p;
                 P.metaB = ctx->metaB.p;
                 const float ms = timed([&] {
@@ -2142,7 +2155,8 @@ extern "C" int care_correct_batch_noalloc(care_context* ctx, uint64_t first, int
         for (int done = 0; done < n; done += B) {
             const int nb = std::min(B, n - done);
             launch_query(ctx->rs, ctx->tables, first + done, nb, ctx->maxCand, ctx->queryCap, ctx->queryRegMax,
-                         o.exclude_ambiguous, o.candidate_limit, candIds, candCount, reinterpret_cast<u32*>(metaA),
+                         o.exclude_ambiguous, o.candidate_limit, candIds, int(mc), candCount,
+                         reinterpret_cast<u32*>(metaA),
                          nullptr, s);
             // queue head and candidate result count start at zero in every batch
             launch_reset_counters(counters, counters + 1, nullptr, nullptr, s);

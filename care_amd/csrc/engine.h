@@ -204,6 +204,9 @@ struct QueryAnchors {
     const int* lens = nullptr;
 };
 int query_spill_rows(int n);
+__host__ __device__ inline size_t query_spill_words(int maxCand) {
+    return 2 * size_t(maxCand) + (size_t(maxCand) + 15) / 16 * 4;  // two buffers of ids, one of hit bytes
+}
 // Where a query lists the anchors that keep more than `min` candidates
 // (list null: nowhere); count starts at 0.
 struct QueryHeavy {
@@ -211,13 +214,15 @@ struct QueryHeavy {
     int* count = nullptr;
     int min = 0;
 };
-// spill: 4 * maxCand words for each of query_spill_rows(n) wavefronts
-// (sort/merge buffers of anchors with more than capL hits); regMax: longest hit list sorted in
+// candIds: a row of `pitch` ids per anchor, pitch at least maxCand or, with
+// candLimit > 0, candLimit; spill: query_spill_words(maxCand) words for each
+// of query_spill_rows(n) wavefronts (sort/merge buffers of anchors with more
+// than capL hits); regMax: longest hit list sorted in
 // registers (0 = the kernel's maximum, 1024), longer lists are merged;
 // rawCount (may be null): table hits per anchor before de-duplication
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
-                  int excludeAmbiguous, int candLimit, u32* candIds, int* candCount, u32* spill, int* rawCount,
-                  hipStream_t stream, const QueryAnchors& anchors = QueryAnchors(),
+                  int excludeAmbiguous, int candLimit, u32* candIds, int pitch, int* candCount, u32* spill,
+                  int* rawCount, hipStream_t stream, const QueryAnchors& anchors = QueryAnchors(),
                   const QueryHeavy& heavy = QueryHeavy());
 // read-store gathers by read id into device buffers (store.hip)
 void launch_gather_sequences(const DevReadStore& rs, const u32* ids, int n, u32* out, int outPitch, hipStream_t s);

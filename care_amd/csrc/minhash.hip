@@ -657,10 +657,10 @@ __device__ __forceinline__ int compact_unique(Buf sorted, int total, u32 self, c
     return written;
 }
 
-// keeps the candLimit candidates with the most hits (ties: smaller id, i.e.
-// earlier in out), in place and in order; hist holds h + 1 ints
+// the candLimit candidates with the most hits (ties: smaller id, i.e.
+// earlier in ids), in order, to out; hist holds h + 1 ints
 template <class HitBuf>
-__device__ __forceinline__ int keep_top(u32* out, HitBuf hits, int written, int candLimit, int h, int* hist,
+__device__ __forceinline__ int keep_top(const u32* ids, u32* out, HitBuf hits, int written, int candLimit, int h, int* hist,
                                         int lane) {
     for (int b = lane; b <= h; b += kWave) hist[b] = 0;
     wave_sync_mem();
@@ -692,18 +692,27 @@ __device__ __forceinline__ int keep_top(u32* out, HitBuf hits, int written, int 
         u32 v = 0;
         int hc = 0;
         if (i < written) {
-            v = out[i];
+            v = ids[i];
             hc = hits[i];
         }
         const u64 bT = __ballot(i < written && hc == T);
         const int rT = __popcll(bT & below);
         const bool keep = i < written && (hc > T || (hc == T && atT + rT < need));
         const u64 bk = __ballot(keep);
-        if (keep) out[kept + __popcll(bk & below)] = v;  // kept + rank <= i: reads of later entries unaffected
+        if (keep) out[kept + __popcll(bk & below)] = v;
         kept += __popcll(bk);
         atT += __popcll(bT);
     }
     return kept;
+}
+
+// the distinct ids to the anchor's row: all, or the candLimit with the most hits
+template <class HitBuf>
+__device__ __forceinline__ int pick(const u32* ids, u32* out, HitBuf hits, int n, int candLimit, int h, int* hist,
+                                    int lane) {
+    if (n > candLimit) return keep_top(ids, out, hits, n, candLimit, h, hist, lane);
+    for (int i = lane; i < n; i += kWave) out[i] = ids[i];
+    return n;
 }
 
 }  // namespace
@@ -711,7 +720,7 @@ __device__ __forceinline__ int keep_top(u32* out, HitBuf hits, int written, int 
 template <int kMaxK>
 __global__ void __launch_bounds__(256) k_query(DevReadStore rs, DevTables t, u64 first, int n, int maxCand, int capL,
                                                int regMax, int excludeAmbiguous, int candLimit, u32* candIds,
-                                               int* candCount, u32* spill, int* rawCount, QueryAnchors qa,
+                                               int pitch, int* candCount, u32* spill, int* rawCount, QueryAnchors qa,
                                                QueryHeavy heavy) {
     HIP_DYNAMIC_SHARED(uint4, ldsRaw)
     const int wave = threadIdx.x / kWave;
@@ -774,26 +783,30 @@ __global__ void __launch_bounds__(256) k_query(DevReadStore rs, DevTables t, u64
         if (lane == 0) counts[h] = total;
         wave_sync_mem();
 
-        u32* out = candIds + u64(a) * maxCand;
-        // this wavefront's row: [maxCand] + [maxCand] + hit bytes
-        u32* gs = spill + (u64(blockIdx.x) * wpb + wave) * 4 * maxCand;
-        u8* gh = reinterpret_cast<u8*>(gs + 2 * maxCand);
+        u32* out = candIds + u64(a) * pitch;
+        // this wavefront's row: two buffers of maxCand ids, hit bytes
+        u32* gs = spill + (u64(blockIdx.x) * wpb + wave) * query_spill_words(maxCand);
         int written;
+        // with a limit, the candidates are picked among the distinct ids in
+        // the buffer that the sort left free; only those go to the row, which
+        // then holds candLimit ids instead of h x cap
         if (total <= capL) {
-            const u32* sorted = la;
+            u32* sorted = la;
             if (total <= regMax) gather_sort_any<kMaxK>(la, counts, lists, h, total, lane);
             else sorted = gather_merge(la, lb, counts, lists, h, total, lane);
-            written = compact_unique(sorted, total, u32(id), rs, excludeAmbiguous, candLimit, out, lh, lane);
+            u32* distinct = candLimit > 0 ? (sorted == la ? lb : la) : out;
+            written = compact_unique(sorted, total, u32(id), rs, excludeAmbiguous, candLimit, distinct, lh, lane);
+            wave_sync_mem();
+            if (candLimit > 0) written = pick(distinct, out, lh, written, candLimit, h, counts, lane);
         } else {
-            const u32* sorted = gs;
+            u8* gh = reinterpret_cast<u8*>(gs + 2 * maxCand);
+            u32* sorted = gs;
             if (total <= regMax) gather_sort_any<kMaxK>(gs, counts, lists, h, total, lane);
             else sorted = gather_merge(gs, gs + maxCand, counts, lists, h, total, lane);
-            written = compact_unique(sorted, total, u32(id), rs, excludeAmbiguous, candLimit, out, gh, lane);
-        }
-        wave_sync_mem();
-        if (candLimit > 0 && written > candLimit) {
-            written = total <= capL ? keep_top(out, lh, written, candLimit, h, counts, lane)
-                                    : keep_top(out, gh, written, candLimit, h, counts, lane);
+            u32* distinct = candLimit > 0 ? (sorted == gs ? gs + maxCand : gs) : out;
+            written = compact_unique(sorted, total, u32(id), rs, excludeAmbiguous, candLimit, distinct, gh, lane);
+            wave_sync_mem();
+            if (candLimit > 0) written = pick(distinct, out, gh, written, candLimit, h, counts, lane);
         }
         if (lane == 0) {
             candCount[a] = written;
@@ -866,13 +879,13 @@ __global__ void __launch_bounds__(256) k_pack_offsets(const int* candCount, int 
     }
 }
 
-__global__ void __launch_bounds__(256) k_pack_candidates(const u32* candIds, const int* candCount, int n, int maxCand,
+__global__ void __launch_bounds__(256) k_pack_candidates(const u32* candIds, const int* candCount, int n, int pitch,
                                                          const u64* starts, u32* packed) {
     const int wpb = blockDim.x / kWave;
     for (int a = blockIdx.x * wpb + threadIdx.x / kWave; a < n; a += gridDim.x * wpb) {
         const u64 at = starts[a];
         const int c = candCount[a];
-        for (int i = lane_id(); i < c; i += kWave) packed[at + i] = candIds[u64(a) * maxCand + i];
+        for (int i = lane_id(); i < c; i += kWave) packed[at + i] = candIds[u64(a) * pitch + i];
     }
 }
 
@@ -898,14 +911,14 @@ int query_lds_bytes(int h, int cap, int maxLen, int threads, int candLimit, int 
     return int(size_t(threads / kWave) * query_wave_lds_bytes(capL, candLimit));
 }
 
-// Wavefronts of a query over n anchors: at most 16,384, two to four times what
-// the 256 compute units hold at once, each taking every so manieth anchor; a
-// spill row per wavefront instead of per anchor bounds the scratch.
-int query_spill_rows(int n) { return std::min(n, 1 << 14); }
+// Wavefronts of a query over n anchors: at most 4,096, what 256 compute units
+// hold at once, each taking every so manieth anchor; a spill row per wavefront
+// instead of per anchor bounds the scratch.
+int query_spill_rows(int n) { return std::min(n, 1 << 12); }
 
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
-                  int excludeAmbiguous, int candLimit, u32* candIds, int* candCount, u32* spill, int* rawCount,
-                  hipStream_t stream, const QueryAnchors& qa, const QueryHeavy& heavy) {
+                  int excludeAmbiguous, int candLimit, u32* candIds, int pitch, int* candCount, u32* spill,
+                  int* rawCount, hipStream_t stream, const QueryAnchors& qa, const QueryHeavy& heavy) {
     if (n <= 0) return;
     const int threads = 256;
     const int wpb = threads / kWave;
@@ -919,10 +932,10 @@ void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, 
     // used only when asked for lists of more than 1024 hits
     if (regMax > 16 * kWave)
         hipLaunchKernelGGL(k_query<32>, dim3(blocks), dim3(threads), lds, stream, rs, t, first, n, maxCand, capL, regMax,
-                           excludeAmbiguous, candLimit, candIds, candCount, spill, rawCount, qa, heavy);
+                           excludeAmbiguous, candLimit, candIds, pitch, candCount, spill, rawCount, qa, heavy);
     else
         hipLaunchKernelGGL(k_query<16>, dim3(blocks), dim3(threads), lds, stream, rs, t, first, n, maxCand, capL, regMax,
-                           excludeAmbiguous, candLimit, candIds, candCount, spill, rawCount, qa, heavy);
+                           excludeAmbiguous, candLimit, candIds, pitch, candCount, spill, rawCount, qa, heavy);
 }
 
 void launch_sum_counts(const int* rawCount, const int* candCount, int n, unsigned long long* totals, int* queue,
