@@ -172,6 +172,11 @@ struct care_context {
     DevBuf<unsigned long long> rawHits;
     DevBuf<float> qweights;
     PinnedBuf<int> hInts;
+    // gate training and evaluation: a chunk of raw features, the bf16
+    // features of a training set, logits of an evaluation (kept between calls)
+    DevBuf<float> mlpRaw, mlpLogits;
+    DevBuf<unsigned short> mlpX;
+    DevBuf<u32> mlpFlag;
     PinnedBuf<unsigned long long> hU64;
 
     care_batch_stats stats{};
@@ -1608,16 +1613,46 @@ extern "C" {
 extern "C++" {
 namespace {
 
-// features rounded to bf16 on the host, exactly as the device rounds
-std::vector<unsigned short> to_bf16(const float* x, uint64_t n) {
-    std::vector<unsigned short> out(size_t(n) * CARE_MLP_FEATURES);
-    for (size_t i = 0; i < out.size(); i++) {
-        unsigned u;
-        std::memcpy(&u, &x[i], 4);
-        u += 0x7FFFu + ((u >> 16) & 1u);
-        out[i] = (unsigned short)(u >> 16);
+// Rows of features on their way to the device: a chunk of raw floats at a
+// time is copied into the context's staging buffer and converted (training)
+// or evaluated there, so neither the rounding to bf16 nor the check for
+// non-finite values is a pass over the features on the host (6 of 8 ms at
+// 500,000 rows), and the staging buffer stays at 32 MB.
+constexpr uint64_t kFeatureChunk = uint64_t(1) << 18;
+
+// fn(rows of the chunk on the device, first row, rows) on every chunk, in
+// stream order; the staging buffer is reused behind the previous chunk's work
+template <class Fn>
+void for_feature_chunks(care_context* ctx, const float* features, uint64_t n, Fn&& fn) {
+    hipStream_t s = ctx->stream;
+    const uint64_t rows = std::min(n, kFeatureChunk);
+    if (ctx->mlpRaw.n < rows * CARE_MLP_FEATURES) ctx->mlpRaw.alloc(size_t(rows) * CARE_MLP_FEATURES);
+    if (!ctx->mlpFlag.p) ctx->mlpFlag.alloc(1);
+    launch_fill_u32(ctx->mlpFlag.p, 1, 0, s);
+    for (uint64_t first = 0; first < n; first += rows) {
+        const uint64_t m = std::min(rows, n - first);
+        HIP_TRY(hipMemcpyAsync(ctx->mlpRaw.p, features + first * CARE_MLP_FEATURES,
+                               sizeof(float) * size_t(m) * CARE_MLP_FEATURES, hipMemcpyHostToDevice, s));
+        fn(ctx->mlpRaw.p, first, m);
+        HIP_TRY(hipGetLastError());
     }
-    return out;
+}
+
+// whether every feature that for_feature_chunks passed was finite (waits)
+bool features_finite(care_context* ctx) {
+    HIP_TRY(hipMemcpyAsync(ctx->hInts.p, ctx->mlpFlag.p, sizeof(u32), hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    return ctx->hInts.p[0] == 0;
+}
+
+// index of the first label that is neither 0 nor 1, or n
+uint64_t first_bad_label(const uint8_t* labels, uint64_t n) {
+    unsigned any = 0;
+    for (uint64_t i = 0; i < n; i++) any |= labels[i];
+    if (any <= 1) return n;
+    uint64_t i = 0;
+    while (labels[i] <= 1) i++;
+    return i;
 }
 
 bool all_finite(const float* x, size_t n) {
@@ -1633,21 +1668,24 @@ int care_mlp_gradient(care_context* ctx, const float* features, const uint8_t* l
                       float* grad_out, float* loss_out) {
     if (!ctx || !features || !labels || !params || !grad_out) return fail(CARE_ERR_ARGUMENT, "null argument");
     if (n < 1 || n > (1 << 20)) return fail(CARE_ERR_ARGUMENT, "n %d outside 1..2^20", n);
-    if (!all_finite(features, size_t(n) * CARE_MLP_FEATURES) || !all_finite(params, CARE_MLP_PARAMS))
-        return fail(CARE_ERR_ARGUMENT, "non-finite input");
-    for (int i = 0; i < n; i++)
-        if (labels[i] > 1) return fail(CARE_ERR_ARGUMENT, "label %d is not 0 or 1", i);
+    if (!all_finite(params, CARE_MLP_PARAMS)) return fail(CARE_ERR_ARGUMENT, "non-finite input");
+    if (const uint64_t i = first_bad_label(labels, uint64_t(n)); i < uint64_t(n))
+        return fail(CARE_ERR_ARGUMENT, "label %d is not 0 or 1", int(i));
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
-        const std::vector<unsigned short> xb = to_bf16(features, uint64_t(n));
         std::vector<u32> perm(static_cast<size_t>(n));
         for (int i = 0; i < n; i++) perm[size_t(i)] = u32(i);
-        DevBuf<unsigned short> X, w1, w2, w3;
+        DevBuf<unsigned short>& X = ctx->mlpX;
+        DevBuf<unsigned short> w1, w2, w3;
         DevBuf<u8> Y;
         DevBuf<u32> P;
         DevBuf<float> master, partial, out;
-        X.alloc(xb.size());
+        if (X.n < size_t(n) * CARE_MLP_FEATURES) X.alloc(size_t(n) * CARE_MLP_FEATURES);
+        for_feature_chunks(ctx, features, uint64_t(n), [&](const float* raw, uint64_t first, uint64_t m) {
+            launch_mlp_convert(raw, m * CARE_MLP_FEATURES, X.p + first * CARE_MLP_FEATURES, ctx->mlpFlag.p, s);
+        });
+        if (!features_finite(ctx)) return fail(CARE_ERR_ARGUMENT, "non-finite input");
         Y.alloc(size_t(n));
         P.alloc(size_t(n));
         master.alloc(CARE_MLP_PARAMS);
@@ -1657,7 +1695,6 @@ int care_mlp_gradient(care_context* ctx, const float* features, const uint8_t* l
         const int np = mlp_partials(n);
         partial.alloc(size_t(np) * mlp_partial_stride());
         out.alloc(CARE_MLP_PARAMS + 1);
-        HIP_TRY(hipMemcpy(X.p, xb.data(), xb.size() * 2, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(Y.p, labels, size_t(n), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(P.p, perm.data(), perm.size() * 4, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(master.p, params, sizeof(float) * CARE_MLP_PARAMS, hipMemcpyHostToDevice));
@@ -1684,18 +1721,22 @@ int care_mlp_train(care_context* ctx, const float* features, const uint8_t* labe
     if (o->epochs < 1 || o->batch < 16 || o->batch > (1 << 16) || !(o->lr > 0.f))
         return fail(CARE_ERR_ARGUMENT, "invalid training options");
     if (!all_finite(params, CARE_MLP_PARAMS)) return fail(CARE_ERR_ARGUMENT, "non-finite initial parameters");
-    if (!all_finite(features, size_t(n) * CARE_MLP_FEATURES)) return fail(CARE_ERR_ARGUMENT, "non-finite features");
-    for (uint64_t i = 0; i < n; i++)
-        if (labels[i] > 1) return fail(CARE_ERR_ARGUMENT, "label %llu is not 0 or 1", (unsigned long long)i);
+    const uint64_t badLabel = first_bad_label(labels, n);
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
-        const std::vector<unsigned short> xb = to_bf16(features, n);
-        DevBuf<unsigned short> X, w1, w2, w3;
+        DevBuf<unsigned short>& X = ctx->mlpX;
+        DevBuf<unsigned short> w1, w2, w3;
         DevBuf<u8> Y;
         DevBuf<u32> P;
         DevBuf<float> master, m1, m2, partial, loss;
-        X.alloc(xb.size());
+        if (X.n < size_t(n) * CARE_MLP_FEATURES) X.alloc(size_t(n) * CARE_MLP_FEATURES);
+        for_feature_chunks(ctx, features, n, [&](const float* raw, uint64_t first, uint64_t m) {
+            launch_mlp_convert(raw, m * CARE_MLP_FEATURES, X.p + first * CARE_MLP_FEATURES, ctx->mlpFlag.p, s);
+        });
+        if (!features_finite(ctx)) return fail(CARE_ERR_ARGUMENT, "non-finite features");
+        if (badLabel < n)
+            return fail(CARE_ERR_ARGUMENT, "label %llu is not 0 or 1", (unsigned long long)badLabel);
         Y.alloc(size_t(n));
         P.alloc(size_t(n));
         master.alloc(CARE_MLP_PARAMS);
@@ -1707,7 +1748,6 @@ int care_mlp_train(care_context* ctx, const float* features, const uint8_t* labe
         const int np = mlp_partials(o->batch);
         partial.alloc(size_t(np) * mlp_partial_stride());
         loss.alloc(1);
-        HIP_TRY(hipMemcpy(X.p, xb.data(), xb.size() * 2, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(Y.p, labels, size_t(n), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(master.p, params, sizeof(float) * CARE_MLP_PARAMS, hipMemcpyHostToDevice));
         std::vector<float> zeros(CARE_MLP_PARAMS, 0.f);
@@ -1758,25 +1798,24 @@ int care_mlp_train(care_context* ctx, const float* features, const uint8_t* labe
 int care_mlp_infer(care_context* ctx, const float* features, uint64_t n, const float* params, float* logits) {
     if (!ctx || !features || !params || !logits) return fail(CARE_ERR_ARGUMENT, "null argument");
     if (n < 1 || n > (uint64_t(1) << 32)) return fail(CARE_ERR_ARGUMENT, "n out of range");
-    if (!all_finite(features, size_t(n) * CARE_MLP_FEATURES) || !all_finite(params, CARE_MLP_PARAMS))
-        return fail(CARE_ERR_ARGUMENT, "non-finite input");
+    if (!all_finite(params, CARE_MLP_PARAMS)) return fail(CARE_ERR_ARGUMENT, "non-finite input");
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
-        const std::vector<unsigned short> xb = to_bf16(features, n);
-        DevBuf<unsigned short> X, w1, w2, w3;
-        DevBuf<float> master, z;
-        X.alloc(xb.size());
+        DevBuf<unsigned short> w1, w2, w3;
+        DevBuf<float> master;
+        DevBuf<float>& z = ctx->mlpLogits;
         master.alloc(CARE_MLP_PARAMS);
         w1.alloc(64 * 32);
         w2.alloc(32 * 64);
         w3.alloc(16 * 32);
-        z.alloc(size_t(n));
-        HIP_TRY(hipMemcpy(X.p, xb.data(), xb.size() * 2, hipMemcpyHostToDevice));
+        if (z.n < size_t(n)) z.alloc(size_t(n));
         HIP_TRY(hipMemcpy(master.p, params, sizeof(float) * CARE_MLP_PARAMS, hipMemcpyHostToDevice));
         launch_mlp_cast(master.p, w1.p, w2.p, w3.p, s);
-        launch_mlp_forward(X.p, n, w1.p, w2.p, w3.p, master.p, z.p, s);
-        HIP_TRY(hipGetLastError());
+        for_feature_chunks(ctx, features, n, [&](const float* raw, uint64_t first, uint64_t m) {
+            launch_mlp_forward(raw, m, w1.p, w2.p, w3.p, master.p, z.p + first, ctx->mlpFlag.p, s);
+        });
+        if (!features_finite(ctx)) return fail(CARE_ERR_ARGUMENT, "non-finite input");
         HIP_TRY(hipMemcpyAsync(logits, z.p, size_t(n) * 4, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
     } catch (const HipError& e) {

@@ -264,7 +264,10 @@ void launch_mlp_reduce(const float* partial, int nPartials, int mode, float* out
                        unsigned short* w2b, unsigned short* w3b, float* lossAcc, hipStream_t s);
 void launch_mlp_cast(const float* master, unsigned short* w1b, unsigned short* w2b, unsigned short* w3b,
                      hipStream_t s);
-void launch_mlp_forward(const unsigned short* X, u64 n, const unsigned short* w1b, const unsigned short* w2b,
-                        const unsigned short* w3b, const float* master, float* zOut, hipStream_t s);
+// X: float features; flag[0] = 1 if one of them is not finite
+void launch_mlp_forward(const float* X, u64 n, const unsigned short* w1b, const unsigned short* w2b,
+                        const unsigned short* w3b, const float* master, float* zOut, u32* flag, hipStream_t s);
+// n floats (a multiple of 8) to bf16; flag[0] = 1 if one of them is not finite
+void launch_mlp_convert(const float* in, u64 n, unsigned short* out, u32* flag, hipStream_t s);
 
 }  // namespace care_engine

@@ -35,6 +35,21 @@ __device__ __forceinline__ ushort4v load4_strided(const bf16raw* p, int stride) 
     return v;
 }
 
+// eight floats (16-byte aligned) rounded to bf16; `bad` is set if one of
+// them is not finite
+__device__ __forceinline__ ushort8 convert8(const float* p, bool& bad) {
+    const floatx4 a = *reinterpret_cast<const floatx4*>(p), b = *reinterpret_cast<const floatx4*>(p + 4);
+    ushort8 v;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        bad |= (__float_as_uint(a[j]) & 0x7F800000u) == 0x7F800000u;
+        bad |= (__float_as_uint(b[j]) & 0x7F800000u) == 0x7F800000u;
+        v[j] = f2bf(a[j]);
+        v[4 + j] = f2bf(b[j]);
+    }
+    return v;
+}
+
 }  // namespace
 
 // One wave per tile of 16 rows: forward, binary cross-entropy with mean over
@@ -197,8 +212,12 @@ __global__ void __launch_bounds__(kReduceParams * kReduceGroups)
     const int j = threadIdx.x % kReduceParams, grp = threadIdx.x / kReduceParams;
     const int i = blockIdx.x * kReduceParams + j;
     float s = 0.f;
-    if (i <= kMlpParams)
+    // eight loads in flight, added in order: one after the other they took a
+    // trip to L2 each (32 of them at 4,096 rows)
+    if (i <= kMlpParams) {
+#pragma unroll 8
         for (int p = grp; p < nPartials; p += kReduceGroups) s += partial[u64(p) * kPartialStride + i];
+    }
     sPart[grp][j] = s;
     __syncthreads();
     if (grp != 0 || i > kMlpParams) return;
@@ -231,9 +250,19 @@ __global__ void k_mlp_cast(const float* master, bf16raw* w1b, bf16raw* w2b, bf16
     if (i < kMlpH3 * kMlpH2) w3b[i] = f2bf(master[kMlpW3 + i]);
 }
 
-// Stand-alone forward pass: one wave per tile of 16 rows of X (bf16), z out.
-__global__ void __launch_bounds__(256) k_mlp_forward(const bf16raw* X, u64 n, const bf16raw* w1b, const bf16raw* w2b,
-                                                     const bf16raw* w3b, const float* master, float* zOut) {
+// n / 8 groups of eight features to bf16
+__global__ void __launch_bounds__(256) k_mlp_convert(const float* in, u64 groups, bf16raw* out, u32* flag) {
+    bool bad = false;
+    for (u64 i = blockIdx.x * u64(blockDim.x) + threadIdx.x; i < groups; i += u64(gridDim.x) * blockDim.x)
+        *reinterpret_cast<ushort8*>(out + 8 * i) = convert8(in + 8 * i, bad);
+    if (bad) atomicExch(reinterpret_cast<int*>(flag), 1);
+}
+
+// Stand-alone forward pass: one wave per tile of 16 rows of X, rounded to
+// bf16 here, z out.
+__global__ void __launch_bounds__(256) k_mlp_forward(const float* X, u64 n, const bf16raw* w1b, const bf16raw* w2b,
+                                                     const bf16raw* w3b, const float* master, float* zOut,
+                                                     u32* flag) {
     __shared__ __attribute__((aligned(16))) bf16raw sX[4][16 * kMlpIn];
     __shared__ __attribute__((aligned(16))) char sScratch[4][kMlpTileScratch];
     __shared__ float sZ[4][16];
@@ -242,7 +271,9 @@ __global__ void __launch_bounds__(256) k_mlp_forward(const bf16raw* X, u64 n, co
     {
         const int row = lane >> 2, part = lane & 3;
         ushort8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (row0 + row < n) v = load8(X + (row0 + row) * kMlpIn + 8 * part);
+        bool bad = false;
+        if (row0 + row < n) v = convert8(X + (row0 + row) * kMlpIn + 8 * part, bad);
+        if (bad) atomicExch(reinterpret_cast<int*>(flag), 1);
         *reinterpret_cast<ushort8*>(sX[wave] + row * kMlpIn + 8 * part) = v;
     }
     wave_fence();
@@ -283,11 +314,19 @@ void launch_mlp_cast(const float* master, bf16raw* w1b, bf16raw* w2b, bf16raw* w
     hipLaunchKernelGGL(k_mlp_cast, dim3((kMlpH1 * kMlpIn + 255) / 256), dim3(256), 0, s, master, w1b, w2b, w3b);
 }
 
-void launch_mlp_forward(const bf16raw* X, u64 n, const bf16raw* w1b, const bf16raw* w2b, const bf16raw* w3b,
-                        const float* master, float* zOut, hipStream_t s) {
+void launch_mlp_convert(const float* in, u64 n, bf16raw* out, u32* flag, hipStream_t s) {
+    const u64 groups = n / 8;
+    if (groups == 0) return;
+    const u64 blocks = (groups + 255) / 256;
+    hipLaunchKernelGGL(k_mlp_convert, dim3(unsigned(blocks < 8192 ? blocks : 8192)), dim3(256), 0, s, in, groups, out,
+                       flag);
+}
+
+void launch_mlp_forward(const float* X, u64 n, const bf16raw* w1b, const bf16raw* w2b, const bf16raw* w3b,
+                        const float* master, float* zOut, u32* flag, hipStream_t s) {
     if (n == 0) return;
     const u64 blocks = (n + 63) / 64;
-    hipLaunchKernelGGL(k_mlp_forward, dim3(unsigned(blocks)), dim3(256), 0, s, X, n, w1b, w2b, w3b, master, zOut);
+    hipLaunchKernelGGL(k_mlp_forward, dim3(unsigned(blocks)), dim3(256), 0, s, X, n, w1b, w2b, w3b, master, zOut, flag);
 }
 
 }  // namespace care_engine
