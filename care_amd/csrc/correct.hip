@@ -125,7 +125,7 @@ struct LdsDims {
         b += (size_t(maxLen) + 3) / 4 * 4;
         b += size_t(chunk) * 2 * sizeof(uint2) * pw();
         b += (size_t(cols) + 3) / 4 * 4;
-        b += sizeof(float) * cols + sizeof(int) * (2 * cols + 1);
+        b += (sizeof(float) * size_t(cols) + 15) / 16 * 16 + sizeof(int) * (2 * size_t(cols) + 1);
         b += 4 * sizeof(u16) * cols + 4 * sizeof(float) * cols;
         b += (sizeof(u16) * size_t(cols) + 3) / 4 * 4;
         b += 32 * sizeof(int);
@@ -140,6 +140,7 @@ __device__ Lds carve(char* base, const LdsDims& d) {
     Lds l;
     char* p = base;
     // 16-byte aligned base: 16- and 8-byte records first
+    l.support = reinterpret_cast<float*>(p); p += (sizeof(float) * size_t(d.cols) + 15) / 16 * 16;
     l.mst = reinterpret_cast<CandMeta*>(p); p += sizeof(CandMeta) * d.chunk;
     l.ap = reinterpret_cast<uint2*>(p); p += sizeof(uint2) * d.pw();
     l.arp = reinterpret_cast<uint2*>(p); p += sizeof(uint2) * d.pw();
@@ -150,7 +151,6 @@ __device__ Lds carve(char* base, const LdsDims& d) {
     l.aw = reinterpret_cast<u32*>(p); p += sizeof(u32) * d.pitch;
     l.differ = reinterpret_cast<u32*>(p); p += sizeof(u32) * d.pitch;
     l.qbin = reinterpret_cast<float*>(p); p += sizeof(float) * 4;
-    l.support = reinterpret_cast<float*>(p); p += sizeof(float) * d.cols;
     l.coverage = reinterpret_cast<int*>(p); p += sizeof(int) * (d.cols + 1);
     l.origCov = reinterpret_cast<int*>(p); p += sizeof(int) * d.cols;
     l.wgt = reinterpret_cast<float*>(p); p += 4 * sizeof(float) * d.cols;
@@ -684,10 +684,14 @@ __device__ __forceinline__ void align_inside(const AlignCtx& A, int c, int dMax,
         const uint2* pf = A.cpl + size_t(2 * c) * A.pw + (dd >> 5) + ((dd & 31) != 0);
         const uint2* pr = pf + A.pw;
         const uint2 f0 = pf[0], f1 = pf[1], f2 = pf[2], r0 = pr[0], r1 = pr[1], r2 = pr[2];
-        const u32 xf = (__builtin_amdgcn_alignbit(f0.x, f1.x, sh) ^ a1.x) | (__builtin_amdgcn_alignbit(f0.y, f1.y, sh) ^ a1.y);
-        const u32 xr = (__builtin_amdgcn_alignbit(r0.x, r1.x, sh) ^ a1.x) | (__builtin_amdgcn_alignbit(r0.y, r1.y, sh) ^ a1.y);
-        const u32 yf = (__builtin_amdgcn_alignbit(f1.x, f2.x, sh) ^ a2.x) | (__builtin_amdgcn_alignbit(f1.y, f2.y, sh) ^ a2.y);
-        const u32 yr = (__builtin_amdgcn_alignbit(r1.x, r2.x, sh) ^ a2.x) | (__builtin_amdgcn_alignbit(r1.y, r2.y, sh) ^ a2.y);
+        const u32 xf = (__builtin_amdgcn_alignbit(f0.x, f1.x, sh) ^ a1.x) |
+                       (__builtin_amdgcn_alignbit(f0.y, f1.y, sh) ^ a1.y);
+        const u32 xr = (__builtin_amdgcn_alignbit(r0.x, r1.x, sh) ^ a1.x) |
+                       (__builtin_amdgcn_alignbit(r0.y, r1.y, sh) ^ a1.y);
+        const u32 yf = (__builtin_amdgcn_alignbit(f1.x, f2.x, sh) ^ a2.x) |
+                       (__builtin_amdgcn_alignbit(f1.y, f2.y, sh) ^ a2.y);
+        const u32 yr = (__builtin_amdgcn_alignbit(r1.x, r2.x, sh) ^ a2.x) |
+                       (__builtin_amdgcn_alignbit(r1.y, r2.y, sh) ^ a2.y);
         const int mf = __popc(xf & m1) + __popc(yf & m2), mr = __popc(xr & m1) + __popc(yr & m2);
         queue_survivors(A, c, d <= dMax && min(mf, mr) < lim, nPos - 1 + d, mf, mr, 2, count);
     }
@@ -851,10 +855,23 @@ __device__ ColumnStats column_stats_wave(const Lds& L, int first, int last) {
     cs.maxCov = wave_max_int(mxc);
     float sum = 0.0f;
     if (lane == 0) {
-        // reads of 32 columns in flight: the additions wait for LDS five times
-        // in 150 columns instead of nineteen times
-#pragma unroll 32
-        for (int c = first; c < last; c++) sum += L.support[c];
+        // four columns a read, sixteen in flight: a read per column issued as
+        // many instructions again as the additions
+        int c = first;
+        for (; c < last && (c & 3); c++) sum += L.support[c];
+        for (; c + 16 <= last; c += 16) {
+            float4 v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = *reinterpret_cast<const float4*>(L.support + c + 4 * k);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                sum += v[k].x;
+                sum += v[k].y;
+                sum += v[k].z;
+                sum += v[k].w;
+            }
+        }
+        for (; c < last; c++) sum += L.support[c];
     }
     cs.avgSupport = sum / float(last - first);
     return cs;
@@ -1142,9 +1159,9 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
         // the binary searches in the mate's candidate list) run in parallel
         // the mate's candidate list is searched in LDS when it fits the
         // alignment keys and survivor slices, which are free until this
-        // chunk's alignment starts (not in the gated modes, where its
-        // registers would cost a wavefront per SIMD)
-        const int mateCap = kGated ? -1 : 2 * dims.chunk + 2 * kSurvivors * dims.waves;
+        // chunk's alignment starts (a search in global memory is a chain of
+        // five or six loads)
+        const int mateCap = 2 * dims.chunk + 2 * kSurvivors * dims.waves;
         for (int c0 = 0; c0 < n; c0 += dims.chunk) {
             const int nc = min(dims.chunk, n - c0);
             __syncthreads();  // the previous chunk's rows and keys are no longer read
@@ -1546,58 +1563,81 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
                 // learned gate on candidate columns (gated mode only): the
                 // forest's candidate range and decision rule, the MLP deciding
                 const bool gateC = kGateCands && P.correctionTypeCands == 3;
-                for (int c = wave; c < m; c += nwaves) {
-                    const CandMeta cm = cur[c];
-                    const int qb = msa.ab + cm.shift;
-                    const int qe = qb + cm.len;
-                    const bool inRange = (forestC || gateC)
-                                             ? (qb >= msa.ab - P.newColumns && qe <= ae + P.newColumns)
-                                             : (msa.ab - P.newColumns <= qb && qb <= msa.ab + P.newColumns &&
-                                                qe <= ae + P.newColumns);
-                    if (!inRange) continue;
-                    int slot = 0;
-                    if (lane == 0) slot = atomicAdd(P.candOutCount, 1);
-                    slot = __shfl(slot, 0, kWave);
-                    if (slot >= P.candOutCap) continue;
-                    CARE_CHECK(cm.id < rs.n && qb >= 0 && qe <= msa.cols);
-                    if (lane == 0) P.candOutIds[slot] = cm.id;
-                    ColumnStats ccs{};
-                    if (forestC || gateC) {
-                        ccs = column_stats_wave(L, qb, qe);
-                        ccs.avgSupport = __uint_as_float(
-                            u32(__builtin_amdgcn_readlane(int(__float_as_uint(ccs.avgSupport)), 0)));
-                    }
-                    // jaccard of the anchor and candidate column ranges
-                    const float jac = float(min(ae, qe) - max(msa.ab, qb)) / float(max(ae, qe) - min(msa.ab, qb));
-                    char* dst = P.candOutSeq + u64(slot) * P.outPitch;
-                    const bool rc = cm.flag == 2;
-                    const u32* enc = rs.seqs + u64(cm.id) * rs.pitch;
-                    u8* cacc = nullptr;
-                    if (gateC) {
-                        char* ws = L.gscr + size_t(wave) * cand_gate_scratch(dims.maxLen);
-                        CARE_CHECK(ws + cand_gate_scratch(dims.maxLen) <= reinterpret_cast<char*>(L.qw));
-                        cacc = reinterpret_cast<u8*>(ws + kCandGateTile);
-                        gate_candidate(P, L, rs, msa.cols, qb, cm, m, ccs, ws, cacc);
-                    }
-                    for (int i = lane; i < cm.len; i += kWave) {
-                        // position i of the candidate in MSA orientation, written
-                        // to its forward-strand position
-                        const int col = qb + i;
-                        u32 b = L.cons[col];
-                        if (forestC) {
-                            const u32 orig = oriented_base(enc, cm.len, i, rc);
-                            if (b != orig) {
-                                float f[14];
-                                column_features(L, msa.cols, col, orig, ccs, P.estimatedCoverage, f);
-                                f[13] = jac;
-                                if (!forest_decide(P.forestC, f)) b = orig;
-                            }
-                        } else if (gateC) {
-                            const u32 orig = oriented_base(enc, cm.len, i, rc);
-                            if (b != orig && !cacc[i]) b = orig;
+                auto inRange = [&](const CandMeta& cm) {
+                    const int qb = msa.ab + cm.shift, qe = qb + cm.len;
+                    return (forestC || gateC) ? (qb >= msa.ab - P.newColumns && qe <= ae + P.newColumns)
+                                              : (msa.ab - P.newColumns <= qb && qb <= msa.ab + P.newColumns &&
+                                                 qe <= ae + P.newColumns);
+                };
+                // a wavefront takes 16 candidates at a time: one lane each
+                // tests the range, and one atomic gets the rows of all that
+                // are inside (one per candidate made every candidate wait for
+                // its own round trip to the counter)
+                constexpr int kGroup = 16;
+                for (int c0 = wave * kGroup; c0 < m; c0 += nwaves * kGroup) {
+                    bool mine = false;
+                    if (lane < kGroup && c0 + lane < m) mine = inRange(load_meta(cur + c0 + lane));
+                    u64 todo = __ballot(mine);
+                    int next = 0;
+                    if (lane == 0 && todo) next = atomicAdd(P.candOutCount, __popcll(todo));
+                    next = __builtin_amdgcn_readfirstlane(next);
+                    for (; todo; todo &= todo - 1) {
+                        const int slot = next++;
+                        if (slot >= P.candOutCap) break;  // counted, reported by the host
+                        const CandMeta cm = load_meta(cur + c0 + __ffsll((long long)todo) - 1);
+                        const int qb = msa.ab + cm.shift;
+                        const int qe = qb + cm.len;
+                        CARE_CHECK(cm.id < rs.n && qb >= 0 && qe <= msa.cols);
+                        if (lane == 0) P.candOutIds[slot] = cm.id;
+                        ColumnStats ccs{};
+                        if (forestC || gateC) {
+                            ccs = column_stats_wave(L, qb, qe);
+                            ccs.avgSupport = __uint_as_float(
+                                u32(__builtin_amdgcn_readlane(int(__float_as_uint(ccs.avgSupport)), 0)));
                         }
-                        const int out = rc ? cm.len - 1 - i : i;
-                        dst[out] = base_char(rc ? 3u - b : b);
+                        // jaccard of the anchor and candidate column ranges
+                        const float jac = float(min(ae, qe) - max(msa.ab, qb)) / float(max(ae, qe) - min(msa.ab, qb));
+                        char* dst = P.candOutSeq + u64(slot) * P.outPitch;
+                        const bool rc = cm.flag == 2;
+                        const u32* enc = rs.seqs + u64(cm.id) * rs.pitch;
+                        u8* cacc = nullptr;
+                        if (gateC) {
+                            char* ws = L.gscr + size_t(wave) * cand_gate_scratch(dims.maxLen);
+                            CARE_CHECK(ws + cand_gate_scratch(dims.maxLen) <= reinterpret_cast<char*>(L.qw));
+                            cacc = reinterpret_cast<u8*>(ws + kCandGateTile);
+                            gate_candidate(P, L, rs, msa.cols, qb, cm, m, ccs, ws, cacc);
+                        }
+                        // the candidate's character at forward-strand position o
+                        auto corrected = [&](int o) {
+                            const int i = rc ? cm.len - 1 - o : o;  // in MSA orientation
+                            const int col = qb + i;
+                            u32 b = L.cons[col];
+                            if (forestC) {
+                                const u32 orig = oriented_base(enc, cm.len, i, rc);
+                                if (b != orig) {
+                                    float f[14];
+                                    column_features(L, msa.cols, col, orig, ccs, P.estimatedCoverage, f);
+                                    f[13] = jac;
+                                    if (!forest_decide(P.forestC, f)) b = orig;
+                                }
+                            } else if (gateC) {
+                                const u32 orig = oriented_base(enc, cm.len, i, rc);
+                                if (b != orig && !cacc[i]) b = orig;
+                            }
+                            return u32(u8(base_char(rc ? 3u - b : b)));
+                        };
+                        if (forestC || gateC) {
+                            for (int o = lane; o < cm.len; o += kWave) dst[o] = char(corrected(o));
+                        } else {
+                            // four characters a store: rows are 16-byte aligned
+                            for (int o = 4 * lane; o < cm.len; o += 4 * kWave) {
+                                u32 v = 0;
+                                const int k = min(4, cm.len - o);
+                                for (int j = 0; j < k; j++) v |= corrected(o + j) << (8 * j);
+                                if (k == 4) *reinterpret_cast<u32*>(dst + o) = v;
+                                else for (int j = 0; j < k; j++) dst[o + j] = char(v >> (8 * j));
+                            }
+                        }
                     }
                 }
             }

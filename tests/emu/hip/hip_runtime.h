@@ -48,6 +48,9 @@ struct uint2 {
     unsigned x, y;
 };
 inline uint2 make_uint2(unsigned a, unsigned b) { return uint2{a, b}; }
+struct alignas(16) float4 {
+    float x, y, z, w;
+};
 struct alignas(16) uint4 {
     unsigned x, y, z, w;
 };
@@ -463,11 +466,12 @@ inline T __shfl_xor(T v, int mask, int width = 64) {
     return emu::exchange(v, (emu::lane() ^ mask) & 63);
 }
 // DPP moves used by the kernels (source lane within the 16-lane row):
-// quad_perm 0x00-0xFF, row_mirror 0x140, row_half_mirror 0x141
+// quad_perm 0x00-0xFF, row_ror:8 0x128, row_mirror 0x140, row_half_mirror 0x141
 inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool) {
     const int l = emu::lane(), row = l & ~15, i = l & 15;
     int src;
     if (ctrl >= 0 && ctrl <= 0xFF) src = (l & ~3) | ((ctrl >> (2 * (l & 3))) & 3);
+    else if (ctrl == 0x128) src = row | ((i + 8) & 15);
     else if (ctrl == 0x140) src = row | (15 - i);
     else if (ctrl == 0x141) src = row | (i & 8) | (7 - (i & 7));
     else {
