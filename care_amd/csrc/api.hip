@@ -275,15 +275,15 @@ void ensure_batch(care_context* ctx, int B, int n) {
 // a quarter of the device memory free when the context was created, between 2
 // and 4 GiB, and a batch holds at most 2^18 anchors.  Fewer, larger batches
 // mean fewer launches and fewer drains of the persistent correction kernel,
-// so a call is cut into eight at the least; beyond that larger batches only
-// take memory.
+// so a call is cut into eight at the least and none smaller than 65,536
+// anchors; beyond that larger batches only take memory.
 int default_batch(care_context* ctx, int n) {
     if (ctx->requestedBatch > 0) return ctx->requestedBatch;
     const size_t perAnchor = size_t(row_candidates(ctx)) * sizeof(u32) + ctx->rs.maxLen + 64;
     const size_t budget = std::min(std::max(ctx->freeAtCreate / 4, size_t(2) << 30), size_t(4) << 30);
     size_t b = budget / perAnchor;
     b = std::max<size_t>(256, std::min<size_t>(b, size_t(1) << 18));
-    if (n > 0) b = std::min<size_t>(b, std::max(32768, n / 8));
+    if (n > 0) b = std::min<size_t>(b, std::max(65536, n / 8));
     return int(b & ~size_t(1));
 }
 
@@ -298,7 +298,7 @@ int default_batch(care_context* ctx, int n) {
 int correct_threads(const care_context* ctx, int n) {
     if (ctx->blockThreads) return ctx->blockThreads;
     const int fill = 8 * ctx->numCUs;
-    return n > (ctx->opt.candidate_limit > 0 ? fill : 32 * fill) ? 128 : 256;
+    return n >= (ctx->opt.candidate_limit > 0 ? fill : 32 * fill) ? 128 : 256;
 }
 
 // Candidates from which an anchor is corrected before the others: about twice

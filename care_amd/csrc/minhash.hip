@@ -512,6 +512,19 @@ __device__ __forceinline__ Buf gather_merge(Buf a, Buf b, const int* counts, con
     return src;
 }
 
+// value of lane ^ x, x a power of two known at compile time: within a row of
+// 16 lanes by DPP moves (x = 4 as lane ^ 7 ^ 3, x = 8 a rotation by 8), which
+// wait for no LDS round trip as a shuffle (ds_bpermute) does; all lanes active
+__device__ __forceinline__ u32 lane_xor(u32 v, int x) {
+    if (x == 1) return u32(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true));
+    if (x == 2) return u32(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true));
+    if (x == 4)
+        return u32(__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(int(v), 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF,
+                                            true));
+    if (x == 8) return u32(__builtin_amdgcn_mov_dpp(int(v), 0x128, 0xF, 0xF, true));
+    return __shfl_xor(v, x, kWave);
+}
+
 // Bitonic sort of 64*K entries held in registers, entry e = lane*K + r in
 // register r: strides below K stay inside a lane, larger ones exchange with
 // lane ^ (stride / K).  Every loop bound is a constant, so the network is
@@ -526,7 +539,9 @@ __device__ __forceinline__ void sort_in_registers(u32 (&v)[K], int lane) {
                 const int lx = stride / K;
 #pragma unroll
                 for (int r = 0; r < K; r++) {
-                    const u32 o = __shfl_xor(v[r], lx, kWave);
+                    // (the 32-entry network has registers for shuffles only: with
+                    // moves it holds 145 and a wavefront per SIMD less)
+                    const u32 o = K < 32 ? lane_xor(v[r], lx) : __shfl_xor(v[r], lx, kWave);
                     const int e = lane * K + r;
                     const bool up = (e & size) == 0;
                     const bool lower = (e & stride) == 0;
