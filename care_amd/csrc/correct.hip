@@ -336,6 +336,7 @@ __device__ Msa build_msa(const CorrectParams& P, const Lds& L, const LdsDims& di
             store_meta(L.mst + i, load_meta(meta + c0 + i));
         }
         if (r0S < rowsS)
+#pragma unroll 2
             for (int c = r0S; c < nc; c += rowsS) {
                 const CandMeta cm = load_meta(meta + c0 + c);
                 const u32* row = rs.seqs + u64(cm.id) * pitch;
@@ -344,6 +345,7 @@ __device__ Msa build_msa(const CorrectParams& P, const Lds& L, const LdsDims& di
         if (!quals || !qpitch) return;
         const int r0Q = (tx * dims.invQ) >> 16, wQ = tx - r0Q * qpitch;
         if (r0Q < rowsQ)
+#pragma unroll 2
             for (int c = r0Q; c < nc; c += rowsQ) {
                 const CandMeta cm = load_meta(meta + c0 + c);
                 const u32* row = rs.quals + u64(cm.id) * qpitch;
@@ -1169,43 +1171,48 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
             if (mateIds && mateN <= mateCap)
                 for (int i = tid; i < mateN; i += blockDim.x) L.keys[i] = mateIds[i];
             __syncthreads();
+            // 2-bit rows, a word a thread; several rows' loads in flight
             const int rS = (tid * dims.invS) >> 16, w = tid - rS * rs.pitch;
-            for (int c = rS < dims.stepS ? rS : nc; c < nc; c += dims.stepS) {
-                const int i = c * rs.pitch + w;
+#pragma unroll 4
+            for (int c = rS < dims.stepS ? rS : nc; c < nc; c += dims.stepS)
+                L.rows[c * rs.pitch + w] = rs.seqs[u64(ids[c0 + c]) * rs.pitch + w];
+            // ids, lengths and pair flags, a candidate a thread: searched by
+            // the threads of the rows' first words, every few rows' loads
+            // waited for a search by a tenth of the lanes
+            for (int c = tid; c < nc; c += blockDim.x) {
                 const u32 cid = ids[c0 + c];
                 CARE_CHECK(cid < rs.n && cid != u32(id) && c < dims.chunk);
-                L.rows[i] = rs.seqs[u64(cid) * rs.pitch + w];
-                if (w == 0) {
-                    L.mst[c].id = cid;
-                    const int lc = rs.lens[cid];
-                    L.mst[c].len = u16(lc);
-                    if (lc != la) sFlag = 1;
-                    L.mst[c].shift = short(min(int(float(lc) * P.maxErrorRate), 32767));  // mismatch limit
-                    // the candidate's mate is a candidate of the anchor's mate
-                    // (include/corrector.hpp:763-807)
-                    u8 paired = 0;
-                    if (mateIds) {
-                        const u32 want = cid ^ 1u;
-                        CARE_CHECK(mateN >= 0 && mateN <= P.maxCand);
-                        int lo2 = 0, hi2 = mateN;
-                        if (mateN <= mateCap) {
-                            while (lo2 < hi2) {
-                                const int mid = (lo2 + hi2) >> 1;
-                                if (L.keys[mid] < want) lo2 = mid + 1;
-                                else hi2 = mid;
-                            }
-                            paired = (lo2 < mateN && L.keys[lo2] == want) ? 1 : 0;
-                        } else {
-                            while (lo2 < hi2) {
-                                const int mid = (lo2 + hi2) >> 1;
-                                if (mateIds[mid] < want) lo2 = mid + 1;
-                                else hi2 = mid;
-                            }
-                            paired = (lo2 < mateN && mateIds[lo2] == want) ? 1 : 0;
+                const int lc = rs.lens[cid];
+                if (lc != la) sFlag = 1;
+                // the candidate's mate is a candidate of the anchor's mate
+                // (include/corrector.hpp:763-807)
+                u8 paired = 0;
+                if (mateIds) {
+                    const u32 want = cid ^ 1u;
+                    CARE_CHECK(mateN >= 0 && mateN <= P.maxCand);
+                    int lo2 = 0, hi2 = mateN;
+                    if (mateN <= mateCap) {
+                        while (lo2 < hi2) {
+                            const int mid = (lo2 + hi2) >> 1;
+                            if (L.keys[mid] < want) lo2 = mid + 1;
+                            else hi2 = mid;
                         }
+                        paired = (lo2 < mateN && L.keys[lo2] == want) ? 1 : 0;
+                    } else {
+                        while (lo2 < hi2) {
+                            const int mid = (lo2 + hi2) >> 1;
+                            if (mateIds[mid] < want) lo2 = mid + 1;
+                            else hi2 = mid;
+                        }
+                        paired = (lo2 < mateN && mateIds[lo2] == want) ? 1 : 0;
                     }
-                    L.mst[c].paired = paired;
                 }
+                CandMeta m{};
+                m.id = cid;
+                m.len = u16(lc);
+                m.shift = short(min(int(float(lc) * P.maxErrorRate), 32767));  // mismatch limit
+                m.paired = paired;
+                store_meta(L.mst + c, m);
             }
             __syncthreads();
             // bit planes of every staged candidate (word 0 is padding): forward ...
