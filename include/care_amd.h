@@ -275,11 +275,14 @@ typedef struct care_tuning {
     int batch_anchors;          /* anchors per internal launch, even (0 = automatic); a call of
                                    more than one launch ends in one of batch_anchors / 8 */
     int correct_threads;        /* threads per correction workgroup, i.e. 2, 3 or 4
-                                   wavefronts per anchor: 128, 192 or 256 (0 = 256) */
+                                   wavefronts per anchor: 128, 192 or 256
+                                   (0 = automatic: 128 on large calls, 256 on
+                                   small ones; reported as for a large call) */
     int correct_blocks_per_cu;  /* persistent correction workgroups per compute unit
                                    (0 = as many as are resident at once) */
     int msa_chunk;              /* candidates staged in LDS per MSA pass, 16..256
-                                   (0 = automatic: about 16 KB of rows) */
+                                   (0 = automatic: at most 16 KB of rows, fewer
+                                   where LDS would hold back workgroups) */
     int query_lds_hits;         /* longest hit list a query wavefront sorts in LDS,
                                    multiple of 16 in 16..4096; longer lists use global
                                    scratch (0 = 512) */
