@@ -246,7 +246,7 @@ void ensure_rows(care_context* ctx, int blocks) {
 
 // Batch buffers of a call over n anchors in device batches of up to B: small
 // calls take what they need, rounded up to a power of two.  Memory costs a
-// program about 25 ms a GiB (allocated, freed and cleared by the driver).
+// program up to about 25 ms a GiB (allocated, freed and cleared by the driver).
 void ensure_batch(care_context* ctx, int B, int n) {
     int batch = 1024;
     while (batch < n && batch < B) batch *= 2;
@@ -794,7 +794,7 @@ int care_minhash_build(care_context* ctx) {
         g.tsize = 1;
         while (g.tsize < 2 * n) g.tsize <<= 1;
         // maps built together: as many as fit 128 MiB of scratch (memory
-        // costs about 25 ms a GiB, a group two waits for the device)
+        // costs up to 25 ms a GiB, a group two waits for the device)
         const u64 perMap = g.tsize * 16 + n * 12 + group_tiles(g.tsize) * 16;
         const int G = int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), (u64(128) << 20) / perMap})));
         DevBuf<u64> keys64;  // tkeys, tile sums, counters
