@@ -140,8 +140,8 @@ struct care_context {
     bool hasTables = false;
     int cap = 0;
 
-    // batch buffers
-    int batchCap = 0;
+    // batch buffers, grown by at_least: what one holds is its own `n` alone,
+    // which an allocation that failed leaves at 0
     int maxCand = 0;
     int queryCap = 0;  // hit lists sorted in LDS up to this length, longer ones in global scratch
     int queryRegMax = 0;  // hit lists sorted in registers up to this length (0 = kernel maximum)
@@ -160,12 +160,10 @@ struct care_context {
     DevBuf<CandMeta> metaA, metaB;  // a row of records per correction workgroup
     DevBuf<u8> outStatus;
     DevBuf<char> outSeq;
-    int outPitch = 0;
-    int outCap = 0;                     // anchors the output buffers hold
+    int outPitch = 0;                   // bytes a row of outSeq and candOutSeq
     std::vector<hipEvent_t> batchEv;    // 3 per device batch of a call
     DevBuf<u32> candOutIds;
     DevBuf<char> candOutSeq;
-    int candOutCap = 0;
     DevBuf<int> counters;  // [0] queue head, [1] candidate output count, [2] recorded columns,
                            // [32], [33] heavy anchors of even and odd device batches
     DevBuf<u32> heavy;     // anchors with long candidate lists, of a batch
@@ -244,31 +242,33 @@ void ensure_rows(care_context* ctx, int blocks) {
     at_least(ctx->metaB, size_t(blocks) * size_t(row_candidates(ctx)));
 }
 
+// Output buffers of `anchors` anchors and `cands` candidate results.
+void ensure_outputs(care_context* ctx, size_t anchors, size_t cands) {
+    ctx->outPitch = (ctx->rs.maxLen + 15) / 16 * 16;
+    at_least(ctx->outStatus, anchors);
+    at_least(ctx->outSeq, anchors * size_t(ctx->outPitch));
+    at_least(ctx->candOutIds, cands);
+    at_least(ctx->candOutSeq, cands * size_t(ctx->outPitch));
+}
+
 // Batch buffers of a call over n anchors in device batches of up to B: small
 // calls take what they need, rounded up to a power of two.  Memory costs a
 // program up to about 25 ms a GiB (allocated, freed and cleared by the driver).
-void ensure_batch(care_context* ctx, int B, int n) {
+// Returns the candidate results that the output buffers hold at least.
+int ensure_batch(care_context* ctx, int B, int n) {
     int batch = 1024;
     while (batch < n && batch < B) batch *= 2;
     batch = std::min(batch, B);
     at_least(ctx->spill, size_t(query_spill_rows(batch)) * query_spill_words(ctx->maxCand));
     at_least(ctx->candIds, size_t(batch) * size_t(row_candidates(ctx)));
-    if (batch <= ctx->batchCap) return;
-    ctx->candCount.alloc(batch);
-    ctx->rawCount.alloc(batch);
-    ctx->heavy.alloc(batch);
-    ctx->outStatus.alloc(batch);
-    ctx->outPitch = (ctx->rs.maxLen + 15) / 16 * 16;
-    ctx->outSeq.alloc(size_t(batch) * ctx->outPitch);
-    ctx->outCap = batch;
-    if (ctx->opt.correct_candidates) {
-        // every HQ anchor corrects at most its candidates within the window;
-        // a generous average bound, checked per batch
-        ctx->candOutCap = int(std::min<size_t>(size_t(batch) * 64, size_t(1) << 26));
-        ctx->candOutIds.alloc(ctx->candOutCap);
-        ctx->candOutSeq.alloc(size_t(ctx->candOutCap) * ctx->outPitch);
-    }
-    ctx->batchCap = batch;
+    at_least(ctx->candCount, size_t(batch));
+    at_least(ctx->rawCount, size_t(batch));
+    at_least(ctx->heavy, size_t(batch));
+    // every HQ anchor corrects at most its candidates within the window;
+    // a generous average bound, checked per batch
+    const int cands = ctx->opt.correct_candidates ? int(std::min<size_t>(size_t(batch) * 64, size_t(1) << 26)) : 0;
+    ensure_outputs(ctx, size_t(batch), size_t(cands));
+    return cands;
 }
 
 // Anchors per device batch of a call over n (0: any): the candidate lists get
@@ -556,7 +556,6 @@ int care_readstore_upload(care_context* ctx, uint64_t num_reads, int max_length,
     ctx->rs.maxLen = max_length;
     ctx->hasReads = true;
     ctx->hasTables = false;
-    ctx->batchCap = 0;
     return CARE_OK;
 }
 
@@ -964,7 +963,6 @@ int care_minhash_import(care_context* ctx, const care_map_view* maps, int num_ma
         ctx->opt.num_hash_maps = num_maps;
         ctx->cap = results_per_map;
         ctx->maxCand = num_maps * results_per_map;
-        ctx->batchCap = 0;  // rows of candIds hold maxCand ids
         ctx->queryCap = std::min((ctx->maxCand + 15) / 16 * 16, kDefaultQueryCap);
         ctx->queryRegMax = 0;
         ctx->sigs.alloc(n * num_maps);
@@ -1265,13 +1263,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         P.candCount = ctx->candCount.p;
         P.metaA = ctx->metaA.p;
         P.metaB = ctx->metaB.p;
-        P.outStatus = ctx->outStatus.p;
-        P.outSeq = ctx->outSeq.p;
-        P.outPitch = ctx->outPitch;
-        P.candOutIds = ctx->candOutIds.p;
-        P.candOutSeq = ctx->candOutSeq.p;
         P.candOutCount = ctx->counters.p + 1;
-        P.candOutCap = ctx->candOutCap;
         P.queueHead = ctx->counters.p;
         P.heavyList = ctx->heavy.p;
         P.heavyMin = heavy_min(ctx);
@@ -1282,17 +1274,11 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         // at the end.  Candidate results come in no particular order: the
         // per-read combination of results does not depend on it.
         const int nBatches = (n + B - 1) / B + 1;  // at most, with the short final batch
-        if (n > ctx->outCap) {
-            ctx->outStatus.alloc(size_t(n));
-            ctx->outSeq.alloc(size_t(n) * ctx->outPitch);
-            ctx->outCap = n;
-        }
         const int candCap = o.correct_candidates ? std::max(0, r->candidate_capacity) : 0;
-        if (candCap > ctx->candOutCap) {
-            ctx->candOutIds.alloc(size_t(candCap));
-            ctx->candOutSeq.alloc(size_t(candCap) * ctx->outPitch);
-            ctx->candOutCap = candCap;
-        }
+        ensure_outputs(ctx, size_t(n), size_t(candCap));
+        P.outStatus = ctx->outStatus.p;
+        P.outSeq = ctx->outSeq.p;
+        P.outPitch = ctx->outPitch;
         P.candOutIds = ctx->candOutIds.p;
         P.candOutSeq = ctx->candOutSeq.p;
         P.candOutCap = candCap;  // results beyond are dropped and reported below
@@ -1960,7 +1946,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         const int B = default_batch(ctx, n);
         n = std::min(n, std::min(B, 65536)) & ~1;
         if (n == 0) n = 2 > int(ctx->rs.n - first) ? 1 : 2;
-        ensure_batch(ctx, B, n);
+        const int candCap = ensure_batch(ctx, B, n);
         hipStream_t s = ctx->stream;
         const int candLimit = o.candidate_limit;
         auto timed = [&](auto&& launch) {
@@ -2023,7 +2009,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         P.candOutIds = ctx->candOutIds.p;
         P.candOutSeq = ctx->candOutSeq.p;
         P.candOutCount = ctx->counters.p + 1;
-        P.candOutCap = ctx->candOutCap;
+        P.candOutCap = candCap;
         P.queueHead = ctx->counters.p;
         P.firstAnchor = first;
         P.numAnchors = n;

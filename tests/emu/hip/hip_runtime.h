@@ -587,17 +587,53 @@ inline hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* nb, K, int, 
     *nb = int(byLds < 8 ? (byLds ? byLds : 1) : 8);
     return hipSuccess;
 }
+// Device memory: live bytes, and the most that lived at once since the last
+// care_emu_memory call.  care_emu_fail_alloc(k) makes the k-th allocation from
+// now on fail (0: none).
+namespace emu {
+struct Memory {
+    std::mutex m;
+    std::map<void*, size_t> allocs;
+    size_t live = 0, peak = 0;
+    int failIn = 0;
+};
+inline Memory& memory() {
+    static Memory* s = new Memory;  // outlives every context
+    return *s;
+}
+}  // namespace emu
+extern "C" __attribute__((used)) inline void care_emu_fail_alloc(int k) { emu::memory().failIn = k; }
+extern "C" __attribute__((used)) inline int care_emu_fail_pending() { return emu::memory().failIn; }
+extern "C" __attribute__((used)) inline void care_emu_memory(unsigned long long* live, unsigned long long* peak) {
+    std::lock_guard<std::mutex> g(emu::memory().m);
+    *live = emu::memory().live;
+    *peak = emu::memory().peak;
+    emu::memory().peak = emu::memory().live;
+}
 // device allocations are 256-byte aligned, as on the device
 template <class T>
 inline hipError_t hipMalloc(T** p, size_t bytes) {
+    emu::Memory& mem = emu::memory();
+    std::lock_guard<std::mutex> g(mem.m);
+    if (mem.failIn && --mem.failIn == 0) return hipErrorInvalidValue;
     const size_t n = (bytes + 255) / 256 * 256 + 256 * (bytes == 0);
     void* v = std::aligned_alloc(256, n);
     if (!v) return hipErrorInvalidValue;
     std::memset(v, emu::poison_byte() >= 0 ? emu::poison_byte() : 0, n);
     *p = static_cast<T*>(v);
+    mem.allocs[v] = bytes;
+    mem.live += bytes;
+    if (mem.live > mem.peak) mem.peak = mem.live;
     return hipSuccess;
 }
 inline hipError_t hipFree(void* p) {
+    emu::Memory& mem = emu::memory();
+    std::lock_guard<std::mutex> g(mem.m);
+    auto it = mem.allocs.find(p);
+    if (it != mem.allocs.end()) {
+        mem.live -= it->second;
+        mem.allocs.erase(it);
+    }
     std::free(p);
     return hipSuccess;
 }

@@ -1,0 +1,76 @@
+"""Device memory of a context: what a call leaves after a failed allocation.
+
+CPU through the HIP emulation, which can make the k-th allocation fail and
+counts live bytes (tests/emu/hip/hip_runtime.h).
+"""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import care_amd
+from tests import helpers
+
+EMU_DIR = os.path.join(helpers.ROOT, "tests", "emu")
+
+
+@pytest.fixture(scope="module")
+def emu():
+    subprocess.run(["sh", os.path.join(EMU_DIR, "build_emu.sh")], check=True)
+    return care_amd._bind(ctypes.CDLL(os.path.join(EMU_DIR, "_build", "libcare_amd_emu.so")), care_amd.ENGINE_SYMBOLS)
+
+
+@pytest.fixture(scope="module")
+def reads(tmp_path_factory):
+    d = str(tmp_path_factory.mktemp("reads"))
+    path, _ = helpers.simulate({"profile": "repeat-pe", "seed": 401, "genome": 2200, "sim_args": ["--length", "60"]}, d)
+    rs = care_amd.ReadSet([path], paired_end=True, qual_bits=0)
+    yield rs
+    rs.close()
+
+
+def _engine(lib, rs, **options):
+    opt = care_amd.default_options(kmer_length=20, num_hash_maps=2, coverage=30.0, paired_end=1, min_overlap=20, **options)
+    eng = care_amd.Engine(opt, device=0, lib=lib)
+    eng.upload_readset(rs)
+    eng.build()
+    return eng
+
+
+def _results(eng, n):
+    """Everything a call returns for the first n reads, candidates in a fixed order."""
+    status, seqs, cids, cseqs = eng.correct(0, n, candidate_capacity=32 * n)
+    ids, offs = eng.query(0, n)
+    width = eng.max_length
+    cands = sorted((int(i), bytes(r[:width])) for i, r in zip(cids, cseqs))
+    return status.tobytes(), seqs[(status & 1) != 0, :width].tobytes(), cands, ids.tobytes(), offs.tobytes()
+
+
+@pytest.mark.parametrize("call,most", [("correct", 99), ("query", 99), ("autotune", 8)])
+def test_small_call_after_a_failed_growth(emu, reads, call, most):
+    """A call needs larger buffers, one of their allocations fails (each in
+    turn, at most `most`); a small call that the old buffers served still
+    gives its results."""
+    assert reads.n > 1024
+    big = reads.n & ~1
+    calls = {"correct": lambda e: e.correct(0, big, candidate_capacity=1 << 18),
+             "query": lambda e: e.query(0, big), "autotune": lambda e: e.autotune(0, big)}
+    with _engine(emu, reads, correct_candidates=1) as eng:
+        want = _results(eng, 2)
+    failures = 0
+    while failures < most:
+        with _engine(emu, reads, correct_candidates=1) as eng:
+            assert _results(eng, 2) == want
+            emu.care_emu_fail_alloc(failures + 1)
+            try:
+                calls[call](eng)
+                assert emu.care_emu_fail_pending() > 0
+                break
+            except care_amd.CareError:
+                failures += 1
+            finally:
+                emu.care_emu_fail_alloc(0)
+            assert _results(eng, 2) == want, failures
+    assert failures >= 3
