@@ -92,7 +92,7 @@ struct Lds {
     int* origCov;
     u16* cnt;       // [4][cols]
     float* wgt;     // [4][cols]
-    int* scratch;   // [32]
+    int* scratch;   // [32], of which 20 are used
     u32* differ;    // [pitch] anchor bases some candidate disagrees with (build_msa)
     float* qbin;    // [4] weights of the quality bins
     u16* clist;     // [cols] columns whose weights are summed (build_msa)
@@ -100,6 +100,13 @@ struct Lds {
     u8* gacc;       // gated mode: accepted flag per anchor position [maxLen]
     char* gscr;     // gated mode: feature tile and MLP scratch, overlays mst/rows/qrows
 };  // MSA columns (cons .. wgt) are those within reach of the anchor, from the first of them
+// The planes of the alignment (arp, cpl) and the arrays of the MSA are not in
+// use at the same time.  Where all of them together pass kMaxLdsBytes
+// (LdsDims::compact: a large msa_chunk, or candidate correction of long reads
+// with new columns of about a read's length), arp lies in coverage and
+// origCov, differ and clist in cpl, qbin behind scratch.  Not otherwise: laid
+// out so, 1M reads of 150 bases took 39.4 ms against 37.9, 40,006 of 300 bases
+// 2.70 against 2.51.
 
 // MSA columns read beyond the anchor's: candidate correction reaches
 // new_columns past it, gate features two columns past a corrected read, the
@@ -109,7 +116,7 @@ __host__ __device__ inline int msa_margin(bool gated, int correctCandidates, int
 }
 
 struct LdsDims {
-    int pitch, qpitch, hw, maxLen, cols, waves, chunk, gated;
+    int pitch, qpitch, hw, maxLen, cols, waves, chunk, gated, compact;
     // threads as (row, word) pairs of rows of pitch, qpitch and pw words:
     // rows the workgroup covers at once, and 65536 / words rounded up (the
     // quotient t / words is t * inverse >> 16 for t < 1024, words <= 64)
@@ -119,16 +126,19 @@ struct LdsDims {
         size_t b = 0;
         b += size_t(chunk) * (sizeof(CandMeta) + sizeof(u32) * (pitch + qpitch));
         b += sizeof(float) * 256;
-        b += sizeof(u32) * 2 * pitch;  // aw, differ
-        b += sizeof(float) * 4;
-        b += 2 * sizeof(uint2) * pw();
+        b += sizeof(u32) * pitch;
+        b += sizeof(uint2) * pw();
         b += (size_t(maxLen) + 3) / 4 * 4;
         b += size_t(chunk) * 2 * sizeof(uint2) * pw();
         b += (size_t(cols) + 3) / 4 * 4;
         b += (sizeof(float) * size_t(cols) + 15) / 16 * 16 + sizeof(int) * (2 * size_t(cols) + 1);
         b += 4 * sizeof(u16) * cols + 4 * sizeof(float) * cols;
-        b += (sizeof(u16) * size_t(cols) + 3) / 4 * 4;
-        b += 32 * sizeof(int);
+        if (compact) {
+            b += (20 + 4) * sizeof(int);
+        } else {
+            b += 32 * sizeof(int) + 4 * sizeof(float) + sizeof(uint2) * pw();  // scratch, qbin, arp
+            b += sizeof(u32) * pitch + (sizeof(u16) * size_t(cols) + 3) / 4 * 4;  // differ, clist
+        }
         b += 2 * sizeof(u32) * size_t(chunk);
         b += 2 * sizeof(u32) * size_t(kSurvivors) * size_t(waves);  // survivor slices after the keys
         if (gated & 1) b += (sizeof(u16) + 1) * ((size_t(maxLen) + 15) / 16 * 16);
@@ -143,25 +153,33 @@ __device__ Lds carve(char* base, const LdsDims& d) {
     l.support = reinterpret_cast<float*>(p); p += (sizeof(float) * size_t(d.cols) + 15) / 16 * 16;
     l.mst = reinterpret_cast<CandMeta*>(p); p += sizeof(CandMeta) * d.chunk;
     l.ap = reinterpret_cast<uint2*>(p); p += sizeof(uint2) * d.pw();
-    l.arp = reinterpret_cast<uint2*>(p); p += sizeof(uint2) * d.pw();
+    l.arp = reinterpret_cast<uint2*>(p); p += d.compact ? 0 : sizeof(uint2) * d.pw();
     l.cpl = reinterpret_cast<uint2*>(p); p += size_t(d.chunk) * 2 * sizeof(uint2) * d.pw();
     l.rows = reinterpret_cast<u32*>(p); p += sizeof(u32) * size_t(d.chunk) * d.pitch;
     l.qrows = reinterpret_cast<u32*>(p); p += sizeof(u32) * size_t(d.chunk) * d.qpitch;
     l.qw = reinterpret_cast<float*>(p); p += sizeof(float) * 256;
     l.aw = reinterpret_cast<u32*>(p); p += sizeof(u32) * d.pitch;
-    l.differ = reinterpret_cast<u32*>(p); p += sizeof(u32) * d.pitch;
-    l.qbin = reinterpret_cast<float*>(p); p += sizeof(float) * 4;
+    l.differ = reinterpret_cast<u32*>(p); p += d.compact ? 0 : sizeof(u32) * d.pitch;
+    l.qbin = reinterpret_cast<float*>(p); p += d.compact ? 0 : sizeof(float) * 4;
     l.coverage = reinterpret_cast<int*>(p); p += sizeof(int) * (d.cols + 1);
     l.origCov = reinterpret_cast<int*>(p); p += sizeof(int) * d.cols;
     l.wgt = reinterpret_cast<float*>(p); p += 4 * sizeof(float) * d.cols;
-    l.scratch = reinterpret_cast<int*>(p); p += 32 * sizeof(int);
+    l.scratch = reinterpret_cast<int*>(p); p += (d.compact ? 20 + 4 : 32) * sizeof(int);
     l.cnt = reinterpret_cast<u16*>(p); p += 4 * sizeof(u16) * d.cols;
-    l.clist = reinterpret_cast<u16*>(p); p += (sizeof(u16) * size_t(d.cols) + 3) / 4 * 4;
+    l.clist = reinterpret_cast<u16*>(p); p += d.compact ? 0 : (sizeof(u16) * size_t(d.cols) + 3) / 4 * 4;
     l.cons = reinterpret_cast<u8*>(p); p += (size_t(d.cols) + 3) / 4 * 4;
     l.anchorQ = reinterpret_cast<char*>(p); p += (size_t(d.maxLen) + 3) / 4 * 4;
     l.keys = reinterpret_cast<u32*>(p); p += 2 * sizeof(u32) * size_t(d.chunk);
     p += 2 * sizeof(u32) * size_t(kSurvivors) * size_t(d.waves);  // survivor slices
     l.gscr = reinterpret_cast<char*>(l.mst);
+    if (d.compact) {
+        l.arp = reinterpret_cast<uint2*>(l.coverage + (reinterpret_cast<uintptr_t>(l.coverage) / 4 & 1));
+        l.differ = reinterpret_cast<u32*>(l.cpl);
+        l.clist = reinterpret_cast<u16*>(l.differ + d.pitch);
+        l.qbin = reinterpret_cast<float*>(l.scratch + 20);
+        CARE_CHECK(l.arp + d.pw() <= reinterpret_cast<uint2*>(l.origCov + d.cols));
+        CARE_CHECK(l.clist + d.cols <= reinterpret_cast<u16*>(l.rows));
+    }
     if (d.gated & 1) {
         const size_t ml = (size_t(d.maxLen) + 15) / 16 * 16;
         l.dec = reinterpret_cast<u16*>(p); p += sizeof(u16) * ml;
@@ -1669,6 +1687,7 @@ static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, in
     // LDS per staged candidate: record, 2-bit and quality rows, bit planes
     const int rowBytes = int(sizeof(CandMeta)) + 4 * (d.pitch + d.qpitch) + 2 * int(sizeof(uint2)) * d.pw();
     d.gated = gated;
+    d.compact = 0;
     d.chunk = 0;
     if (chunk > 0) {
         d.chunk = chunk;
@@ -1696,6 +1715,7 @@ static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, in
         if (gated & 2) need = std::max(need, d.waves * cand_gate_scratch(maxLen));
         while (d.chunk * rowBytes < need) d.chunk++;
     }
+    d.compact = d.bytes() > size_t(kMaxLdsBytes);
     return d;
 }
 
@@ -1705,16 +1725,17 @@ size_t correct_lds_bytes(int maxLen, int useQuality, int qpitch, int threads, in
                      msa_margin((gated & 1) != 0, correctCandidates, newColumns)).bytes();
 }
 
-// A launch shape is accepted for a read length if its staging area and 37
-// bytes for each of 3 maxLen + 2 columns (an MSA of candidates that reach a
-// whole read past both ends of the anchor) stay within kMaxLdsBytes.  The
-// kernel itself needs less, see make_dims.
+// A launch shape is accepted for a read length if this many bytes stay within
+// kMaxLdsBytes: its staging area, two of the gate's feature tiles and 37 bytes
+// for each of 3 maxLen + 2 columns (an MSA of candidates that reach a whole
+// read past both ends of the anchor).  What the kernel is launched with
+// (make_dims) is never more.
 size_t correct_capacity_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk) {
     const LdsDims d = make_dims(maxLen, useQuality, qpitch, threads, 0, 16, 0);
     const size_t cols = 3 * size_t(maxLen) + 2;
     const size_t row = sizeof(CandMeta) + sizeof(u32) * (d.pitch + d.qpitch) + 2 * sizeof(uint2) * d.pw();
     size_t c = chunk > 0 ? size_t(chunk) : std::max<size_t>(16, std::min<size_t>(256, 16384 / row));
-    size_t need = gated & 1 ? 14592 : 0;
+    size_t need = gated & 1 ? 2 * kCandGateTile : 0;
     if (gated & 2) need = std::max<size_t>(need, size_t(d.waves) * cand_gate_scratch(maxLen));
     while (c * row < need) c++;
     size_t b = c * (row + 8);
