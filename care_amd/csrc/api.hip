@@ -1141,7 +1141,7 @@ int prepare_params(care_context* ctx, CorrectParams& P) {
     P.pairedEnd = o.paired_end;
     P.useQuality = o.use_quality;
     P.correctCandidates = o.correct_candidates;
-    P.newColumns = o.new_columns_to_correct;
+    P.newColumns = std::min(std::max(o.new_columns_to_correct, -kMaxNewColumns), kMaxNewColumns);
     P.minOverlap = o.min_overlap;
     P.maxErrorRate = o.max_mismatch_ratio;
     P.minOverlapRatio = o.min_overlap_ratio;

@@ -112,7 +112,7 @@ struct Lds {
 // new_columns past it, gate features two columns past a corrected read, the
 // plain and forest decisions none
 __host__ __device__ inline int msa_margin(bool gated, int correctCandidates, int newColumns) {
-    return correctCandidates ? max(0, newColumns) + 2 : gated ? 2 : 0;
+    return correctCandidates ? max(0, min(newColumns, kMaxNewColumns)) + 2 : gated ? 2 : 0;
 }
 
 struct LdsDims {

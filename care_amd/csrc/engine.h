@@ -16,6 +16,9 @@ using u64 = std::uint64_t;
 constexpr u64 kEmptyKey = ~u64(0);
 // dynamic LDS a kernel of the engine may request per workgroup
 constexpr int kMaxLdsBytes = 64 * 1024;
+// new_columns_to_correct is cut to this: reads have at most 1,000 bases, so
+// more columns change no result
+constexpr int kMaxNewColumns = 1000;
 // default longest hit list a query wavefront merges in LDS
 constexpr int kDefaultQueryCap = 512;
 

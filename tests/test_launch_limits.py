@@ -105,3 +105,25 @@ def test_emulated_compact_layout(emu, length, bits, threads, tmp_path):
 def test_gpu_compact_layout(length, bits, threads, tmp_path):
     print("compact layout", length, bits, threads, flush=True)
     _compact_like_default(None, care_amd.engine(), str(tmp_path), length, bits, threads, 60000)
+
+
+@pytest.mark.parametrize("columns", [1 << 20, 1 << 30, (1 << 31) - 1, -(1 << 31)])
+def test_emulated_any_number_of_new_columns(emu, columns, tmp_path):
+    """Beyond the longest read more (or fewer) new columns change nothing."""
+    reads, _ = helpers.simulate({"profile": "repeat-pe", "seed": 405, "genome": 1500,
+                                 "sim_args": ["--length", "100"]}, str(tmp_path))
+    rs = care_amd.ReadSet([reads], paired_end=True, qual_bits=0)
+    results = []
+    for new in (1000 if columns > 0 else -1000, columns):
+        opt = care_amd.default_options(kmer_length=20, num_hash_maps=8, coverage=30.0, paired_end=1,
+                                       correct_candidates=1, new_columns_to_correct=new)
+        with care_amd.Engine(opt, device=0, lib=emu) as eng:
+            eng.upload_readset(rs)
+            eng.build()
+            status, seqs, cids, cseqs = eng.correct(0, rs.n, candidate_capacity=64 * rs.n)
+            corrected = (status & 1) != 0
+            assert corrected.any() and (len(cids) > 0) == (columns > 0)
+            rows = sorted((int(i), bytes(r[:rs.lengths[i]])) for i, r in zip(cids, cseqs))
+            results.append((status.tobytes(), seqs[corrected, :100].tobytes(), rows))
+    assert results[0] == results[1]
+    rs.close()
