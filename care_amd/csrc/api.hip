@@ -470,7 +470,7 @@ int care_get_tuning(care_context* ctx, care_tuning* out) {
     out->batch_anchors = ctx->rs.n ? default_batch(ctx, 0) : ctx->requestedBatch;
     out->correct_threads = T;
     out->msa_chunk = correct_msa_chunk(ctx->rs.maxLen ? ctx->rs.maxLen : 1, o.use_quality, ctx->rs.qpitch, T, gatedK,
-                                       ctx->msaChunk);
+                                       ctx->msaChunk, o.correct_candidates, o.new_columns_to_correct);
     out->query_lds_hits = ctx->queryCap;
     // the query kernel sorts up to 1024 hits in registers, 2048 when lists can be longer
     const int regLimit = ctx->maxCand > 1024 ? 2048 : 1024;
@@ -2017,7 +2017,8 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         int bestT = ctx->blockThreads, bestChunk = ctx->msaChunk;
         float bestC = 1e30f;
         for (int T : {256, 192, 128}) {
-            const int autoChunk = correct_msa_chunk(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, 0);
+            const int autoChunk = correct_msa_chunk(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, 0,
+                                                    o.correct_candidates, o.new_columns_to_correct);
             for (int chunk : {0, autoChunk / 2}) {
                 if (chunk != 0 && (chunk < 16 || chunk == autoChunk)) continue;
                 if (correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, chunk) >

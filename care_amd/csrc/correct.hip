@@ -1745,8 +1745,10 @@ size_t correct_capacity_bytes(int maxLen, int useQuality, int qpitch, int thread
     return b;
 }
 
-int correct_msa_chunk(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk) {
-    return make_dims(maxLen, useQuality, qpitch, threads, gated, chunk, 0).chunk;
+int correct_msa_chunk(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk,
+                      int correctCandidates, int newColumns) {
+    return make_dims(maxLen, useQuality, qpitch, threads, gated, chunk,
+                     msa_margin((gated & 1) != 0, correctCandidates, newColumns)).chunk;
 }
 
 int correct_resident_blocks(int threads, size_t ldsBytes, int gated) {

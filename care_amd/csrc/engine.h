@@ -251,7 +251,8 @@ void launch_correct(const CorrectParams& p, int blocks, int threads, int chunk, 
 size_t correct_lds_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk,
                          int correctCandidates, int newColumns);
 size_t correct_capacity_bytes(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk);
-int correct_msa_chunk(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk);
+int correct_msa_chunk(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk,
+                      int correctCandidates, int newColumns);
 // correction workgroups resident per compute unit at once (occupancy)
 int correct_resident_blocks(int threads, size_t ldsBytes, int gated);
 int query_lds_bytes(int h, int cap, int maxLen, int threads, int candLimit, int capL);

@@ -7,6 +7,7 @@ import ctypes
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 import care_amd
@@ -127,3 +128,21 @@ def test_emulated_any_number_of_new_columns(emu, columns, tmp_path):
             results.append((status.tobytes(), seqs[corrected, :100].tobytes(), rows))
     assert results[0] == results[1]
     rs.close()
+
+
+@pytest.mark.parametrize("gated,candidates", MODES)
+@pytest.mark.parametrize("length,bits", [(100, 0), (150, 2), (250, 8)])
+def test_reported_chunk_is_the_launched_one(emu, length, bits, gated, candidates):
+    """The staging area that care_get_tuning reports, set by hand, takes the
+    LDS of the automatic one."""
+    opt = care_amd.default_options(kmer_length=20, num_hash_maps=4, coverage=30.0, use_quality=int(bits > 0),
+                                   correct_candidates=candidates, correction_type=3 if gated else 0,
+                                   correction_type_cands=3 if gated & 2 else 0)
+    qpitch = (bits * length + 31) // 32
+    with care_amd.Engine(opt, device=0, lib=emu) as eng:
+        eng.upload(np.zeros((2, (length + 15) // 16), np.uint32), np.full(2, length, np.int32), None,
+                   np.zeros((2, qpitch), np.uint32) if bits else None, bits or 8, length)
+        t = eng.tuning()
+    lds = _function(emu, "correct_lds_bytes", 8)
+    args = (length, int(bits > 0), qpitch, t["correct_threads"], gated)
+    assert lds(*args, t["msa_chunk"], candidates, 15) == lds(*args, 0, candidates, 15)
