@@ -149,6 +149,7 @@ struct care_context {
     int blocksPerCU = 0;     // persistent correction workgroups per CU (0 = resident maximum)
     int msaChunk = 0;        // candidates per MSA staging pass (0 = automatic)
     int requestedBatch = 0;
+    care_tuning reported{};  // what care_get_tuning last gave for each field while it was automatic
     DevBuf<u32> candIds;
     DevBuf<int> candCount;
     DevBuf<int> rawCount;  // table hits per anchor of a batch (statistics)
@@ -437,8 +438,17 @@ int care_set_launch_config(care_context* ctx, int batch_anchors, int block_threa
     return CARE_OK;
 }
 
-int care_set_tuning(care_context* ctx, const care_tuning* t) {
-    if (!ctx || !t) return fail(CARE_ERR_ARGUMENT, "null argument");
+int care_set_tuning(care_context* ctx, const care_tuning* tuning) {
+    if (!ctx || !tuning) return fail(CARE_ERR_ARGUMENT, "null argument");
+    // the automatic shapes differ between small and large calls, so a value
+    // that stands for them is not a shape to pin
+    const care_tuning& seen = ctx->reported;
+    care_tuning asked = *tuning;
+    care_tuning* t = &asked;
+    if (t->batch_anchors == seen.batch_anchors) t->batch_anchors = 0;
+    if (t->correct_threads == seen.correct_threads) t->correct_threads = 0;
+    if (t->correct_blocks_per_cu == seen.correct_blocks_per_cu) t->correct_blocks_per_cu = 0;
+    if (t->msa_chunk == seen.msa_chunk) t->msa_chunk = 0;
     if (t->batch_anchors < 0 || (t->batch_anchors & 1)) return fail(CARE_ERR_ARGUMENT, "batch_anchors must be even and >= 0");
     if (t->correct_threads != 0 && t->correct_threads != 128 && t->correct_threads != 192 && t->correct_threads != 256)
         return fail(CARE_ERR_ARGUMENT, "correct_threads must be 128, 192 or 256");
@@ -486,6 +496,10 @@ int care_get_tuning(care_context* ctx, care_tuning* out) {
             return fail(CARE_ERR_DEVICE, "%s: %s", e.what, hipGetErrorString(e.err));
         }
     }
+    if (!ctx->requestedBatch) ctx->reported.batch_anchors = out->batch_anchors;
+    if (!ctx->blockThreads) ctx->reported.correct_threads = out->correct_threads;
+    if (!ctx->blocksPerCU) ctx->reported.correct_blocks_per_cu = out->correct_blocks_per_cu;
+    if (!ctx->msaChunk) ctx->reported.msa_chunk = out->msa_chunk;
     return CARE_OK;
 }
 

@@ -277,7 +277,7 @@ typedef struct care_tuning {
     int correct_threads;        /* threads per correction workgroup, i.e. 2, 3 or 4
                                    wavefronts per anchor: 128, 192 or 256
                                    (0 = automatic: 128 on large calls, 256 on
-                                   small ones; reported as for a large call) */
+                                   small ones) */
     int correct_blocks_per_cu;  /* persistent correction workgroups per compute unit
                                    (0 = as many as are resident at once) */
     int msa_chunk;              /* candidates staged in LDS per MSA pass, 16..256
@@ -294,8 +294,11 @@ typedef struct care_tuning {
                                    registers), above it the 32-per-lane one */
 } care_tuning;
 
+/* A value that care_get_tuning reported for an automatic field leaves the
+ * field automatic, so setting what was reported changes nothing;
+ * care_set_launch_config pins a batch or workgroup size whatever its value. */
 int care_set_tuning(care_context* ctx, const care_tuning* tuning);
-/* Current shapes with automatic values resolved. */
+/* Current shapes with automatic values resolved, as for a large call. */
 int care_get_tuning(care_context* ctx, care_tuning* out);
 
 /* Times candidate shapes of the query and correction kernels on anchors
