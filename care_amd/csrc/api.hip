@@ -172,7 +172,8 @@ struct care_context {
     DevBuf<float> qweights;
     PinnedBuf<int> hInts;
     // gate training and evaluation: a chunk of raw features, the bf16
-    // features of a training set, logits of an evaluation (kept between calls)
+    // features of a training set, logits of an evaluation (kept between calls,
+    // the last two up to kKeptBytes)
     DevBuf<float> mlpRaw, mlpLogits;
     DevBuf<unsigned short> mlpX;
     DevBuf<u32> mlpFlag;
@@ -1622,6 +1623,18 @@ namespace {
 // 500,000 rows), and the staging buffer stays at 32 MB.
 constexpr uint64_t kFeatureChunk = uint64_t(1) << 18;
 
+// A buffer that grows with a call's rows is given back at the end of the call
+// when it is larger than this (524,288 training rows, 8M evaluated ones): the
+// allocation it saves the next call is small beside that many rows' work.
+constexpr size_t kKeptBytes = size_t(32) << 20;
+template <class T>
+struct GiveBack {
+    DevBuf<T>& buf;
+    ~GiveBack() {
+        if (buf.n * sizeof(T) > kKeptBytes) buf.release();
+    }
+};
+
 // fn(rows of the chunk on the device, first row, rows) on every chunk, in
 // stream order; the staging buffer is reused behind the previous chunk's work
 template <class Fn>
@@ -1679,6 +1692,7 @@ int care_mlp_gradient(care_context* ctx, const float* features, const uint8_t* l
         std::vector<u32> perm(static_cast<size_t>(n));
         for (int i = 0; i < n; i++) perm[size_t(i)] = u32(i);
         DevBuf<unsigned short>& X = ctx->mlpX;
+        const GiveBack<unsigned short> giveBack{X};
         DevBuf<unsigned short> w1, w2, w3;
         DevBuf<u8> Y;
         DevBuf<u32> P;
@@ -1728,6 +1742,7 @@ int care_mlp_train(care_context* ctx, const float* features, const uint8_t* labe
         HIP_TRY(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
         DevBuf<unsigned short>& X = ctx->mlpX;
+        const GiveBack<unsigned short> giveBack{X};
         DevBuf<unsigned short> w1, w2, w3;
         DevBuf<u8> Y;
         DevBuf<u32> P;
@@ -1807,6 +1822,7 @@ int care_mlp_infer(care_context* ctx, const float* features, uint64_t n, const f
         DevBuf<unsigned short> w1, w2, w3;
         DevBuf<float> master;
         DevBuf<float>& z = ctx->mlpLogits;
+        const GiveBack<float> giveBack{z};
         master.alloc(CARE_MLP_PARAMS);
         w1.alloc(64 * 32);
         w2.alloc(32 * 64);

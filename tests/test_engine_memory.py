@@ -74,3 +74,32 @@ def test_small_call_after_a_failed_growth(emu, reads, call, most):
                 emu.care_emu_fail_alloc(0)
             assert _results(eng, 2) == want, failures
     assert failures >= 3
+
+
+def _live(lib):
+    live, peak = ctypes.c_uint64(), ctypes.c_uint64()
+    lib.care_emu_memory(ctypes.byref(live), ctypes.byref(peak))
+    return live.value
+
+
+def test_gate_buffers_are_given_back(emu):
+    """The features of a large training set do not stay on the device after
+    the call (here one that ends at a non-finite feature); what small calls
+    use stays, bounded by 32 MiB of staged features and 32 MiB of converted
+    ones."""
+    with care_amd.Engine(care_amd.default_options(), device=0, lib=emu) as eng:
+        before = _live(emu)
+        p = np.zeros(care_amd.MLP_PARAMS, np.float32)
+        x = np.zeros((1 << 20, 32), np.float32)
+        y = np.zeros(len(x), np.uint8)
+        eng.mlp_train(x[:100], y[:100], p, epochs=1, batch=16, lr=1e-3, seed=1)
+        kept = _live(emu)
+        assert kept > before
+        eng.mlp_train(x[:100], y[:100], p, epochs=1, batch=16, lr=1e-3, seed=1)
+        assert _live(emu) == kept
+        x[-1, -1] = np.inf
+        for call in (lambda: eng.mlp_train(x, y, p, epochs=1, batch=16, lr=1e-3, seed=1),
+                     lambda: eng.mlp_gradient(x, y, p)):
+            with pytest.raises(care_amd.CareError):
+                call()
+            assert _live(emu) - before <= 64 << 20
