@@ -238,10 +238,14 @@ int row_candidates(const care_context* ctx) {
     return limit > 0 ? std::min(limit, ctx->maxCand) : ctx->maxCand;
 }
 
-// Record rows of the correction workgroups.
-void ensure_rows(care_context* ctx, int blocks) {
-    at_least(ctx->metaA, size_t(blocks) * size_t(row_candidates(ctx)));
-    at_least(ctx->metaB, size_t(blocks) * size_t(row_candidates(ctx)));
+// Record rows of the correction workgroups, at most `most` of them, rounded up
+// to a power of two: calls that grow by a few anchors find their rows there.
+void ensure_rows(care_context* ctx, int blocks, int most) {
+    int rows = 1;
+    while (rows < blocks) rows *= 2;
+    rows = std::max(blocks, std::min(rows, most));
+    at_least(ctx->metaA, size_t(rows) * size_t(row_candidates(ctx)));
+    at_least(ctx->metaB, size_t(rows) * size_t(row_candidates(ctx)));
 }
 
 // Output buffers of `anchors` anchors and `cands` candidate results.
@@ -1272,7 +1276,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         const int blocksPerCU = ctx->blocksPerCU > 0 ? ctx->blocksPerCU
                                                      : correct_resident_blocks(T, lds, gatedK | (P.gatedRefine ? 4 : 0));
         hipStream_t s = ctx->stream;
-        ensure_rows(ctx, std::min(std::min(n, B), ctx->numCUs * blocksPerCU));
+        ensure_rows(ctx, std::min(std::min(n, B), ctx->numCUs * blocksPerCU), ctx->numCUs * blocksPerCU);
         P.maxCand = row_candidates(ctx);
         P.candIds = ctx->candIds.p;
         P.candCount = ctx->candCount.p;
@@ -2058,7 +2062,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
                                                      o.correct_candidates, o.new_columns_to_correct);
                 const int bpc = ctx->blocksPerCU > 0 ? ctx->blocksPerCU : correct_resident_blocks(T, lds, gatedK);
                 const int blocks = std::max(1, std::min(n, ctx->numCUs * bpc));
-                ensure_rows(ctx, blocks);
+                ensure_rows(ctx, blocks, ctx->numCUs * bpc);
                 P.metaA = ctx->metaA.p;
                 P.metaB = ctx->metaB.p;
                 const float ms = timed([&] {

@@ -103,3 +103,18 @@ def test_gate_buffers_are_given_back(emu):
             with pytest.raises(care_amd.CareError):
                 call()
             assert _live(emu) - before <= 64 << 20
+
+
+def test_growing_calls_allocate_seldom(emu, reads):
+    """Calls that grow by a pair at a time find most of their buffers there:
+    records per workgroup are not allocated again for each of them."""
+    with _engine(emu, reads) as eng:
+        eng.set_tuning(correct_blocks_per_cu=64)  # 128 workgroups
+        allocations = 0
+        for n in range(2, 131, 2):
+            emu.care_emu_fail_alloc(1 << 30)
+            eng.correct(0, n)
+            allocations += (1 << 30) - emu.care_emu_fail_pending()
+            emu.care_emu_fail_alloc(0)
+        # two buffers of records for each power of two from 2 to 128, and at most a dozen others
+        assert allocations <= 2 * 7 + 12
