@@ -157,8 +157,7 @@ struct care_context {
     DevBuf<u64> packStarts;
     DevBuf<int> packOffsets;
     DevBuf<u32> packed;
-    DevBuf<u32> spill;  // query_spill_words(maxCand) words per query wavefront
-    DevBuf<CandMeta> metaA, metaB;  // a row of records per correction workgroup
+    DevBuf<CandMeta> work;  // spill rows of the query, then records of the correction (ensure_work)
     DevBuf<u8> outStatus;
     DevBuf<char> outSeq;
     int outPitch = 0;                   // bytes a row of outSeq and candOutSeq
@@ -238,16 +237,6 @@ int row_candidates(const care_context* ctx) {
     return limit > 0 ? std::min(limit, ctx->maxCand) : ctx->maxCand;
 }
 
-// Record rows of the correction workgroups, at most `most` of them, rounded up
-// to a power of two: calls that grow by a few anchors find their rows there.
-void ensure_rows(care_context* ctx, int blocks, int most) {
-    int rows = 1;
-    while (rows < blocks) rows *= 2;
-    rows = std::max(blocks, std::min(rows, most));
-    at_least(ctx->metaA, size_t(rows) * size_t(row_candidates(ctx)));
-    at_least(ctx->metaB, size_t(rows) * size_t(row_candidates(ctx)));
-}
-
 // Output buffers of `anchors` anchors and `cands` candidate results.
 void ensure_outputs(care_context* ctx, size_t anchors, size_t cands) {
     ctx->outPitch = (ctx->rs.maxLen + 15) / 16 * 16;
@@ -257,15 +246,56 @@ void ensure_outputs(care_context* ctx, size_t anchors, size_t cands) {
     at_least(ctx->candOutSeq, cands * size_t(ctx->outPitch));
 }
 
-// Batch buffers of a call over n anchors in device batches of up to B: small
-// calls take what they need, rounded up to a power of two.  Memory costs a
-// program up to about 25 ms a GiB (allocated, freed and cleared by the driver).
+// Device memory for the batch scratch of a call: a quarter of what was free
+// when the context was created, between 2 and 24 GiB.  Half of it, at most
+// 4 GiB, is for the candidate lists, half for the work rows.  A batch size
+// that the caller set stands for its own memory: 36 bytes for each of the
+// h x cap candidates of every anchor.
+size_t batch_budget(const care_context* ctx) {
+    return std::min(std::max(ctx->freeAtCreate / 4, size_t(2) << 30), size_t(24) << 30);
+}
+
+// Work rows of `bytes` each that a call may take, of the `wanted` ones.
+int work_rows(const care_context* ctx, int wanted, size_t bytes) {
+    if (ctx->requestedBatch > 0) return wanted;
+    return int(std::min<size_t>(size_t(wanted), std::max<size_t>(64, batch_budget(ctx) / 2 / bytes)));
+}
+
+// Query wavefronts over a batch of n anchors, each with a spill row.
+int spill_rows(const care_context* ctx, int n) {
+    return work_rows(ctx, query_spill_rows(n), query_spill_words(ctx->maxCand) * sizeof(u32));
+}
+
+// Correction workgroups, each with two rows of records.
+int record_rows(const care_context* ctx, int blocks) {
+    return work_rows(ctx, blocks, 2 * sizeof(CandMeta) * size_t(row_candidates(ctx)));
+}
+
+// Scratch of a call's kernels: the spill rows of `wavefronts` query wavefronts
+// and, after them in time and in the same memory, the records of `blocks`
+// correction workgroups.  These are rounded up to a power of two, at most
+// `most`: calls that grow by a few anchors find their rows there.
+void ensure_work(care_context* ctx, int wavefronts, int blocks, int most) {
+    int rows = 1;
+    while (rows < blocks) rows *= 2;
+    rows = std::max(blocks, std::min(rows, most));
+    const size_t spill = size_t(wavefronts) * query_spill_words(ctx->maxCand);
+    at_least(ctx->work, std::max((spill * sizeof(u32) + sizeof(CandMeta) - 1) / sizeof(CandMeta),
+                                 2 * size_t(rows) * size_t(row_candidates(ctx))));
+}
+
+u32* spill_memory(const care_context* ctx) { return reinterpret_cast<u32*>(ctx->work.p); }
+
+// Batch buffers of a call over n anchors in device batches of up to B, with up
+// to `most` correction workgroups: small calls take what they need, rounded
+// up to a power of two.  Memory costs a program up to about 25 ms a GiB
+// (allocated, freed and cleared by the driver).
 // Returns the candidate results that the output buffers hold at least.
-int ensure_batch(care_context* ctx, int B, int n) {
+int ensure_batch(care_context* ctx, int B, int n, int most) {
     int batch = 1024;
     while (batch < n && batch < B) batch *= 2;
     batch = std::min(batch, B);
-    at_least(ctx->spill, size_t(query_spill_rows(batch)) * query_spill_words(ctx->maxCand));
+    ensure_work(ctx, spill_rows(ctx, batch), std::min(std::min(n, B), most), most);
     at_least(ctx->candIds, size_t(batch) * size_t(row_candidates(ctx)));
     at_least(ctx->candCount, size_t(batch));
     at_least(ctx->rawCount, size_t(batch));
@@ -277,19 +307,17 @@ int ensure_batch(care_context* ctx, int B, int n) {
     return cands;
 }
 
-// Anchors per device batch of a call over n (0: any): the candidate lists get
-// a quarter of the device memory free when the context was created, between 2
-// and 4 GiB, and a batch holds at most 2^18 anchors.  Fewer, larger batches
-// mean fewer launches and fewer drains of the persistent correction kernel,
-// so batches hold at least 65,536 anchors, and an eighth of the call's: 1M
+// Anchors per device batch of a call over n (0: any): what the candidate
+// lists' share of the memory holds, at most 2^18.  Fewer, larger batches mean
+// fewer launches and fewer drains of the persistent correction kernel, so
+// batches hold at least 65,536 anchors, and an eighth of the call's: 1M
 // anchors in quarters take 2 % less kernel time and 1.2 GB (30 ms to a
 // program) more.  With a candidate limit the lists are small and a batch holds
 // a quarter.
-int default_batch(care_context* ctx, int n) {
+int default_batch(const care_context* ctx, int n) {
     if (ctx->requestedBatch > 0) return ctx->requestedBatch;
     const size_t perAnchor = size_t(row_candidates(ctx)) * sizeof(u32) + ctx->rs.maxLen + 64;
-    const size_t budget = std::min(std::max(ctx->freeAtCreate / 4, size_t(2) << 30), size_t(4) << 30);
-    size_t b = budget / perAnchor;
+    size_t b = std::min(batch_budget(ctx) / 2, size_t(4) << 30) / perAnchor;
     b = std::max<size_t>(256, std::min<size_t>(b, size_t(1) << 18));
     if (n > 0) b = std::min<size_t>(b, std::max(65536, n / (ctx->opt.candidate_limit > 0 ? 4 : 8)));
     return int(b & ~size_t(1));
@@ -763,7 +791,8 @@ int care_minhash_query_async(care_context* ctx, const uint32_t* d_seqs, int seq_
         qa.ids = d_read_ids;
         qa.lens = d_lengths;
         launch_query(ctx->rs, ctx->tables, 0, n, ctx->maxCand, ctx->queryCap, ctx->queryRegMax, o.exclude_ambiguous,
-                     o.candidate_limit, d_candidates, ctx->maxCand, d_counts, spill, nullptr, stream, qa);
+                     o.candidate_limit, d_candidates, ctx->maxCand, d_counts, spill, query_spill_rows(n), nullptr,
+                     stream, qa);
         HIP_TRY(hipGetLastError());
     } catch (const HipError& e) {
         return fail(CARE_ERR_DEVICE, "%s: %s", e.what, hipGetErrorString(e.err));
@@ -1069,14 +1098,15 @@ int care_minhash_query(care_context* ctx, uint64_t first, int n, uint32_t* ids, 
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         const int B = default_batch(ctx, n);
-        ensure_batch(ctx, B, n);
+        ensure_batch(ctx, B, n, 0);
         const int pitch = row_candidates(ctx);
         uint64_t written = 0;
         for (int done = 0; done < n; done += B) {
             const int nb = std::min(B, n - done);
             launch_query(ctx->rs, ctx->tables, first + done, nb, ctx->maxCand, ctx->queryCap, ctx->queryRegMax,
                          ctx->opt.exclude_ambiguous, ctx->opt.candidate_limit,
-                         ctx->candIds.p, pitch, ctx->candCount.p, ctx->spill.p, nullptr, ctx->stream);
+                         ctx->candIds.p, pitch, ctx->candCount.p, spill_memory(ctx), spill_rows(ctx, nb), nullptr,
+                         ctx->stream);
             HIP_TRY(hipGetLastError());
             // the lists are packed on the device, so that only their entries
             // are copied, straight into the caller's arrays (the rows of
@@ -1263,7 +1293,6 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         const int B = default_batch(ctx, n);
-        ensure_batch(ctx, B, n);
         const int T = correct_threads(ctx, std::min(n, B));
         const int gatedK = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
         const size_t need = correct_capacity_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch,
@@ -1276,12 +1305,13 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
         const int blocksPerCU = ctx->blocksPerCU > 0 ? ctx->blocksPerCU
                                                      : correct_resident_blocks(T, lds, gatedK | (P.gatedRefine ? 4 : 0));
         hipStream_t s = ctx->stream;
-        ensure_rows(ctx, std::min(std::min(n, B), ctx->numCUs * blocksPerCU), ctx->numCUs * blocksPerCU);
+        const int mostBlocks = record_rows(ctx, ctx->numCUs * blocksPerCU);
+        ensure_batch(ctx, B, n, mostBlocks);
         P.maxCand = row_candidates(ctx);
         P.candIds = ctx->candIds.p;
         P.candCount = ctx->candCount.p;
-        P.metaA = ctx->metaA.p;
-        P.metaB = ctx->metaB.p;
+        P.metaA = ctx->work.p;
+        P.metaB = P.metaA + size_t(std::min(std::min(n, B), mostBlocks)) * size_t(P.maxCand);
         P.candOutCount = ctx->counters.p + 1;
         P.queueHead = ctx->counters.p;
         P.heavyList = ctx->heavy.p;
@@ -1323,7 +1353,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
                                                "anchor_sequences (care_host_buffer_alloc)");
             key_append(key, first, n, r->anchor_status, r->anchor_sequences, r->sequence_pitch, candCap, B, T,
                        blocksPerCU, ctx->msaChunk, ctx->queryCap, ctx->queryRegMax, ctx->numCUs, ctx->outPitch, o,
-                       P, ctx->tables, ctx->rs, ctx->candIds.p, ctx->candCount.p, ctx->metaA.p, ctx->spill.p, ctx->rawCount.p,
+                       P, ctx->tables, ctx->rs, ctx->candIds.p, ctx->candCount.p, ctx->rawCount.p,
                        ctx->rawHits.p, ctx->counters.p, ctx->outStatus.p, ctx->outSeq.p);
         }
         const bool replay = graph && gc.exec && gc.key == key;
@@ -1347,7 +1377,8 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
                     int* heavyCount = ctx->counters.p + 32 + (bi & 1);
                     launch_query(ctx->rs, ctx->tables, first + done, nb, ctx->maxCand, ctx->queryCap,
                                  ctx->queryRegMax, o.exclude_ambiguous, o.candidate_limit, ctx->candIds.p,
-                                 P.maxCand, ctx->candCount.p, ctx->spill.p, ctx->rawCount.p, s,
+                                 P.maxCand, ctx->candCount.p, spill_memory(ctx), spill_rows(ctx, nb),
+                                 ctx->rawCount.p, s,
                                  QueryAnchors(), QueryHeavy{ctx->heavy.p, heavyCount, P.heavyMin});
                     launch_sum_counts(ctx->rawCount.p, ctx->candCount.p, nb, ctx->rawHits.p, ctx->counters.p,
                                       ctx->counters.p + 32 + ((bi + 1) & 1), s);
@@ -1357,7 +1388,7 @@ int correct_batch_impl(care_context* ctx, uint64_t first, int n, care_batch_resu
                     P.numAnchors = nb;
                     P.outStatus = ctx->outStatus.p + size_t(done);
                     P.outSeq = ctx->outSeq.p + size_t(done) * ctx->outPitch;
-                    const int blocks = std::max(1, std::min(nb, ctx->numCUs * blocksPerCU));
+                    const int blocks = std::max(1, std::min(nb, mostBlocks));
                     launch_correct(P, blocks, T, ctx->msaChunk, s);
                     HIP_TRY(hipGetLastError());
                     HIP_TRY(hipEventRecord(e[2], s));
@@ -1980,7 +2011,7 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         const int B = default_batch(ctx, n);
         n = std::min(n, std::min(B, 65536)) & ~1;
         if (n == 0) n = 2 > int(ctx->rs.n - first) ? 1 : 2;
-        const int candCap = ensure_batch(ctx, B, n);
+        const int candCap = ensure_batch(ctx, B, n, 0);
         hipStream_t s = ctx->stream;
         const int candLimit = o.candidate_limit;
         auto timed = [&](auto&& launch) {
@@ -1999,7 +2030,8 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         };
         auto query = [&](int capL, int regMax) {
             launch_query(ctx->rs, ctx->tables, first, n, ctx->maxCand, capL, regMax, o.exclude_ambiguous, candLimit,
-                         ctx->candIds.p, row_candidates(ctx), ctx->candCount.p, ctx->spill.p, nullptr, s);
+                         ctx->candIds.p, row_candidates(ctx), ctx->candCount.p, spill_memory(ctx), spill_rows(ctx, n),
+                         nullptr, s);
         };
         // query: LDS hit capacities up to the longest possible list and, for
         // tables whose lists can exceed 1024 hits (unless pinned by
@@ -2025,7 +2057,8 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         ctx->queryRegMax = bestReg;
         launch_reset_counters(ctx->counters.p, nullptr, ctx->counters.p + 32, nullptr, s);
         launch_query(ctx->rs, ctx->tables, first, n, ctx->maxCand, bestCap, bestReg, o.exclude_ambiguous, candLimit,
-                     ctx->candIds.p, row_candidates(ctx), ctx->candCount.p, ctx->spill.p, nullptr, s,
+                     ctx->candIds.p, row_candidates(ctx), ctx->candCount.p, spill_memory(ctx), spill_rows(ctx, n),
+                     nullptr, s,
                      QueryAnchors(), QueryHeavy{ctx->heavy.p, ctx->counters.p + 32, heavy_min(ctx)});
         HIP_TRY(hipGetLastError());
         P.heavyList = ctx->heavy.p;
@@ -2035,8 +2068,6 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
         // correction: 2, 3 or 4 wavefronts per anchor, automatic and halved MSA chunks
         P.candIds = ctx->candIds.p;
         P.candCount = ctx->candCount.p;
-        P.metaA = ctx->metaA.p;
-        P.metaB = ctx->metaB.p;
         P.outStatus = ctx->outStatus.p;
         P.outSeq = ctx->outSeq.p;
         P.outPitch = ctx->outPitch;
@@ -2061,10 +2092,11 @@ int care_autotune(care_context* ctx, uint64_t first, int n, care_tuning* chosen)
                 const size_t lds = correct_lds_bytes(ctx->rs.maxLen, o.use_quality, ctx->rs.qpitch, T, gatedK, chunk,
                                                      o.correct_candidates, o.new_columns_to_correct);
                 const int bpc = ctx->blocksPerCU > 0 ? ctx->blocksPerCU : correct_resident_blocks(T, lds, gatedK);
-                const int blocks = std::max(1, std::min(n, ctx->numCUs * bpc));
-                ensure_rows(ctx, blocks, ctx->numCUs * bpc);
-                P.metaA = ctx->metaA.p;
-                P.metaB = ctx->metaB.p;
+                const int mostBlocks = record_rows(ctx, ctx->numCUs * bpc);
+                const int blocks = std::max(1, std::min(n, mostBlocks));
+                ensure_work(ctx, spill_rows(ctx, n), blocks, mostBlocks);
+                P.metaA = ctx->work.p;
+                P.metaB = P.metaA + size_t(blocks) * size_t(P.maxCand);
                 const float ms = timed([&] {
                     launch_reset_counters(ctx->counters.p, ctx->counters.p + 1, nullptr, nullptr, s);
                     launch_correct(P, blocks, T, chunk, s);
@@ -2218,8 +2250,7 @@ extern "C" int care_correct_batch_noalloc(care_context* ctx, uint64_t first, int
             const int nb = std::min(B, n - done);
             launch_query(ctx->rs, ctx->tables, first + done, nb, ctx->maxCand, ctx->queryCap, ctx->queryRegMax,
                          o.exclude_ambiguous, o.candidate_limit, candIds, int(mc), candCount,
-                         reinterpret_cast<u32*>(metaA),
-                         nullptr, s);
+                         reinterpret_cast<u32*>(metaA), query_spill_rows(nb), nullptr, s);
             // queue head and candidate result count start at zero in every batch
             launch_reset_counters(counters, counters + 1, nullptr, nullptr, s);
             P.firstAnchor = first + done;

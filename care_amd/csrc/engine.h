@@ -219,13 +219,13 @@ struct QueryHeavy {
 };
 // candIds: a row of `pitch` ids per anchor, pitch at least maxCand or, with
 // candLimit > 0, candLimit; spill: query_spill_words(maxCand) words for each
-// of query_spill_rows(n) wavefronts (sort/merge buffers of anchors with more
+// of spillRows wavefronts, n or at least 4 (sort/merge buffers of anchors with more
 // than capL hits); regMax: longest hit list sorted in
 // registers (0 = the kernel's maximum, 1024), longer lists are merged;
 // rawCount (may be null): table hits per anchor before de-duplication
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
                   int excludeAmbiguous, int candLimit, u32* candIds, int pitch, int* candCount, u32* spill,
-                  int* rawCount, hipStream_t stream, const QueryAnchors& anchors = QueryAnchors(),
+                  int spillRows, int* rawCount, hipStream_t stream, const QueryAnchors& anchors = QueryAnchors(),
                   const QueryHeavy& heavy = QueryHeavy());
 // read-store gathers by read id into device buffers (store.hip)
 void launch_gather_sequences(const DevReadStore& rs, const u32* ids, int n, u32* out, int outPitch, hipStream_t s);

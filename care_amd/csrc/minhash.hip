@@ -933,12 +933,13 @@ int query_spill_rows(int n) { return std::min(n, 1 << 12); }
 
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
                   int excludeAmbiguous, int candLimit, u32* candIds, int pitch, int* candCount, u32* spill,
-                  int* rawCount, hipStream_t stream, const QueryAnchors& qa, const QueryHeavy& heavy) {
+                  int spillRows, int* rawCount, hipStream_t stream, const QueryAnchors& qa, const QueryHeavy& heavy) {
     if (n <= 0) return;
     const int threads = 256;
     const int wpb = threads / kWave;
     const int lds = query_lds_bytes(t.h, maxCand / t.h, rs.maxLen, threads, candLimit, capL);
-    const int blocks = (query_spill_rows(n) + wpb - 1) / wpb;
+    // (wavefronts of a last, incomplete workgroup have no anchor)
+    const int blocks = spillRows < n ? std::max(1, spillRows / wpb) : (n + wpb - 1) / wpb;
     const bool wide = maxCand > 16 * kWave;  // lists may exceed the 16-per-lane network
     const int kernelMax = wide ? 32 * kWave : 16 * kWave;
     regMax = regMax > 0 ? std::min(regMax, kernelMax) : kernelMax;

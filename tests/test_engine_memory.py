@@ -6,6 +6,7 @@ counts live bytes (tests/emu/hip/hip_runtime.h).
 import ctypes
 import os
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -118,3 +119,48 @@ def test_growing_calls_allocate_seldom(emu, reads):
             emu.care_emu_fail_alloc(0)
         # two buffers of records for each power of two from 2 to 128, and at most a dozen others
         assert allocations <= 2 * 7 + 12
+
+
+# A call with 64,000 candidate slots an anchor on a device of 256 compute units: peak memory above what was live
+# before it, and the results.  argv: emulation folder, read file, anchors per batch (0 automatic), workgroups per CU.
+WIDE = """
+import ctypes, hashlib, os, sys
+import care_amd
+lib = care_amd._bind(ctypes.CDLL(os.path.join(sys.argv[1], "_build", "libcare_amd_emu.so")), care_amd.ENGINE_SYMBOLS)
+rs = care_amd.ReadSet([sys.argv[2]], paired_end=True, qual_bits=0)
+opt = care_amd.default_options(kmer_length=20, num_hash_maps=64, coverage=400.0, paired_end=1, min_overlap=20)
+live, peak = ctypes.c_uint64(), ctypes.c_uint64()
+with care_amd.Engine(opt, device=0, lib=lib) as eng:
+    eng.upload_readset(rs)
+    eng.build()
+    eng.set_tuning(batch_anchors=int(sys.argv[3]), correct_blocks_per_cu=int(sys.argv[4]), query_lds_hits=16,
+                   query_register_hits=64)
+    lib.care_emu_memory(ctypes.byref(live), ctypes.byref(peak))
+    before = live.value
+    n = min(1024, rs.n)
+    status, seqs, _, _ = eng.correct(0, n)
+    lib.care_emu_memory(ctypes.byref(live), ctypes.byref(peak))
+    print(n, peak.value - before)
+    print(hashlib.md5(status.tobytes() + seqs[(status & 1) != 0, :eng.max_length].tobytes()).hexdigest())
+"""
+
+
+def test_batch_memory_is_bounded(tmp_path):
+    """The scratch of a call stays within a quarter of the free memory (2 GiB
+    of the emulated 8), and with a batch size set by the caller within 36
+    bytes a candidate slot; with fewer rows than anchors the results are the
+    same."""
+    subprocess.run(["sh", os.path.join(EMU_DIR, "build_emu.sh")], check=True)
+    path, _ = helpers.simulate({"profile": "repeat-pe", "seed": 402, "genome": 2200,
+                                "sim_args": ["--length", "60"]}, str(tmp_path))
+    got = []
+    for batch, per_cu in ((0, 8), (64, 8)):
+        p = subprocess.run([sys.executable, "-c", WIDE, EMU_DIR, path, str(batch), str(per_cu)],
+                           env=dict(os.environ, EMU_CUS="256", PYTHONPATH=helpers.ROOT), stdout=subprocess.PIPE,
+                           stderr=subprocess.STDOUT, text=True, timeout=600)
+        assert p.returncode == 0, p.stdout[-2000:]
+        n, took, digest = p.stdout.split()
+        outputs = int(n) * (64 + 64)  # rows of results, counters
+        assert int(took) <= (36 * 64000 * batch if batch else 2 << 30) + outputs + (1 << 20), (batch, took)
+        got.append(digest)
+    assert got[0] == got[1]

@@ -1,7 +1,7 @@
 """Setting the launch shapes that care_get_tuning reported changes nothing.
 
 Automatic shapes depend on the size of a call; what is launched is seen in
-the device memory that a call takes (records per workgroup, rows per batch).
+the device memory that a call takes (records per workgroup).
 CPU through the HIP emulation.
 """
 import os
@@ -52,7 +52,7 @@ with care_amd.Engine(opt, device=0, lib=lib) as eng:
 
 
 def _run(how):
-    env = dict(os.environ, EMU_CUS="16", PYTHONPATH=helpers.ROOT)
+    env = dict(os.environ, EMU_CUS="256", PYTHONPATH=helpers.ROOT)
     p = subprocess.run([sys.executable, "-c", SCRIPT, how, EMU_DIR], env=env, stdout=subprocess.PIPE,
                        stderr=subprocess.STDOUT, text=True, timeout=300)
     assert p.returncode == 0, p.stdout[-2000:]
