@@ -840,14 +840,14 @@ int care_minhash_build(care_context* ctx) {
         // scratch tables at load <= 0.5
         g.tsize = 1;
         while (g.tsize < 2 * n) g.tsize <<= 1;
-        // maps built together: as many as fit 128 MiB of scratch (memory
+        // maps built together: as many as fit kBuildScratch, 128 MiB (memory
         // costs up to 25 ms a GiB, a group two waits for the device)
         const u64 perMap = g.tsize * 16 + n * 12 + group_tiles(g.tsize) * 16;
-        const int G = int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), (u64(128) << 20) / perMap})));
-        DevBuf<u64> keys64;  // tkeys, tile sums, counters
-        DevBuf<u32> words;   // tcount, toff, slot, arrival, packed, overflow
-        keys64.alloc(size_t(G) * (g.tsize + 2 * group_tiles(g.tsize) + 2));
-        words.alloc(size_t(G) * (2 * g.tsize + 3 * n) + 1);
+        const int G = int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), kBuildScratch / perMap})));
+        DevBuf<u64> keys64;  // tkeys, tile sums, counters, overflow
+        DevBuf<u32> words;   // tcount, toff, slot, arrival, packed
+        keys64.alloc(size_t(G) * (g.tsize + 2 * group_tiles(g.tsize) + 2) + 1);
+        words.alloc(size_t(G) * (2 * g.tsize + 3 * n));
         PinnedBuf<unsigned long long> totals;
         totals.alloc(size_t(2) * G + 1);
         g.tkeys = keys64.p;
@@ -855,21 +855,27 @@ int care_minhash_build(care_context* ctx) {
         g.counters = reinterpret_cast<unsigned long long*>(g.tileSums + size_t(G) * 2 * group_tiles(g.tsize));
         g.tcount = words.p;
         g.toff = g.tcount + size_t(G) * g.tsize;
-        g.slot = g.toff + size_t(G) * g.tsize;
-        g.arrival = g.slot + size_t(G) * n;
+        g.slot = reinterpret_cast<BuildSlot*>(g.toff + size_t(G) * g.tsize);
+        g.arrival = g.toff + size_t(G) * (g.tsize + n);
         g.packed = g.arrival + size_t(G) * n;
-        g.overflow = reinterpret_cast<int*>(g.packed + size_t(G) * n);
         ctx->hasTables = false;
         ctx->maps.clear();
         std::vector<DevMap> hostMaps(h);
         for (int m0 = 0; m0 < h; m0 += G) {
             g.first = m0;
             g.count = std::min(G, h - m0);
+            g.overflow = reinterpret_cast<int*>(g.counters + 2 * g.count);
+            const auto overflowed = [&] {
+                if (!*reinterpret_cast<const int*>(totals.p + 2 * g.count)) return 0;
+                return fail(CARE_ERR_DEVICE, "hash table overflow while building maps %d to %d", m0,
+                            m0 + g.count - 1);
+            };
             launch_group_count(g, s);
             HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(totals.p, g.counters, size_t(2 * g.count) * sizeof(unsigned long long),
+            HIP_TRY(hipMemcpyAsync(totals.p, g.counters, size_t(2 * g.count + 1) * sizeof(unsigned long long),
                                    hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
+            if (const int rc = overflowed()) return rc;
             // one allocation for the group's tables: all keys, all ranges,
             // all values
             u64 slots = 0, values = 0;
@@ -903,10 +909,9 @@ int care_minhash_build(care_context* ctx) {
             }
             launch_group_fill(g, s);
             HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(totals.p + 2 * G, g.overflow, sizeof(int), hipMemcpyDeviceToHost, s));
+            HIP_TRY(hipMemcpyAsync(totals.p + 2 * g.count, g.overflow, sizeof(int), hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
-            if (*reinterpret_cast<const int*>(totals.p + 2 * G))
-                return fail(CARE_ERR_DEVICE, "hash table overflow while building maps %d to %d", m0, m0 + g.count - 1);
+            if (const int rc = overflowed()) return rc;
         }
         ctx->devMaps.alloc(h);
         HIP_TRY(hipMemcpy(ctx->devMaps.p, hostMaps.data(), sizeof(DevMap) * h, hipMemcpyHostToDevice));

@@ -45,6 +45,19 @@ struct DevMap {
     u64 mask;
 };
 
+// Sizes of the scratch: bytes that the maps built together may take, slots of
+// a scratch table (2^32 at most), wavefronts of a query.  CARE_SMALL_SCRATCH
+// makes them small enough for the emulated tests to reach them.
+#ifdef CARE_SMALL_SCRATCH
+constexpr u64 kBuildScratch = u64(128) << 10;
+using BuildSlot = u16;
+constexpr int kQueryWavefronts = 8;
+#else
+constexpr u64 kBuildScratch = u64(128) << 20;
+using BuildSlot = u32;
+constexpr int kQueryWavefronts = 1 << 12;
+#endif
+
 // A group of maps while they are built (minhash.hip): scratch arrays indexed
 // [map][slot] or, per read, [read][map]; `fin` holds the finished tables.
 constexpr int kMaxBuildMaps = 64;
@@ -57,12 +70,12 @@ struct MapGroup {
     u64* tkeys;   // [count][tsize]
     u32* tcount;  // [count][tsize]
     u32* toff;    // [count][tsize]
-    u32* slot;    // [n][count] scratch slot of the read's key, ~0 if the table overflowed
+    BuildSlot* slot;  // [n][count] scratch slot of the read's key (no value marks a missing one)
     u32* arrival; // [n][count] how many reads of the key came before
     u32* packed;  // [n * count] value ranges, unsorted
     u64* tileSums;
     unsigned long long* counters;  // [count][2] values, keys
-    int* overflow;
+    int* overflow;                 // in the word behind the counters
     DevMap fin[kMaxBuildMaps];
 };
 

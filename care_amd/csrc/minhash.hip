@@ -159,11 +159,10 @@ __global__ void k_count_keys(MapGroup g) {
         const int m = int(i - r * u32(g.count));
         const u64 slot = find_or_insert(g.tkeys + u64(m) * g.tsize, g.tsize - 1, g.sigs[r * g.h + g.first + m]);
         if (slot == ~u64(0)) {
-            atomicExch(g.overflow, 1);
-            g.slot[i] = ~0u;
+            atomicExch(g.overflow, 1);  // the host goes no further
             continue;
         }
-        g.slot[i] = u32(slot);
+        g.slot[i] = BuildSlot(slot);
         g.arrival[i] = atomicAdd(&g.tcount[u64(m) * g.tsize + slot], 1u);
     }
 }
@@ -297,7 +296,6 @@ __global__ void k_scatter_values(MapGroup g) {
         const u64 r = i / u32(g.count);
         const int m = int(i - r * u32(g.count));
         const u32 slot = g.slot[i];
-        if (slot == ~0u) continue;
         const u32 off = g.toff[u64(m) * g.tsize + slot];
         if (off == 0xFFFFFFFFu) continue;
         g.packed[u64(m) * g.n + off + g.arrival[i]] = u32(r);
@@ -314,7 +312,6 @@ __global__ void k_rank_values(MapGroup g) {
         const u64 r = i / u32(g.count);
         const int m = int(i - r * u32(g.count));
         const u32 slot = g.slot[i];
-        if (slot == ~0u) continue;
         const u32 off = g.toff[u64(m) * g.tsize + slot];
         if (off == 0xFFFFFFFFu) continue;
         const int c = int(g.tcount[u64(m) * g.tsize + slot]);
@@ -371,7 +368,7 @@ void launch_fill_u32(u32* p, u64 n, u32 v, hipStream_t s) {
 u64 group_tiles(u64 tsize) { return (tsize + kTile - 1) / kTile; }
 
 // keys counted and value ranges assigned: counters hold every map's values
-// and keys once the stream is done
+// and keys once the stream is done, overflow is set if a table was full
 void launch_group_count(const MapGroup& g, hipStream_t s) {
     const u64 slots = u64(g.count) * g.tsize;
     const unsigned nt = unsigned(group_tiles(g.tsize));
@@ -383,7 +380,8 @@ void launch_group_count(const MapGroup& g, hipStream_t s) {
     hipLaunchKernelGGL(k_tile_offsets, dim3(nt, g.count), dim3(256), 0, s, g);
 }
 
-// the tables of g.fin (keys cleared before)
+// the tables of g.fin (keys cleared before); every read has its slot, any of
+// the table's
 void launch_group_fill(const MapGroup& g, hipStream_t s) {
     hipLaunchKernelGGL(k_insert_final, dim3(std::min(grid_for(g.tsize, 256), 4096), g.count), dim3(256), 0, s, g);
     hipLaunchKernelGGL(k_scatter_values, dim3(grid_for(g.n * u64(g.count), 256)), dim3(256), 0, s, g);
@@ -929,7 +927,7 @@ int query_lds_bytes(int h, int cap, int maxLen, int threads, int candLimit, int 
 // Wavefronts of a query over n anchors: at most 4,096, what 256 compute units
 // hold at once, each taking every so manieth anchor; a spill row per wavefront
 // instead of per anchor bounds the scratch.
-int query_spill_rows(int n) { return std::min(n, 1 << 12); }
+int query_spill_rows(int n) { return std::min(n, kQueryWavefronts); }
 
 void launch_query(const DevReadStore& rs, const DevTables& t, u64 first, int n, int maxCand, int capL, int regMax,
                   int excludeAmbiguous, int candLimit, u32* candIds, int pitch, int* candCount, u32* spill,

@@ -8,6 +8,8 @@
 #                          kernels' index checks (CARE_EMU_CHECKS) and the
 #                          address and undefined-behaviour sanitizers (CPU
 #                          code only: nothing here is built for a GPU)
+#   build_emu.sh small     the library into tests/emu/_build/small/, with the
+#                          small scratch of CARE_SMALL_SCRATCH (engine.h)
 set -e
 here="$(cd "$(dirname "$0")" && pwd)"
 root="$(dirname "$(dirname "$here")")"
@@ -19,6 +21,10 @@ if [ "$1" = "checked" ]; then
     SAN="-fsanitize=address,undefined -fno-sanitize-recover=undefined -fno-omit-frame-pointer"
     FLAGS="$FLAGS -O1 -DCARE_EMU_CHECKS $SAN"
     HOSTFLAGS="$HOSTFLAGS -g $SAN"
+fi
+if [ "$1" = "small" ]; then
+    out="$out/small"
+    FLAGS="$FLAGS -DCARE_SMALL_SCRATCH -DCARE_EMU_CHECKS"
 fi
 mkdir -p "$out"
 # up to date: both outputs newer than every source they are built from
