@@ -20,6 +20,8 @@ namespace care_engine {
 void launch_fill_u64(u64* p, u64 n, u64 v, hipStream_t s);
 void launch_fill_u32(u32* p, u64 n, u32 v, hipStream_t s);
 u64 group_tiles(u64 tsize);
+u64 build_slots(u64 n);
+int build_group(u64 n, int h);
 void launch_group_count(const MapGroup& g, hipStream_t s);
 void launch_group_fill(const MapGroup& g, hipStream_t s);
 void launch_sort_buckets(const u32* toff, const u32* tcount, u64 tsize, u32* values, hipStream_t s);
@@ -837,13 +839,8 @@ int care_minhash_build(care_context* ctx) {
         g.n = n;
         g.h = h;
         g.cap = ctx->cap;
-        // scratch tables at load <= 0.5
-        g.tsize = 1;
-        while (g.tsize < 2 * n) g.tsize <<= 1;
-        // maps built together: as many as fit kBuildScratch, 128 MiB (memory
-        // costs up to 25 ms a GiB, a group two waits for the device)
-        const u64 perMap = g.tsize * 16 + n * 12 + group_tiles(g.tsize) * 16;
-        const int G = int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), kBuildScratch / perMap})));
+        g.tsize = build_slots(n);
+        const int G = build_group(n, h);
         DevBuf<u64> keys64;  // tkeys, tile sums, counters, overflow
         DevBuf<u32> words;   // tcount, toff, slot, arrival, packed
         keys64.alloc(size_t(G) * (g.tsize + 2 * group_tiles(g.tsize) + 2) + 1);

@@ -367,6 +367,20 @@ void launch_fill_u32(u32* p, u64 n, u32 v, hipStream_t s) {
 }
 u64 group_tiles(u64 tsize) { return (tsize + kTile - 1) / kTile; }
 
+// slots of a scratch table over n reads: load at most 0.5
+u64 build_slots(u64 n) {
+    u64 slots = 1;
+    while (slots < 2 * n) slots <<= 1;
+    return slots;
+}
+
+// maps of n reads built together: as many as fit kBuildScratch, 128 MiB
+// (memory costs up to 25 ms a GiB, a group two waits for the device)
+int build_group(u64 n, int h) {
+    const u64 perMap = build_slots(n) * 16 + n * 12 + group_tiles(build_slots(n)) * 16;
+    return int(std::max<u64>(1, std::min<u64>({u64(h), u64(kMaxBuildMaps), kBuildScratch / perMap})));
+}
+
 // keys counted and value ranges assigned: counters hold every map's values
 // and keys once the stream is done, overflow is set if a table was full
 void launch_group_count(const MapGroup& g, hipStream_t s) {
