@@ -325,18 +325,43 @@ int default_batch(const care_context* ctx, int n) {
     return int(b & ~size_t(1));
 }
 
-// Threads of a correction workgroup over n anchors, unless they were set.
-// Two wavefronts an anchor take the least time in all (fewer barriers and idle
-// wavefronts; 1M reads 2x150: plain 35.0 ms, 44.7 with four wavefronts, gated
-// 18.5 against 27.1), four the least time for one anchor.  The latter decides
-// where there are few anchors for the workgroups the device holds, and, when
-// candidate lists have no limit, while a long list of a repeat (thousands of
-// candidates) takes as long as all others together: 40,000 anchors of 300
-// bases 2.41 against 2.45 ms, 10,000 of 100-250 bases 1.27 against 1.77.
+// Threads of a correction workgroup over n anchors, unless they were set: two
+// wavefronts an anchor (128) or four (256).  Correction times in ms, two
+// wavefronts against four, sets at 30x with repeats:
+//   plain, 150 bases: 4,000 anchors 0.58 / 0.40, 10,000 0.80 / 0.55, 20,000
+//     0.95 / 0.87, 40,000 1.36 / 1.67, 65,536 2.18 / 2.70, 1M 32.4 / 40.7
+//   plain, without repeats: 4,000 0.16 / 0.17, 65,536 1.64 / 2.10
+//   candidates corrected: 65,536 2.42 / 2.71, 300,000 11.6 / 12.5
+//   20 candidates (gated): 1,000 0.054 / 0.050, 2,048 0.079 / 0.079, 10,000
+//     0.22 / 0.28, 100,000 1.83 / 2.58
+// Two take the least time in all (fewer barriers and idle wavefronts), four
+// the least for one anchor.  The latter counts while there are few anchors for
+// the workgroups the device holds and, where lists have no limit, while the
+// long list of a repeat (thousands of candidates) takes as long as all others
+// together.  That ends between 20,000 and 40,000 anchors in these sets (100 to
+// 250 bases at 50x: 10,000 1.42 / 0.95, 40,000 3.27 / 3.33); the line lies
+// above, as it moves with the longest list of a set.
+// Long reads leave two wavefronts too little LDS.  A staging area of at most
+// 17 candidates costs lists without limit more than the second wavefront pair
+// does (65,536 anchors: 300 bases 3.94 / 3.72, with 2-bit qualities 4.98 /
+// 4.40, 8-bit 7.06 / 5.51; 250 bases, 8-bit 4.37 / 4.23, 2-bit, 22 candidates,
+// 3.21 / 3.39).  With a limit, fewer than seven workgroups a compute unit do
+// (200,000 anchors: 300 bases, 2-bit, seven, 6.30 / 7.13; 8-bit, six, 8.42 /
+// 7.74).
 int correct_threads(const care_context* ctx, int n) {
     if (ctx->blockThreads) return ctx->blockThreads;
+    const auto& o = ctx->opt;
+    const bool limited = o.candidate_limit > 0;
     const int fill = 8 * ctx->numCUs;
-    return n >= (ctx->opt.candidate_limit > 0 ? fill : 32 * fill) ? 128 : 256;
+    if (n < (limited ? fill : 32 * fill)) return 256;
+    const int gated = correct_gate_mode(o.correction_type, o.correct_candidates, o.correction_type_cands);
+    const int maxLen = std::max(1, ctx->rs.maxLen);
+    const bool room = limited ? 7 * correct_lds_bytes(maxLen, o.use_quality, ctx->rs.qpitch, 128, gated, 0,
+                                                      o.correct_candidates, o.new_columns_to_correct) <=
+                                    size_t(160) * 1024
+                              : correct_msa_chunk(maxLen, o.use_quality, ctx->rs.qpitch, 128, gated, 0,
+                                                  o.correct_candidates, o.new_columns_to_correct) > 17;
+    return room ? 128 : 256;
 }
 
 // Candidates from which an anchor is corrected before the others: about twice

@@ -277,7 +277,7 @@ typedef struct care_tuning {
     int correct_threads;        /* threads per correction workgroup, i.e. 2, 3 or 4
                                    wavefronts per anchor: 128, 192 or 256
                                    (0 = automatic: 128 on large calls, 256 on
-                                   small ones) */
+                                   small ones and for long reads) */
     int correct_blocks_per_cu;  /* persistent correction workgroups per compute unit
                                    (0 = as many as are resident at once) */
     int msa_chunk;              /* candidates staged in LDS per MSA pass, 16..256

@@ -146,3 +146,17 @@ def test_reported_chunk_is_the_launched_one(emu, length, bits, gated, candidates
     lds = _function(emu, "correct_lds_bytes", 8)
     args = (length, int(bits > 0), qpitch, t["correct_threads"], gated)
     assert lds(*args, t["msa_chunk"], candidates, 15) == lds(*args, 0, candidates, 15)
+
+
+@pytest.mark.parametrize("length,bits,limit,threads",
+                         [(150, 2, 0, 128), (225, 1, 0, 128), (250, 2, 0, 128), (250, 8, 0, 256), (300, 0, 0, 256),
+                          (300, 8, 0, 256), (400, 0, 0, 256), (250, 8, 20, 128), (300, 2, 20, 128), (300, 8, 20, 256)])
+def test_two_wavefronts_an_anchor_where_lds_has_room(emu, length, bits, limit, threads):
+    """The workgroup of a large call; 256 where 128 threads were measured slower."""
+    opt = care_amd.default_options(kmer_length=20, num_hash_maps=4, coverage=30.0, use_quality=int(bits > 0),
+                                   candidate_limit=limit, correction_type=3 if limit else 0)
+    qpitch = (bits * length + 31) // 32
+    with care_amd.Engine(opt, device=0, lib=emu) as eng:
+        eng.upload(np.zeros((2, (length + 15) // 16), np.uint32), np.full(2, length, np.int32), None,
+                   np.zeros((2, qpitch), np.uint32) if bits else None, bits or 8, length)
+        assert eng.tuning()["correct_threads"] == threads
