@@ -775,7 +775,8 @@ int care_stream_synchronize(care_context* ctx, struct ihipStream_t* stream) {
 namespace {
 // workspace of care_minhash_query_async: signature rows (8 h bytes per
 // anchor) and the query's spill rows for long hit lists (16 maxCand bytes
-// per anchor), 256-byte aligned parts
+// per anchor, of which launch_query uses query_spill_words(maxCand) words for
+// each of at most 4,096 wavefronts), 256-byte aligned parts
 size_t query_workspace_sig_bytes(const care_context* ctx, int n) {
     return (size_t(n) * size_t(ctx->opt.num_hash_maps) * sizeof(u64) + 255) / 256 * 256;
 }

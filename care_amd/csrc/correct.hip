@@ -64,9 +64,9 @@ __device__ __forceinline__ uint2 plane_word(u32 x0, u32 x1, int valid) {
     return make_uint2(((a & 0xFFFF0000u) | (b >> 16)) & mask, ((a << 16) | (b & 0xFFFFu)) & mask);
 }
 
-// Shifts still under their mismatch limit after the first 64 bases, queued
-// per wavefront: (candidate << 11 | order index, mismatches forward | reverse
-// << 16).  A slice holds one wavefront's worth.
+// Shifts still under their mismatch limit after their window's words, queued
+// per wavefront: (words compared << 20 | candidate << 11 | order index,
+// mismatches forward | reverse << 16).  A slice holds one wavefront's worth.
 constexpr int kSurvivors = 64;
 
 // LDS of one workgroup.  A sequence is held as interleaved bit planes: word
@@ -119,7 +119,8 @@ struct LdsDims {
     int pitch, qpitch, hw, maxLen, cols, waves, chunk, gated, compact;
     // threads as (row, word) pairs of rows of pitch, qpitch and pw words:
     // rows the workgroup covers at once, and 65536 / words rounded up (the
-    // quotient t / words is t * inverse >> 16 for t < 1024, words <= 64)
+    // quotient t / words is t * inverse >> 16 for t < 256, words <= 256; a row
+    // of 8-bit qualities has up to 109, fewer than the smallest workgroup)
     int stepS, stepQ, stepP, invS, invQ, invP;
     __host__ __device__ int pw() const { return hw + 3; }
     __host__ __device__ size_t bytes() const {
@@ -797,8 +798,6 @@ __device__ __forceinline__ int choose_orientation(const Aln& f, const Aln& r, in
     return 3;
 }
 
-// include/forest.hpp:57-68, 211-226: mean leaf probability over the trees,
-// accepting as soon as the running mean reaches the threshold
 // candidate record from its staged id / length / pair flag and the two
 // alignment keys: orientation chosen, shift, overlap and mismatches of it
 __device__ __forceinline__ CandMeta aligned_meta(const CandMeta& st, u32 kf, u32 kr, int la, int minov,
@@ -820,6 +819,8 @@ __device__ __forceinline__ CandMeta aligned_meta(const CandMeta& st, u32 kf, u32
     return m;
 }
 
+// include/forest.hpp:57-68, 211-226: mean leaf probability over the trees,
+// accepting as soon as the running mean reaches the threshold
 __device__ bool forest_decide(const DevForest& F, const float* f) {
     float sum = 0.f;
     for (int t = 0; t < F.numTrees; t++) {
@@ -1157,7 +1158,8 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
         }
         __syncthreads();
 
-        // ---- phase A: alignments, one wave per candidate ----
+        // ---- phase A: alignments; a wavefront takes (window of 64 shifts,
+        // candidate) pairs over all staged candidates (align_chunk) ----
         const int minovA = max(P.minOverlap, int(float(la) * P.minOverlapRatio));
         const u32* mateIds = nullptr;
         int mateN = 0;
@@ -1672,9 +1674,9 @@ __global__ void __launch_bounds__(256) k_correct(CorrectParams P, LdsDims dims) 
     }
 }
 
-// LDS shape of k_correct; MSA chunks hold up to 256 candidates and about
-// 16 KiB of staged rows; column arrays span the anchor and the margin
-// chunk: candidates staged per MSA pass (0 = about 16 KB of staged rows)
+// LDS shape of k_correct; column arrays span the anchor and the margin
+// chunk: candidates staged per MSA pass (0 = 16 to 256, at most 16 KiB of
+// staged rows and what leaves LDS for 16 wavefronts per compute unit)
 // margin: MSA columns held on either side of the anchor's
 static LdsDims make_dims(int maxLen, int useQuality, int qpitch, int threads, int gated, int chunk, int margin) {
     LdsDims d;

@@ -417,7 +417,8 @@ void launch_insert_triples(const u64* keys, const u32* offs, const u32* counts, 
 // gathered and merged pairwise, then unique, self and ambiguous reads are
 // removed in order.  Hit lists of up to `capL` entries are merged in the
 // wave's LDS slice; longer ones (heavy repeats) in the wavefront's row of
-// the global scratch `spill` (4 * maxCand words).
+// the global scratch `spill`: query_spill_words(maxCand) words, read and
+// written a word or a byte at a time (rows are 8-byte aligned).
 // ---------------------------------------------------------------------------
 // With candLimit > 0 only the candLimit candidates hit by the most maps are
 // kept (ties broken by smaller read id), still in ascending id order.

@@ -50,6 +50,7 @@ def test_accepted_shapes_launch_within_the_lds_limit(emu, gated, candidates):
                     if capacity(length, int(bits > 0), qpitch, asked, gated, chunk) > MAX_LDS:
                         continue
                     accepted += 1
+                    assert qpitch <= threads, (length, bits, threads)  # rows are staged a word a thread
                     for columns in (15, length // 2, length, 1 << 20) if candidates else (0,):
                         got = lds(length, int(bits > 0), qpitch, threads, gated, chunk, candidates, columns)
                         assert got <= MAX_LDS, (length, bits, threads, asked, chunk, columns)
