@@ -1747,8 +1747,7 @@ int care_mlp_gradient(care_context* ctx, const float* features, const uint8_t* l
     if (!ctx || !features || !labels || !params || !grad_out) return fail(CARE_ERR_ARGUMENT, "null argument");
     if (n < 1 || n > (1 << 20)) return fail(CARE_ERR_ARGUMENT, "n %d outside 1..2^20", n);
     if (!all_finite(params, CARE_MLP_PARAMS)) return fail(CARE_ERR_ARGUMENT, "non-finite input");
-    if (const uint64_t i = first_bad_label(labels, uint64_t(n)); i < uint64_t(n))
-        return fail(CARE_ERR_ARGUMENT, "label %d is not 0 or 1", int(i));
+    const int badLabel = int(first_bad_label(labels, uint64_t(n)));
     try {
         HIP_TRY(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
@@ -1765,6 +1764,7 @@ int care_mlp_gradient(care_context* ctx, const float* features, const uint8_t* l
             launch_mlp_convert(raw, m * CARE_MLP_FEATURES, X.p + first * CARE_MLP_FEATURES, ctx->mlpFlag.p, s);
         });
         if (!features_finite(ctx)) return fail(CARE_ERR_ARGUMENT, "non-finite input");
+        if (badLabel < n) return fail(CARE_ERR_ARGUMENT, "label %d is not 0 or 1", badLabel);
         Y.alloc(size_t(n));
         P.alloc(size_t(n));
         master.alloc(CARE_MLP_PARAMS);

@@ -116,6 +116,19 @@ def test_emulated_training_learns_rule(emu_engine):
     assert np.mean((z > 0) == (y == 1)) > 0.9
 
 
+@pytest.mark.parametrize("call", ["mlp_gradient", "mlp_train"])
+@pytest.mark.parametrize("feature,label,message", [(np.nan, 2, "non-finite"), (-np.inf, 1, "non-finite"),
+                                                   (1.0, 2, "label 69 is not 0 or 1")])
+def test_emulated_invalid_inputs_named_in_order(emu_engine, call, feature, label, message):
+    """Features that are not finite are named before a label that is not 0 or 1."""
+    x, y = _data(70, 13)
+    x[69, 31] = feature
+    y[69] = label
+    options = {"mlp_train": {"epochs": 1, "batch": 16}}.get(call, {})
+    with pytest.raises(care_amd.CareError, match=message):
+        getattr(emu_engine, call)(x, y, mlp_oracle.init_params(14), **options)
+
+
 # ------------------------------------------------------------------- GPU
 
 @pytest.mark.gpu
